@@ -26,6 +26,7 @@
 // step) is k_attn_dec in decode.hip.
 #include "common.h"
 #include "kernels.h"
+#include "split.h"
 
 namespace {
 
@@ -34,7 +35,8 @@ constexpr int KT = 64;  // keys per LDS tile
 template <int HS>
 __global__ void __launch_bounds__(256, 2)
     k_attn_causal(const float* __restrict__ qkv, long seq_stride, float* __restrict__ out, int B,
-                  int T, int C, int H, int nqb, float scale, float* __restrict__ lse) {
+                  int T, int C, int H, int nqb, float scale, float* __restrict__ lse,
+                  const float* __restrict__ split_scale) {
     constexpr int HALF = HS / 2;            // d values per lane half in Q K^T
     constexpr int F4 = HS / 4;              // float4 per head row
     constexpr int ROW = HS + 4;             // padded LDS row
@@ -179,9 +181,12 @@ __global__ void __launch_bounds__(256, 2)
         __syncthreads();
     }
 
+    // (both lanes of a query, l and l + 32, take the same branch: they swap
+    // halves of the split rows below)
     if (qi < T) {
         if (lse && lh == 0) lse[((long)b * H + h) * T + qi] = m_run + log2f(l_run);
         const float inv = 1.0f / l_run;
+        const float osc = split_scale ? *split_scale : 1.f;
         float* op = out + ((long)b * T + qi) * C + h * HS;
 #pragma unroll
         for (int d = 0; d < NDB; d++)
@@ -191,7 +196,16 @@ __global__ void __launch_bounds__(256, 2)
                 if (dd < HS) {
                     f32x4 v = {o[d][4 * g] * inv, o[d][4 * g + 1] * inv, o[d][4 * g + 2] * inv,
                                o[d][4 * g + 3] * inv};
-                    *(f32x4*)(op + dd) = v;
+                    if (split_scale) {
+                        unsigned h0, h1, l0, l1;
+                        split_pair(v[0] * osc, v[1] * osc, h0, l0);
+                        split_pair(v[2] * osc, v[3] * osc, h1, l1);
+                        swap32(h0, l0);
+                        swap32(h1, l1);
+                        *(u32x4*)(op + dd) = u32x4{h0, h1, l0, l1};
+                    } else {
+                        *(f32x4*)(op + dd) = v;
+                    }
                 }
             }
     }
@@ -227,7 +241,8 @@ template <int HS, int CB>
 __global__ void __launch_bounds__(256, 2)
     k_attn_ks(const float* __restrict__ qkv, long seq_stride, float* __restrict__ out, int B,
               int T, int C, int H, int nqb, float scale, float* __restrict__ lse,
-              const float* __restrict__ W, float* __restrict__ part) {
+              const float* __restrict__ W, float* __restrict__ part,
+              const float* __restrict__ split_scale) {
     constexpr int HALF = HS / 2;
     constexpr int NDB = (HS + 31) / 32;
     constexpr int OS = NDB * 32 + 1;  // LDS row of a merged query
@@ -392,7 +407,16 @@ __global__ void __launch_bounds__(256, 2)
         if constexpr (CB > 0) {
             on[q * PS + d] = v / l;
         } else {
-            out[((long)b * T + q0 + q) * C + h * HS + d] = v / l;
+            float* op = out + ((long)b * T + q0 + q) * C + h * HS;
+            if (split_scale) {
+                const float y = v / l * *split_scale;
+                const _Float16 hi = (_Float16)y;
+                _Float16* oh = (_Float16*)(op + (d & ~7)) + (d & 7);
+                oh[0] = hi;
+                oh[8] = (_Float16)(y - (float)hi);
+            } else {
+                op[d] = v / l;
+            }
             if (lse && d == 0) lse[((long)b * H + h) * T + q0 + q] = mx + log2f(l);
         }
     }
@@ -447,7 +471,7 @@ __global__ void __launch_bounds__(256, 2)
 
 template <int HS>
 hipError_t causal_hs(const float* qkv, long seq_stride, float* out, int B, int T, int C, int H,
-                     float* lse, hipStream_t s) {
+                     float* lse, const float* split_scale, hipStream_t s) {
     const int nqb = (T + 127) / 128;
     const float scale = 1.0f / sqrtf((float)HS);
     // (the key split holds a 32-key block of K and V per lane: up to HS = 64)
@@ -458,26 +482,28 @@ hipError_t causal_hs(const float* qkv, long seq_stride, float* out, int B, int T
         if ((long)nqb * B * H < 512) {
             const int nqb32 = (T + 31) / 32;
             k_attn_ks<HS, 0><<<nqb32 * B * H, 256, 0, s>>>(qkv, seq_stride, out, B, T, C, H,
-                                                            nqb32, scale, lse, nullptr, nullptr);
+                                                            nqb32, scale, lse, nullptr, nullptr,
+                                                            split_scale);
             return hipGetLastError();
         }
     }
     k_attn_causal<HS><<<nqb * B * H, 256, 0, s>>>(qkv, seq_stride, out, B, T, C, H, nqb, scale,
-                                                   lse);
+                                                   lse, split_scale);
     return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t launch_attention_causal(const float* qkv, long seq_stride, float* out, int B, int T,
-                                   int C, int H, hipStream_t s, float* lse) {
+                                   int C, int H, hipStream_t s, float* lse,
+                                   const float* split_scale) {
     if (B <= 0 || T <= 0) return hipSuccess;
     switch (C / H) {
-        case 8: return causal_hs<8>(qkv, seq_stride, out, B, T, C, H, lse, s);
-        case 16: return causal_hs<16>(qkv, seq_stride, out, B, T, C, H, lse, s);
-        case 32: return causal_hs<32>(qkv, seq_stride, out, B, T, C, H, lse, s);
-        case 64: return causal_hs<64>(qkv, seq_stride, out, B, T, C, H, lse, s);
-        case 128: return causal_hs<128>(qkv, seq_stride, out, B, T, C, H, lse, s);
+        case 8: return causal_hs<8>(qkv, seq_stride, out, B, T, C, H, lse, split_scale, s);
+        case 16: return causal_hs<16>(qkv, seq_stride, out, B, T, C, H, lse, split_scale, s);
+        case 32: return causal_hs<32>(qkv, seq_stride, out, B, T, C, H, lse, split_scale, s);
+        case 64: return causal_hs<64>(qkv, seq_stride, out, B, T, C, H, lse, split_scale, s);
+        case 128: return causal_hs<128>(qkv, seq_stride, out, B, T, C, H, lse, split_scale, s);
     }
     return hipErrorInvalidValue;
 }
@@ -504,12 +530,12 @@ hipError_t launch_attention_proj(const float* qkv, long seq_stride, const float*
     const float scale = 1.0f / sqrtf(64.0f);
     if (CB == 4)
         k_attn_ks<64, 4><<<grid, 256, 0, s>>>(qkv, seq_stride, nullptr, B, T, C, H, nqb32, scale,
-                                              nullptr, W, part);
+                                              nullptr, W, part, nullptr);
     else if (CB == 3)
         k_attn_ks<64, 3><<<grid, 256, 0, s>>>(qkv, seq_stride, nullptr, B, T, C, H, nqb32, scale,
-                                              nullptr, W, part);
+                                              nullptr, W, part, nullptr);
     else
         k_attn_ks<64, 2><<<grid, 256, 0, s>>>(qkv, seq_stride, nullptr, B, T, C, H, nqb32, scale,
-                                              nullptr, W, part);
+                                              nullptr, W, part, nullptr);
     return hipGetLastError();
 }

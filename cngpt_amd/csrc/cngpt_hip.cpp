@@ -158,6 +158,26 @@ struct cngpt_hip_ctx {
     bool use_qkv_fold = true;
     std::vector<Packed> packs;
     std::unordered_map<const float*, const float*> packed_of;
+    // Split copies (split.h) of the same matrices and the input scales of
+    // their products (launch_split_scales), in the same allocation, for the
+    // forwards over more than SPLIT_MIN_ROWS rows. Made with the packed copies
+    // and stale when they are; split_state is 1 where the split products are
+    // as accurate as fp32 ones, -1 where they are not, 0 while the device's
+    // verdict has not been read. CNGPT_HIP_SPLIT=0 at create time: none.
+    struct SplitMat {
+        const float* W;
+        SplitWeights o;
+        int N, K;
+        int in;            // slot of its input's scale
+        const float* typ;  // typical sizes of its inputs (launch_split_w)
+        const float* typ_b;
+    };
+    bool use_split = true;
+    int split_state = 0;
+    std::vector<SplitMat> splits;
+    std::unordered_map<const float*, SplitWeights> split_of;
+    float *sp_bound = nullptr, *sp_scale = nullptr, *sp_typ = nullptr;
+    int* sp_bad = nullptr;
 
     // activation arena: one allocation, carved below
     char* d_act = nullptr;
@@ -208,7 +228,7 @@ struct cngpt_hip_ctx {
     // cngpt_hip_forward_resident replay it; captured on the first call of a
     // shape, again after the arena or the parameters moved)
     hipGraphExec_t fwd_exec = nullptr;
-    int fwd_B = 0, fwd_T = 0, fwd_mode = -1;
+    int fwd_B = 0, fwd_T = 0, fwd_mode = -1, fwd_split = 0;
     const void *fwd_act = nullptr, *fwd_par = nullptr;
 
     // state of the last forward / decode
@@ -274,7 +294,40 @@ struct Timed {
 constexpr int SKINNY = 2;
 
 int run_ln(cngpt_hip_ctx* h, const float* x, long in_stride, const float* w, const float* b,
-           float* out, int rows);
+           float* out, int rows, const float* split_scale = nullptr);
+
+// Rows above which a forward's layer products take the split operands
+// (split.hip); up to them the few-row products stream the weights.
+constexpr int SPLIT_MIN_ROWS = 128;
+
+// Y = epi(X . W^T) over split rows X. out_scale: the GELU epilogue's output
+// scale. With lnout, also LayerNorm(Y rows) as split rows times *lnscale.
+int run_split(cngpt_hip_ctx* h, const float* X, const float* W, const float* bias, float* Y, int M,
+              int N, int K, int epi, const float* out_scale = nullptr, int seg = 0,
+              long seg_stride = 0, const float* lnw = nullptr, const float* lnb = nullptr,
+              float* lnout = nullptr, const float* lnscale = nullptr) {
+    const auto it = h->split_of.find(W);
+    if (it == h->split_of.end()) return fail("no split copy of a weight matrix");
+    SplitGemmArgs a{};
+    a.X = X; a.W = it->second.W; a.winv = it->second.winv;
+    a.bias = bias; a.Y = Y;
+    a.M = M; a.N = N; a.K = K;
+    a.ldy = N;
+    a.seg = seg; a.seg_stride = seg_stride;
+    a.epi = epi;
+    a.out_scale = out_scale;
+    a.part = h->gemm_part; a.part_cap = GEMM_PART_FLOATS;
+    const bool ln_in_sum = lnout && launch_split_gemm_splits(a) > 1;
+    if (ln_in_sum) {
+        a.ln_w = lnw; a.ln_b = lnb; a.ln_out = lnout; a.ln_scale = lnscale;
+    }
+    {
+        Timed t(h, CNGPT_K_GEMM, 2.0 * M * N * K,
+                4.0 * ((double)M * K + (double)N * K + (double)M * N * (epi == EPI_RESID ? 2 : 1)));
+        HIP_TRY(launch_split_gemm(a, h->stream));
+    }
+    return lnout && !ln_in_sum ? run_ln(h, Y, N, lnw, lnb, lnout, M, lnscale) : 0;
+}
 
 // With lnw / lnb / lnout set, also LayerNorm(Y rows) into lnout (the next
 // product's input); over more than SKINNY rows the split-K sum forms it.
@@ -332,10 +385,11 @@ int run_gemm(cngpt_hip_ctx* h, const float* X, const float* W, const float* bias
 }
 
 int run_ln(cngpt_hip_ctx* h, const float* x, long in_stride, const float* w, const float* b,
-           float* out, int rows) {
+           float* out, int rows, const float* split_scale) {
     const int C = h->cfg.n_embd;
     Timed t(h, CNGPT_K_LAYERNORM, 0.0, 8.0 * C * rows);
-    HIP_TRY(launch_layernorm(x, in_stride, w, b, out, C, rows, C, h->stream));
+    HIP_TRY(launch_layernorm(x, in_stride, w, b, out, C, rows, C, h->stream, nullptr, nullptr,
+                             split_scale));
     return 0;
 }
 
@@ -638,6 +692,10 @@ int enqueue_forward(cngpt_hip_ctx* h, int B, int T, int mode, bool kv, bool want
     const int C = c.n_embd, L = c.n_layer, H = c.n_head;
     const long rows = (long)B * T;
     const long seq_stride = kv ? h->capKV : T;
+    // with sp, ln, aout and hid hold split rows (the same bytes), each scaled
+    // by its slot's power of two
+    const bool sp = h->split_state == 1 && rows > SPLIT_MIN_ROWS;
+    auto scale = [&](int l, int slot) { return sp ? h->sp_scale + 4 * l + slot : nullptr; };
     {
         Timed t(h, CNGPT_K_EMBED, 0.0, 12.0 * C * rows);
         HIP_TRY(launch_embed(h->tok, h->wte, h->wpe, h->x, rows, T, C, c.vocab_size, 0, nullptr,
@@ -646,13 +704,16 @@ int enqueue_forward(cngpt_hip_ctx* h, int B, int T, int mode, bool kv, bool want
     // LayerNorm 1 of layer 0; every later LayerNorm over all rows is formed
     // by the residual product before it (while it sums its K splits, or in a
     // launch right after it), into ln
-    if (run_ln(h, h->x, C, h->layers[0].ln1_w, h->layers[0].ln1_b, h->ln, (int)rows)) return -1;
+    if (run_ln(h, h->x, C, h->layers[0].ln1_w, h->layers[0].ln1_b, h->ln, (int)rows, scale(0, 0)))
+        return -1;
     for (int l = 0; l < L; l++) {
         const LayerW& w = h->layers[l];
         const bool last = (mode == CNGPT_LAST) && (l == L - 1);
         float* qkv = kv ? h->qkv + (size_t)l * B * h->capKV * 3 * C : h->qkv;
-        if (run_gemm(h, h->ln, w.attn_w, w.attn_b, qkv, (int)rows, 3 * C, C, EPI_BIAS,
-                     kv ? T : 0, seq_stride, 3L * C))
+        if (sp ? run_split(h, h->ln, w.attn_w, w.attn_b, qkv, (int)rows, 3 * C, C, EPI_BIAS,
+                           nullptr, kv ? T : 0, seq_stride)
+               : run_gemm(h, h->ln, w.attn_w, w.attn_b, qkv, (int)rows, 3 * C, C, EPI_BIAS,
+                          kv ? T : 0, seq_stride, 3L * C))
             return -1;
         if (!last) {
             // the next LayerNorm after the MLP: layer l+1's first, or the
@@ -684,7 +745,17 @@ int enqueue_forward(cngpt_hip_ctx* h, int B, int T, int mode, bool kv, bool want
                     double by = 4.0 * rows * C * 4;  // q,k,v read + out written
                     Timed t(h, CNGPT_K_ATTN, fl, by);
                     HIP_TRY(launch_attention_causal(qkv, seq_stride, h->aout, B, T, C, H,
-                                                    h->stream));
+                                                    h->stream, nullptr, scale(l, 1)));
+                }
+                if (sp) {
+                    if (run_split(h, h->aout, w.proj_w, w.proj_b, h->x, (int)rows, C, C, EPI_RESID,
+                                  nullptr, 0, 0, w.ln2_w, w.ln2_b, h->ln, scale(l, 2)) ||
+                        run_split(h, h->ln, w.fc_w, w.fc_b, h->hid, (int)rows, 4 * C, C,
+                                  EPI_BIAS_GELU, scale(l, 3)) ||
+                        run_split(h, h->hid, w.mlp_w, w.mlp_b, h->x, (int)rows, C, 4 * C, EPI_RESID,
+                                  nullptr, 0, 0, nw, nb, h->ln, scale(l + 1, 0)))
+                        return -1;
+                    continue;
                 }
                 if (run_gemm(h, h->aout, w.proj_w, w.proj_b, h->x, (int)rows, C, C, EPI_RESID, 0,
                              0, -1, 0, nullptr, w.ln2_w, w.ln2_b, h->ln))
@@ -711,7 +782,10 @@ int enqueue_forward(cngpt_hip_ctx* h, int B, int T, int mode, bool kv, bool want
     }
     if (mode == CNGPT_ALL) {
         // ln holds the final LayerNorm of every row (formed by the last proj)
-        if (run_gemm(h, h->ln, h->wte, nullptr, h->logits, (int)rows, c.vocab_size, C, EPI_STORE))
+        if (sp ? run_split(h, h->ln, h->wte, nullptr, h->logits, (int)rows, c.vocab_size, C,
+                           EPI_STORE)
+               : run_gemm(h, h->ln, h->wte, nullptr, h->logits, (int)rows, c.vocab_size, C,
+                          EPI_STORE))
             return -1;
         h->logits_count = (size_t)rows * c.vocab_size;
     } else {
@@ -729,6 +803,7 @@ int enqueue_forward(cngpt_hip_ctx* h, int B, int T, int mode, bool kv, bool want
 int run_forward(cngpt_hip_ctx* h, int B, int T, int mode) {
     if (h->prof || !h->use_graph) return enqueue_forward(h, B, T, mode, false, false);
     if (!h->fwd_exec || h->fwd_B != B || h->fwd_T != T || h->fwd_mode != mode ||
+        h->fwd_split != h->split_state ||
         h->fwd_act != h->d_act || h->fwd_par != h->d_params) {
         drop_fwd_graph(h);
         hipGraph_t g = nullptr;
@@ -746,6 +821,7 @@ int run_forward(cngpt_hip_ctx* h, int B, int T, int mode) {
         if (ei != hipSuccess) return fail("forward graph instantiate: %s", hipGetErrorString(ei));
         h->fwd_exec = ex;
         h->fwd_B = B; h->fwd_T = T; h->fwd_mode = mode;
+        h->fwd_split = h->split_state;
         h->fwd_act = h->d_act;
         h->fwd_par = h->d_params;
     }
@@ -1009,15 +1085,45 @@ size_t packed_bytes(const cngpt_hip_config* cfg) {
     return align_up(packed_w_floats(cfg->vocab_size, C) * sizeof(float)) + layer * cfg->n_layer;
 }
 
-// Packs the weight matrices (again, after an AdamW update marked them
-// stale: ctx_params_written) in kernels on the handle's stream, ordered
-// before what follows.
-int fresh_packed(cngpt_hip_ctx* h) {
-    if (!h->use_packed || h->packed_fresh) return 0;
-    HIP_TRY(hipSetDevice(h->device));
-    for (const cngpt_hip_ctx::Packed& p : h->packs)
-        HIP_TRY(launch_pack_w(p.W, p.Wp, p.N, p.K, h->stream));
-    h->packed_fresh = true;
+// Bytes of the split copies: the same matrices with a scale per row, the
+// 4 L + 1 input bounds and scales, the typical sizes and the verdict. The
+// split products take K in steps of 16.
+size_t split_bytes(const cngpt_hip_config* cfg) {
+    const size_t C = cfg->n_embd, V = cfg->vocab_size, L = cfg->n_layer;
+    if (C % 16) return 0;
+    auto mat = [](size_t N, size_t K) { return align_up(4 * N * K) + align_up(4 * N); };
+    return mat(V, C) + L * (mat(3 * C, C) + mat(C, C) + mat(4 * C, C) + mat(C, 4 * C)) +
+           2 * align_up(4 * (4 * L + 1)) + align_up(4 * 5 * C * L) + align_up(sizeof(int));
+}
+
+// Makes the packed and split copies of the weight matrices (again, after an
+// AdamW update marked them stale: ctx_params_written) in kernels on the
+// handle's stream, ordered before what follows. resolve: also read the
+// verdict on the split products, if it is not known (this synchronises).
+int fresh_packed(cngpt_hip_ctx* h, bool resolve = true) {
+    if (!h->packed_fresh) {
+        HIP_TRY(hipSetDevice(h->device));
+        for (const cngpt_hip_ctx::Packed& p : h->packs)
+            HIP_TRY(launch_pack_w(p.W, p.Wp, p.N, p.K, h->stream));
+        if (!h->splits.empty()) {
+            const int L = h->cfg.n_layer;
+            HIP_TRY(launch_split_scales(h->d_layers, h->layers.data(), h->lnf_w, h->lnf_b, L,
+                                        h->cfg.n_embd, h->sp_bound, h->sp_scale, h->sp_typ,
+                                        h->sp_bad, h->stream));
+            for (const cngpt_hip_ctx::SplitMat& m : h->splits)
+                HIP_TRY(launch_split_w(m.W, m.o, m.N, m.K, m.typ, m.typ_b, h->sp_bound + m.in,
+                                       h->sp_scale + m.in, h->sp_bad, h->stream));
+            h->split_state = 0;
+        }
+        h->packed_fresh = true;
+    }
+    if (resolve && !h->splits.empty() && h->split_state == 0) {
+        int bad = 0;
+        HIP_TRY(hipSetDevice(h->device));
+        HIP_TRY(hipMemcpyAsync(&bad, h->sp_bad, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+        HIP_TRY(hipStreamSynchronize(h->stream));
+        h->split_state = bad ? -1 : 1;
+    }
     return 0;
 }
 
@@ -1043,11 +1149,12 @@ int params_prepare(cngpt_hip_ctx* h, const cngpt_hip_config* cfg) {
     h->have_params = false;
     h->d_layers = nullptr;
     // one allocation: the parameters, the table of per-layer pointers into
-    // them that the persistent decode reads, the packed weight copies
+    // them that the persistent decode reads, the packed and split weight copies
     const long want = params_of(cfg);
     const size_t bytes = align_up((size_t)want * sizeof(float)) +
                          align_up((size_t)cfg->n_layer * sizeof(LayerW)) +
-                         (h->use_packed ? packed_bytes(cfg) : 0);
+                         (h->use_packed ? packed_bytes(cfg) : 0) +
+                         (h->use_split ? split_bytes(cfg) : 0);
     if (hipMalloc(&h->d_params, bytes) != hipSuccess) {
         (void)hipGetLastError();
         h->d_params = nullptr;
@@ -1089,15 +1196,19 @@ int params_commit(cngpt_hip_ctx* h, const cngpt_hip_config* cfg) {
                       hipMemcpyHostToDevice));
     h->packs.clear();
     h->packed_of.clear();
+    h->splits.clear();
+    h->split_of.clear();
     h->packed_fresh = false;
+    h->split_state = 0;
+    char* q = (char*)h->d_layers + align_up((size_t)cfg->n_layer * sizeof(LayerW));
+    auto take = [&](size_t bytes) { char* r = q; q += align_up(bytes); return r; };
+    const int c = (int)C;
     if (h->use_packed) {
-        char* q = (char*)h->d_layers + align_up((size_t)cfg->n_layer * sizeof(LayerW));
         auto add = [&](const float* W, int N, int K) {
-            h->packs.push_back({W, (float*)q, N, K});
-            h->packed_of[W] = (const float*)q;
-            q += align_up(packed_w_floats(N, K) * sizeof(float));
+            float* Wp = (float*)take(packed_w_floats(N, K) * sizeof(float));
+            h->packs.push_back({W, Wp, N, K});
+            h->packed_of[W] = Wp;
         };
-        const int c = (int)C;
         add(h->wte, (int)V, c);
         for (const LayerW& w : h->layers) {
             add(w.attn_w, 3 * c, c);
@@ -1105,8 +1216,31 @@ int params_commit(cngpt_hip_ctx* h, const cngpt_hip_config* cfg) {
             add(w.fc_w, 4 * c, c);
             add(w.mlp_w, c, 4 * c);
         }
-        if (fresh_packed(h)) return -1;
     }
+    if (h->use_split && split_bytes(cfg)) {
+        const int L = cfg->n_layer;
+        h->sp_bound = (float*)take(4 * (4 * (size_t)L + 1));
+        h->sp_scale = (float*)take(4 * (4 * (size_t)L + 1));
+        h->sp_typ = (float*)take(4 * 5 * (size_t)C * L);
+        h->sp_bad = (int*)take(sizeof(int));
+        auto add = [&](const float* W, int N, int K, int in, const float* typ, const float* typ_b) {
+            SplitWeights o;
+            o.W = take((size_t)N * K * sizeof(float));
+            o.winv = (float*)take((size_t)N * sizeof(float));
+            h->splits.push_back({W, o, N, K, in, typ, typ_b});
+            h->split_of[W] = o;
+        };
+        add(h->wte, (int)V, c, 4 * L, h->lnf_w, h->lnf_b);
+        for (int l = 0; l < L; l++) {
+            const LayerW& w = h->layers[l];
+            const float* t = h->sp_typ + (size_t)l * 5 * C;
+            add(w.attn_w, 3 * c, c, 4 * l, w.ln1_w, w.ln1_b);
+            add(w.proj_w, c, c, 4 * l + 1, t, nullptr);
+            add(w.fc_w, 4 * c, c, 4 * l + 2, w.ln2_w, w.ln2_b);
+            add(w.mlp_w, c, 4 * c, 4 * l + 3, t + C, nullptr);
+        }
+    }
+    if (fresh_packed(h)) return -1;
     h->have_params = true;
     return 0;
 }
@@ -1386,6 +1520,8 @@ int cngpt_hip_create(int device, cngpt_hip_ctx** out) {
     if (pp && pp[0] == '0') h->decode_path = CNGPT_DECODE_KERNELS;
     const char* pk = getenv("CNGPT_HIP_PACK");
     h->use_packed = !(pk && pk[0] == '0');
+    const char* sv = getenv("CNGPT_HIP_SPLIT");
+    h->use_split = !(sv && sv[0] == '0');
     const char* ap = getenv("CNGPT_HIP_ATTNPROJ");
     h->use_attn_proj = !(ap && ap[0] == '0');
     // 2, 3 or 4: that many column blocks per wavefront where they divide C
@@ -1487,7 +1623,9 @@ int cngpt_hip_forward_resident(cngpt_hip_ctx* h, int B, int T, int mode) {
 
 int cngpt_hip_forward_noalloc(cngpt_hip_ctx* h, const int* tokens, int B, int T, int mode,
                               float* logits, int* err) {
-    if (need_params(h) || fresh_packed(h)) return -1;
+    // (without a synchronisation: until another entry point has read the
+    // verdict on copies made here, the fp32 products run)
+    if (need_params(h) || fresh_packed(h, false)) return -1;
     if (mode != CNGPT_LAST && mode != CNGPT_ALL) return fail("bad mode %d", mode);
     if (!tokens || !logits) return fail("forward_noalloc: null device pointer");
     if (B <= 0 || T <= 0) return fail("B=%d T=%d must be positive", B, T);

@@ -45,6 +45,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "split.h"
 
 namespace {
 
@@ -1255,11 +1256,15 @@ __global__ void __launch_bounds__(256) k_stream_reduce_ln(GemmArgs a, int KS) {
         }
     const float rstd = 1.0f / sqrtf(block_sum(q) / (float)a.N + 1e-5f);
     float* orow = a.ln_out + (long)r * a.N;
+    const float sc = a.ln_scale ? *a.ln_scale : 1.f;
 #pragma unroll
     for (int i = 0; i < NCH; i++) {
         const int c4 = tid + 256 * i;
-        if (c4 < N4)
-            *(f32x4*)(orow + 4 * c4) = (y[i] - mean) * rstd * lw[i] + lb[i];
+        if (c4 < N4) {
+            const f32x4 o = (y[i] - mean) * rstd * lw[i] + lb[i];
+            if (a.ln_scale) *(u32x4*)(orow + 4 * c4) = split_quad(o * sc, lane);
+            else *(f32x4*)(orow + 4 * c4) = o;
+        }
     }
 }
 
@@ -1675,7 +1680,8 @@ hipError_t launch_pack_w(const float* W, float* Wp, int N, int K, hipStream_t s)
 
 hipError_t launch_sum_heads(const GemmArgs& a, int KS, hipStream_t s) {
     if (a.M <= 0) return hipSuccess;
-    if (KS < 1 || (long)KS * a.M * a.N > a.part_cap || (a.N & 3) || (a.ln_out && a.N > 2048))
+    if (KS < 1 || (long)KS * a.M * a.N > a.part_cap || (a.N & 3) || (a.ln_out && a.N > 2048) ||
+        (a.ln_scale && (!a.ln_out || (a.N & 7))))
         return hipErrorInvalidValue;
     return reduce_splits<EPI_RESID>(a, KS, s);
 }

@@ -3,14 +3,23 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+// Parameter pointers of one layer (the carve order of assign_weights).
+struct LayerW {
+    const float *ln1_w, *ln1_b, *attn_w, *attn_b, *proj_w, *proj_b;
+    const float *ln2_w, *ln2_b, *fc_w, *fc_b, *mlp_w, *mlp_b;
+};
+
 // rowops.hip
 hipError_t launch_embed(const int* tok, const float* wte, const float* wpe, float* x, long rows,
                         int T, int C, int V, int pos0, const int* pos_dev, int* err,
                         int* hist, long hist_stride, hipStream_t s);
-// With mean / rstd set (both or neither), also each row's mean and rstd.
+// With mean / rstd set (both or neither), also each row's mean and rstd; with
+// split_scale set, out as split rows (split.h) times *split_scale (C a
+// multiple of 8).
 hipError_t launch_layernorm(const float* x, long in_stride, const float* w, const float* b,
                             float* out, long out_stride, int rows, int C, hipStream_t s,
-                            float* mean = nullptr, float* rstd = nullptr);
+                            float* mean = nullptr, float* rstd = nullptr,
+                            const float* split_scale = nullptr);
 hipError_t launch_gather_rows(const float* src, long src_stride, float* dst, int rows, int C,
                               hipStream_t s);
 
@@ -43,6 +52,7 @@ struct GemmArgs {
     const float* ln_w;
     const float* ln_b;
     float* ln_out;
+    const float* ln_scale;  // launch_sum_heads: ln_out as split rows (split.h) times *ln_scale
     // Optional K-major operands (M > SKINNY_MAX_M, K a multiple of 32):
     // km = 3, both, with the residual epilogue: X is [K][ldx] (row k holds
     // the M rows' k-th values), W is [K][ldw]; km = 2, W only, with the
@@ -74,6 +84,49 @@ hipError_t launch_sum_heads(const GemmArgs& a, int KS, hipStream_t s);
 // that writes it (K a multiple of 4).
 size_t packed_w_floats(int N, int K);
 hipError_t launch_pack_w(const float* W, float* Wp, int N, int K, hipStream_t s);
+
+// split.hip: the same products on the fp16 matrix cores, both operands split
+// rows (split.h) whose scales winv[n] undoes per output column (K a multiple of
+// 16). The GELU epilogue writes split rows scaled by *out_scale; with ln_out
+// (EPI_RESID) the LayerNorm of every row as split rows scaled by *ln_scale,
+// formed in the split-K sum (launch_split_gemm_splits > 1 only).
+struct SplitGemmArgs {
+    const void* X;
+    const void* W;
+    const float* winv;
+    const float* bias;
+    float* Y;
+    int M, N, K;
+    long ldy;
+    int seg;           // output row mapping as in GemmArgs
+    long seg_stride;
+    int epi;
+    const float* out_scale;
+    float* part;
+    long part_cap;
+    const float* ln_w;
+    const float* ln_b;
+    float* ln_out;
+    const float* ln_scale;
+};
+hipError_t launch_split_gemm(const SplitGemmArgs& a, hipStream_t s);
+int launch_split_gemm_splits(const SplitGemmArgs& a);
+int launch_split_gemm_plan(const SplitGemmArgs& a);  // splits + 256 x tile shape
+// Input scales and split weights of a model: bound and scale hold 4 L + 1
+// floats (slot 4 l: layer l's LayerNorm 1 output, + 1 attention output, + 2
+// LayerNorm 2 output, + 3 GELU output; 4 L the final LayerNorm's), typ L x 5 C
+// floats. *bad becomes non-zero where split products would be less accurate
+// than fp32 ones.
+struct SplitWeights {
+    void* W;      // split rows
+    float* winv;  // per row
+};
+hipError_t launch_split_scales(const LayerW* d_layers, const LayerW* layers, const float* lnf_w,
+                               const float* lnf_b, int L, int C, float* bound, float* scale,
+                               float* typ, int* bad, hipStream_t s);
+hipError_t launch_split_w(const float* W, const SplitWeights& o, int N, int K, const float* typ,
+                          const float* typ_b, const float* bound, const float* scale, int* bad,
+                          hipStream_t s);
 
 // decode.hip
 // Partials of the split one-query attention, merged by their consumer:
@@ -206,11 +259,6 @@ hipError_t launch_sample(const float* logits, int rows, int V, float temp, int t
                          hipStream_t s);
 
 // persist.hip
-// Parameter pointers of one layer (the carve order of assign_weights).
-struct LayerW {
-    const float *ln1_w, *ln1_b, *attn_w, *attn_b, *proj_w, *proj_b;
-    const float *ln2_w, *ln2_b, *fc_w, *fc_b, *mlp_w, *mlp_b;
-};
 // Greedy decode of one sequence (B = 1, head size 64) for n_steps steps as
 // one cooperative launch: feeds *tok at position *pos, leaves the logits of
 // the last step in logits, the tokens fed in hist[pos..], the next token in
@@ -256,9 +304,11 @@ hipError_t launch_decode_persist(const PersistArgs& a, int G, hipStream_t s);
 // qkv + (b * seq_stride + t) * 3C. out row (b*T + t) gets the merged heads.
 // With lse set, also the log-sum-exp of every query's scores in base 2 (of
 // the scores times scale * log2(e)) at lse[(b * H + h) * T + t], which the
-// attention backward uses to recompute the probabilities.
+// attention backward uses to recompute the probabilities. With split_scale
+// set, out as split rows (split.h) times *split_scale.
 hipError_t launch_attention_causal(const float* qkv, long seq_stride, float* out, int B, int T,
-                                   int C, int H, hipStream_t s, float* lse = nullptr);
+                                   int C, int H, hipStream_t s, float* lse = nullptr,
+                                   const float* split_scale = nullptr);
 // The same attention (64-wide heads, keys split over a workgroup's
 // wavefronts) with each head's share of the c_proj product applied in the
 // launch: part[(h * B * T + row) * C + n] = sum over d of out[row][h * 64 +

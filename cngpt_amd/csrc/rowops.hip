@@ -6,6 +6,7 @@
 // shuffles), so no LDS or block barrier is needed.
 #include "common.h"
 #include "kernels.h"
+#include "split.h"
 
 // x[i, :] = wte[tok[i], :] + wpe[pos0 + i % T, :]   (reference fast.c:245-254)
 // One thread per float4. pos0 comes from *pos_dev when pos_dev is set, so a
@@ -39,6 +40,8 @@ __global__ void __launch_bounds__(256) k_embed(const int* __restrict__ tok,
 // variance of (x - mean), rstd = 1/sqrtf(var + 1e-5), out = (x-m)*rstd*w + b;
 // with mean_out / rstd_out set, also each row's mean and rstd (the training
 // forward keeps them for the backward, as layernorm_fwd does).
+// With split_scale the row is written as split values (split.h) times it, the
+// operand of the next product (in place of its fp32 form, the same bytes).
 // NCH = float4 chunks per lane, so C <= 256 * NCH. Rows are read at stride
 // in_stride and written at stride out_stride (floats), which lets the final
 // LayerNorm of the last-position pass gather rows b*T + T-1.
@@ -48,7 +51,8 @@ __global__ void __launch_bounds__(256) k_layernorm(const float* __restrict__ x, 
                                                    const float* __restrict__ b, float* __restrict__ out,
                                                    long out_stride, int rows, int C,
                                                    float* __restrict__ mean_out,
-                                                   float* __restrict__ rstd_out) {
+                                                   float* __restrict__ rstd_out,
+                                                   const float* __restrict__ split_scale) {
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
@@ -81,10 +85,15 @@ __global__ void __launch_bounds__(256) k_layernorm(const float* __restrict__ x, 
         rstd_out[row] = rs;
     }
     float* orow = out + (long)row * out_stride;
+    const float sc = split_scale ? *split_scale : 1.f;
 #pragma unroll
     for (int j = 0; j < NCH; j++) {
         int c = (lane + j * 64) * 4;
-        if (c < C) *(f32x4*)(orow + c) = (v[j] - m) * rs * wv[j] + bv[j];
+        if (c < C) {
+            const f32x4 o = (v[j] - m) * rs * wv[j] + bv[j];
+            if (split_scale) *(u32x4*)(orow + c) = split_quad(o * sc, lane);
+            else *(f32x4*)(orow + c) = o;
+        }
     }
 }
 
@@ -113,21 +122,26 @@ hipError_t launch_embed(const int* tok, const float* wte, const float* wpe, floa
 
 hipError_t launch_layernorm(const float* x, long in_stride, const float* w, const float* b,
                             float* out, long out_stride, int rows, int C, hipStream_t s,
-                            float* mean, float* rstd) {
+                            float* mean, float* rstd, const float* split_scale) {
     if (rows == 0) return hipSuccess;
-    if (!mean != !rstd) return hipErrorInvalidValue;
+    if (!mean != !rstd || (split_scale && (C & 7))) return hipErrorInvalidValue;
     dim3 grid((rows + 3) / 4), block(256);
     int nch = (C + 255) / 256;
     if (nch <= 1)
-        k_layernorm<1><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd);
+        k_layernorm<1><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd,
+                                            split_scale);
     else if (nch <= 2)
-        k_layernorm<2><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd);
+        k_layernorm<2><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd,
+                                            split_scale);
     else if (nch <= 3)
-        k_layernorm<3><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd);
+        k_layernorm<3><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd,
+                                            split_scale);
     else if (nch <= 4)
-        k_layernorm<4><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd);
+        k_layernorm<4><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd,
+                                            split_scale);
     else if (nch <= 8)
-        k_layernorm<8><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd);
+        k_layernorm<8><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd,
+                                            split_scale);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();

@@ -1,0 +1,46 @@
+// split.h - fp32 values as pairs of fp16 values (hi + lo), the operand form of
+// the products on the fp16 matrix cores (split.hip).
+//
+// A split row of K values (K a multiple of 16) has the bytes of K floats: each
+// group of 8 values is 16 bytes of hi halves, then 16 bytes of lo halves, so a
+// lane's operand of a 16-k matrix instruction is one 16-byte granule.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "common.h"
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// hi and lo halves of two values (round to nearest, so that lo is at most
+// half a unit of hi's last place): |v - hi - lo| <= 2^-23 |v| while |v| <=
+// 2^15 and lo is a normal fp16, at most 2^-25 below that.
+__device__ __forceinline__ void split_pair(float x, float y, unsigned& hi, unsigned& lo) {
+    const f16x2 h = {(_Float16)x, (_Float16)y};
+    const f16x2 l = {(_Float16)(x - (float)h[0]), (_Float16)(y - (float)h[1])};
+    hi = __builtin_bit_cast(unsigned, h);
+    lo = __builtin_bit_cast(unsigned, l);
+}
+
+// lanes 32-63 of a <-> lanes 0-31 of b
+__device__ __forceinline__ void swap32(unsigned& a, unsigned& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+
+// Four consecutive values (columns c .. c + 3 of a split row, c = 4 x the
+// lane's place in the row, neighbouring lanes holding neighbouring quads):
+// an even lane gets the pair's hi granule, an odd lane its lo granule, each
+// stored at the byte offset 4 c of the row. Both lanes of a pair are active.
+__device__ __forceinline__ u32x4 split_quad(const f32x4& v, int lane) {
+    unsigned h0, h1, l0, l1;
+    split_pair(v[0], v[1], h0, l0);
+    split_pair(v[2], v[3], h1, l1);
+    const bool odd = lane & 1;
+    const unsigned s0 = odd ? h0 : l0, s1 = odd ? h1 : l1;
+    const unsigned r0 = __builtin_amdgcn_mov_dpp(s0, 0xB1, 0xF, 0xF, false);
+    const unsigned r1 = __builtin_amdgcn_mov_dpp(s1, 0xB1, 0xF, 0xF, false);
+    return odd ? u32x4{r0, r1, l0, l1} : u32x4{h0, h1, r0, r1};
+}

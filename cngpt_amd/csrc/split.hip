@@ -1,0 +1,668 @@
+// split.hip - fp32 products Y[M,N] = epi(X[M,K] . W[N,K]^T) on the fp16
+// matrix cores of gfx950.
+//
+// Each fp32 operand value is held as hi + lo, two fp16 values (split.h): hi is
+// the value rounded to 11 bits, lo the remainder rounded to 11 bits, exact for
+// three values in four and off by one unit of fp32's last place otherwise. A
+// product is hi hi + hi lo + lo hi, three v_mfma_f32_32x32x16_f16 summed in
+// fp32 (the missing lo lo is below 2^-22 of the product). The fp32 matrix
+// instructions add their products to the accumulator two k at a time, and
+// that chain's rounding is what their error is made of; sixteen k at a time
+// it is a quarter as long, so the split products are the nearer of the two to
+// float64 (M=300 N=500 K=768, unit inputs: 2.7e-7 against 4.4e-7 relative in
+// the 2-norm for an fp32 chain). The fp16 units run at 16 times the fp32 rate,
+// so three instructions per product are about five times the fp32 peak.
+//
+// Range: fp16 reaches 65504, and its smallest step is 2^-24. Operands are
+// scaled by powers of two (exact) so that no value can exceed 2^15: a weight
+// row by its own largest value, an input by a bound that follows from the
+// weights alone. LayerNorm outputs are at most sqrt(C) max|g| + max|b|; a
+// product of one, y = w . (g x^ + b) + c with |x^| <= sqrt(C), is at most
+// sqrt(C) |w g| + |w . b + c|, which bounds v, so the attention's output (an
+// average of v rows), and fc, so GELU's. The scales are powers of two, so
+// results do not depend on them until values fall 2^-16 below their bound and
+// lo starts losing bits: an absolute error of 2^-39 of the bound. k_split_w
+// compares that with each output's typical size and flags matrices where it
+// could exceed 2^-24 of it (gains or rows many thousands of times apart, or
+// values that are not finite); a model with a flagged matrix keeps the fp32
+// kernels.
+#include <algorithm>
+#include <type_traits>
+
+#include "common.h"
+#include "kernels.h"
+#include "split.h"
+
+namespace {
+
+constexpr int SP_BK = 16;  // k per stage and per matrix instruction
+
+__device__ __forceinline__ int xcd_order(int pid, int nt) {
+    const int per = nt / 8, rem = nt % 8;
+    const int xcd = pid % 8, idx = pid / 8;
+    return (xcd < rem) ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
+}
+
+// Tile of work id p: groups of 8 row tiles, so that neighbours share X and W
+// rows in the XCD's L2 (4 and 16 measured 1-3 % slower).
+__device__ __forceinline__ void group_coords(int p, int tiles_m, int tiles_n, int& tm, int& tn) {
+    const int GM = 8;
+    const int group = p / (GM * tiles_n);
+    const int first_m = group * GM;
+    const int gsize = min(tiles_m - first_m, GM);
+    const int in_group = p % (GM * tiles_n);
+    tm = first_m + in_group % gsize;
+    tn = in_group / gsize;
+}
+
+template <int EPI>
+__device__ __forceinline__ float epi_value(float v, float b, float old) {
+    if (EPI == EPI_STORE) return v;
+    if (EPI == EPI_BIAS) return v + b;
+    if (EPI == EPI_BIAS_GELU) return gelu_tanh(v + b);
+    return (old + v) + b;
+}
+
+// A workgroup of WR x WC wavefronts owns a tile of 64 WR rows x 32 CB WC
+// columns, each wavefront 2 x CB blocks of 32 x 32. Both operands go from
+// global memory straight into LDS (lds_dma16) through a ring of S stages of 16
+// k, 64 bytes a row: granule 2 q + p of a row is plane p (hi, lo) of its k
+// octet q, stored at slot (2 q + p) ^ (row / 4 % 4), so that the 16 rows a
+// quarter wavefront reads at one granule fall in 16 different granules of a
+// 256-byte bank line. A step waits for stage kt + 1, passes one barrier
+// (every wavefront has stage kt in registers by then, so its slot is free for
+// stage kt + S), and then multiplies stage kt while it reads stage kt + 1 and
+// issues the loads of stage kt + S, one such instruction between two matrix
+// instructions: issued together ahead of them they left the matrix cores idle
+// for as long as the LDS queue took (QKV at M=16384, 181 -> 171 us; proj 224
+// -> 208). Wave priority as in gemm.hip.
+//
+// The bound is the matrix cores at the clock the chip holds under them: a
+// register-only loop of these instructions on random data reaches 1300-1560
+// TFLOP/s (2500 nominal), and the 256 x 192 tiles at K = 3072 run 1200 of
+// raw products (399 of fp32 work, against 134 on the fp32 cores).
+//
+// VEC: the operands swapped, so that a lane holds four consecutive columns of
+// a row and moves them as 16 bytes (N, ldy and the pointers multiples of
+// four); without it 32 lanes cover 32 columns of a row, which takes any
+// alignment (the lm_head's odd row length). The GELU epilogue writes Y as split
+// rows scaled by *out_scale, the next product's operand. KS > 1 (EPI_STORE):
+// K split over workgroups, partials to a.part + ks M N.
+template <int EPI, int WR, int WC, int CB, int S, int OCC, bool VEC>
+__global__ void __launch_bounds__(64 * WR * WC, OCC * WR * WC / 4)
+    k_gemm_split(SplitGemmArgs a, int tiles_m, int tiles_n, int KR, int KS) {
+    constexpr int NW = WR * WC, TM = 64 * WR, TN = 32 * CB * WC;
+    constexpr int ROWS = (TM + TN + 16 * NW - 1) / (16 * NW) * 16 * NW;  // padded: whole loads
+    constexpr int NI = ROWS / (16 * NW);  // load instructions per wavefront and stage
+    constexpr int STAGE = ROWS * 64;      // bytes
+    constexpr bool OUT_SPLIT = EPI == EPI_BIAS_GELU;
+    static_assert(S >= 2 && OCC * S * STAGE <= 160 * 1024, "LDS");
+    __shared__ __attribute__((aligned(1024))) char sm[S * STAGE];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int tiles = tiles_m * tiles_n;
+    int p = xcd_order(blockIdx.x, tiles * KS);
+    const int ks = p / tiles;
+    p -= ks * tiles;
+    int tm, tn;
+    group_coords(p, tiles_m, tiles_n, tm, tn);
+    const int m0 = tm * TM, n0 = tn * TN, K = a.K, kb = ks * KR;
+    const int nk = (min(KR, K - kb)) / SP_BK;
+
+    // load instruction i of this wavefront covers stage rows 16 (NW i + wave)
+    // .. +15 (X rows, then W rows, then padding): lane -> row lane / 4, slot
+    // lane % 4; rows past M or N re-read the last one (their results are not
+    // stored)
+    const char* src[NI];
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const int row = 16 * (NW * i + wave) + (lane >> 2);
+        const int g = (lane & 3) ^ ((row >> 2) & 3);
+        src[i] = (row < TM ? (const char*)a.X + (long)min(m0 + row, a.M - 1) * K * 4
+                           : (const char*)a.W + (long)min(n0 + row - TM, a.N - 1) * K * 4) +
+                 (long)kb * 4 + 16 * g;
+    }
+    auto issue1 = [&](int kt, int slot, int i) {
+        lds_dma16(src[i] + (long)kt * 64,
+                  (const float*)(sm + slot * STAGE + (NW * i + wave) * 1024));
+    };
+    const int wm = (wave / WC) * 64, wn = (wave % WC) * 32 * CB;
+    const int lr = lane & 31, lh = lane >> 5;
+    // byte offsets of this lane's hi granules in a stage (lo: bit 4 flipped)
+    const int sw = 16 * ((2 * lh) ^ ((lr >> 2) & 3));
+    const int ah = (wm + lr) * 64 + sw, bh = (TM + wn + lr) * 64 + sw;
+    const int al = ah ^ 16, bl = bh ^ 16;
+
+    f32x16 acc[2][CB];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < CB; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+
+    struct Ops {
+        f16x8 ah[2], al[2], bh[CB], bl[CB];
+    };
+    constexpr int NR = 2 * CB + 4, NM = 6 * CB;  // reads and products of a step
+    constexpr int NQ = (NR + NI + NM - 1) / NM;  // reads and loads per product
+    // read q of a stage, in the order the products use them
+    auto read1 = [&](int slot, Ops& o, int q) {
+        const char* base = sm + slot * STAGE;
+        if (q < CB) o.bh[q] = *(const f16x8*)(base + bh + q * 2048);
+        else if (q < CB + 2) o.al[q - CB] = *(const f16x8*)(base + al + (q - CB) * 2048);
+        else if (q < CB + 4) o.ah[q - CB - 2] = *(const f16x8*)(base + ah + (q - CB - 2) * 2048);
+        else o.bl[q - CB - 4] = *(const f16x8*)(base + bl + (q - CB - 4) * 2048);
+    };
+    // product q: lo hi, hi hi, hi lo over the blocks
+    auto mul1 = [&](const Ops& o, int q) {
+        const int pr = q / (2 * CB), j = (q % (2 * CB)) / 2, i = q & 1;
+        const f16x8 x = pr == 0 ? o.al[i] : o.ah[i], w = pr == 2 ? o.bl[j] : o.bh[j];
+        acc[i][j] = VEC ? __builtin_amdgcn_mfma_f32_32x32x16_f16(w, x, acc[i][j], 0, 0, 0)
+                        : __builtin_amdgcn_mfma_f32_32x32x16_f16(x, w, acc[i][j], 0, 0, 0);
+    };
+
+#pragma unroll
+    for (int st = 0; st < S; st++)
+        if (st < nk)
+#pragma unroll
+            for (int i = 0; i < NI; i++) issue1(st, st, i);
+    if (nk >= S) wait_vmcnt<NI * (S - 1)>();
+    else wait_vmcnt<0>();
+    asm volatile("s_barrier" ::: "memory");
+    Ops o0, o1;
+#pragma unroll
+    for (int q = 0; q < NR; q++) read1(0, o0, q);
+    int slot = 0;  // kt % S
+    // FULL: stage kt + S exists
+    auto step = [&](int kt, const Ops& cur, Ops& nxt, auto full) {
+        const int next = slot + 1 == S ? 0 : slot + 1;
+        if constexpr (decltype(full)::value) {
+            // stage kt + 1 has landed once at most stages kt + 2 .. kt + S - 1
+            // are in flight
+            wait_vmcnt<NI * (S - 2)>();
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int q = 0; q < NM; q++) {
+#pragma unroll
+                for (int u = NQ * q; u < NQ * q + NQ; u++) {
+                    if (u < NR) read1(next, nxt, u);
+                    else if (u - NR < NI) issue1(kt + S, slot, u - NR);
+                }
+                mul1(cur, q);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __builtin_amdgcn_s_setprio(0);
+        } else {
+            if (kt + 1 < nk) {
+                if (kt + S - 1 < nk) wait_vmcnt<NI * (S - 2)>();
+                else wait_vmcnt<0>();
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                if (kt + S < nk)
+#pragma unroll
+                    for (int i = 0; i < NI; i++) issue1(kt + S, slot, i);
+#pragma unroll
+                for (int q = 0; q < NR; q++) read1(next, nxt, q);
+            }
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int q = 0; q < NM; q++) mul1(cur, q);
+            __builtin_amdgcn_s_setprio(0);
+        }
+        slot = next;
+    };
+    int kt = 0;
+    for (; kt + 1 + S < nk; kt += 2) {
+        step(kt, o0, o1, std::true_type{});
+        step(kt + 1, o1, o0, std::true_type{});
+    }
+    for (; kt + 1 < nk; kt += 2) {
+        step(kt, o0, o1, std::false_type{});
+        step(kt + 1, o1, o0, std::false_type{});
+    }
+    if (kt < nk) step(kt, o0, o1, std::false_type{});
+
+    if constexpr (VEC) {
+        // acc[i][j][4 g + e]: row m0 + wm + 32 i + lane % 32, column n0 + wn
+        // + 32 j + 8 g + 4 (lane / 32) + e. The scales, bias and residual of
+        // block column j + 1 are loaded before block column j is stored: a
+        // load after a store would wait for that store too (the vector-memory
+        // counter counts both).
+        const bool part = EPI == EPI_STORE && KS > 1;
+        float* yrow[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int row = min(m0 + wm + 32 * i + lr, a.M - 1);
+            const long orow = a.seg ? (long)(row / a.seg) * a.seg_stride + row % a.seg : row;
+            yrow[i] = part ? a.part + ((long)ks * a.M + row) * a.N : a.Y + orow * a.ldy;
+        }
+        const float os = OUT_SPLIT ? *a.out_scale : 1.f;
+        constexpr bool AHEAD = EPI != EPI_RESID || OCC < 3;  // (three per CU: registers)
+        f32x4 s[2][4], b[2][4], old[2][2][4];
+        auto load = [&](int j, int t) {
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int c = min(n0 + wn + 32 * j + 4 * lh + 8 * g, a.N - 4);
+                s[t][g] = *(const f32x4*)(a.winv + c);
+                if (EPI != EPI_STORE) b[t][g] = *(const f32x4*)(a.bias + c);
+                if (EPI == EPI_RESID)
+#pragma unroll
+                    for (int i = 0; i < 2; i++) old[t][i][g] = *(const f32x4*)(yrow[i] + c);
+            }
+        };
+        if (AHEAD) load(0, 0);
+#pragma unroll
+        for (int j = 0; j < CB; j++) {
+            const int t = AHEAD ? j & 1 : 0;
+            if (!AHEAD) load(j, 0);
+            else if (j + 1 < CB) load(j + 1, t ^ 1);
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const bool rok = m0 + wm + 32 * i + lr < a.M;
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const int c = n0 + wn + 32 * j + 4 * lh + 8 * g;
+                    f32x4 v;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const float y = acc[i][j][4 * g + e] * s[t][g][e];
+                        v[e] = epi_value<EPI>(y, EPI == EPI_STORE ? 0.f : b[t][g][e],
+                                              EPI == EPI_RESID ? old[t][i][g][e] : 0.f);
+                    }
+                    if constexpr (OUT_SPLIT) {
+                        // lanes l and l + 32 hold columns 0-3 and 4-7 of an
+                        // octet: the lower lane stores its hi granule, the
+                        // upper its lo granule
+                        unsigned h0, h1, l0, l1;
+                        split_pair(v[0] * os, v[1] * os, h0, l0);
+                        split_pair(v[2] * os, v[3] * os, h1, l1);
+                        swap32(h0, l0);
+                        swap32(h1, l1);
+                        if (rok && c < a.N) *(u32x4*)(yrow[i] + c) = u32x4{h0, h1, l0, l1};
+                    } else if (rok && c < a.N) {
+                        *(f32x4*)(yrow[i] + c) = v;
+                    }
+                }
+            }
+        }
+    } else {
+        // acc[i][j][r]: row m0 + wm + 32 i + 8 (r / 4) + 4 (lane / 32) + r %
+        // 4, column n0 + wn + 32 j + lane % 32 (stored only: the lm_head)
+        static_assert(VEC || EPI == EPI_STORE, "plain stores");
+        float s[CB];
+#pragma unroll
+        for (int j = 0; j < CB; j++) s[j] = a.winv[min(n0 + wn + 32 * j + lr, a.N - 1)];
+        const bool inside = m0 + TM <= a.M && n0 + TN <= a.N;
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * lh + (r & 3);
+                float* yr = a.Y + (long)row * a.ldy + n0 + wn + lr;
+#pragma unroll
+                for (int j = 0; j < CB; j++)
+                    if (inside || (row < a.M && n0 + wn + 32 * j + lr < a.N))
+                        yr[32 * j] = acc[i][j][r] * s[j];
+            }
+    }
+}
+
+// Y = epi(sum of the KS partials in order), eight columns per thread; with
+// out_scale split rows.
+template <int EPI>
+__global__ void __launch_bounds__(256) k_split_reduce(SplitGemmArgs a, int KS) {
+    const int n8 = a.N >> 3;
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (long)a.M * n8) return;
+    const int row = (int)(i / n8), c = (int)(i - (long)row * n8) * 8;
+    const long MN = (long)a.M * a.N;
+    const float* p = a.part + (long)row * a.N + c;
+    const long orow = a.seg ? (long)(row / a.seg) * a.seg_stride + row % a.seg : row;
+    float* y = a.Y + orow * a.ldy + c;
+    f32x4 b[2] = {}, old[2] = {}, v[2] = {};
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        if (EPI != EPI_STORE) b[h] = *(const f32x4*)(a.bias + c + 4 * h);
+        if (EPI == EPI_RESID) old[h] = *(const f32x4*)(y + 4 * h);
+    }
+    for (int q0 = 0; q0 < KS; q0 += 4) {
+        f32x4 t[4][2];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                t[j][h] = *(const f32x4*)(p + min(q0 + j, KS - 1) * MN + 4 * h);
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (q0 + j < KS)
+#pragma unroll
+                for (int h = 0; h < 2; h++) v[h] += t[j][h];
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[h][e] = epi_value<EPI>(v[h][e], b[h][e], old[h][e]);
+    if (a.out_scale) {
+        const float os = *a.out_scale;
+        u32x4 hi, lo;
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                unsigned hp, lp;
+                split_pair(v[h][2 * e] * os, v[h][2 * e + 1] * os, hp, lp);
+                hi[2 * h + e] = hp;
+                lo[2 * h + e] = lp;
+            }
+        *(u32x4*)y = hi;
+        *(u32x4*)(y + 4) = lo;
+    } else {
+        *(f32x4*)y = v[0];
+        *(f32x4*)(y + 4) = v[1];
+    }
+}
+
+// ---------------------------------------------------------------- scales
+
+__device__ __forceinline__ float block_max(float v, float* red) {
+    v = wave_max(v);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+}
+
+// max that keeps a NaN (fmaxf drops it)
+__device__ __forceinline__ float max_nan(float m, float v) { return v <= m ? m : v; }
+
+// Bounds of the LayerNorm outputs: slot 4 l of layer l's LayerNorm 1, 4 l + 2
+// of its LayerNorm 2, 4 L of the final one; the other slots are cleared for
+// k_split_bound.
+__global__ void __launch_bounds__(256) k_split_ln_bound(const LayerW* layers, const float* lnf_w,
+                                                        const float* lnf_b, int L, int C,
+                                                        float* bound, int* bad) {
+    __shared__ float red[4];
+    const int i = blockIdx.x, l = i >> 1;
+    const float* g = i == 2 * L ? lnf_w : i & 1 ? layers[l].ln2_w : layers[l].ln1_w;
+    const float* b = i == 2 * L ? lnf_b : i & 1 ? layers[l].ln2_b : layers[l].ln1_b;
+    float mg = 0.f, mb = 0.f;
+    bool fin = true;
+    for (int c = threadIdx.x; c < C; c += 256) {
+        mg = fmaxf(mg, fabsf(g[c]));
+        mb = fmaxf(mb, fabsf(b[c]));
+        fin = fin && fabsf(g[c]) < 1e30f && fabsf(b[c]) < 1e30f;
+    }
+    mg = block_max(mg, red);
+    mb = block_max(mb, red);
+    if (!fin) atomicOr(bad, 1);
+    if (threadIdx.x == 0) {
+        bound[2 * i] = sqrtf((float)C) * mg + mb;
+        if (i < 2 * L) bound[2 * i + 1] = 0.f;
+    }
+}
+
+__global__ void k_split_clear(int* bad) { *bad = 0; }
+
+// Of each row n of W [N, K] applied to a LayerNorm output (gains g, biases
+// b): typ[n], the output's size for inputs of unit variance, and the
+// largest possible |output| over all rows into *bound. One wavefront per row.
+__global__ void __launch_bounds__(256) k_split_bound(const float* __restrict__ W,
+                                                     const float* __restrict__ g,
+                                                     const float* __restrict__ b,
+                                                     const float* __restrict__ bias, int N, int K,
+                                                     float* __restrict__ typ, float* bound,
+                                                     int* bad) {
+    const int n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (n >= N) return;
+    float s2 = 0.f, sb = 0.f;
+    for (int k = 4 * lane; k < K; k += 256) {
+        const f32x4 w = *(const f32x4*)(W + (long)n * K + k);
+        const f32x4 gg = *(const f32x4*)(g + k), bb = *(const f32x4*)(b + k);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            s2 += (w[e] * gg[e]) * (w[e] * gg[e]);
+            sb += w[e] * bb[e];
+        }
+    }
+    s2 = wave_sum(s2);
+    sb = wave_sum(sb) + bias[n];
+    if (lane) return;
+    const float y = sqrtf((float)K) * sqrtf(s2) + fabsf(sb);
+    typ[n] = sqrtf(s2 + sb * sb);
+    if (y < 1e30f) atomicMax((int*)bound, __float_as_int(y));  // non-negative: ordered as ints
+    else atomicOr(bad, 1);
+}
+
+// scale = the power of two that takes the bound into [2^14, 2^15)
+__global__ void k_split_scales(const float* bound, float* scale, int n) {
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    if (i >= n) return;
+    const float b = bound[i];
+    scale[i] = b > 1e-30f && b < 1e30f ? ldexpf(1.f, 14 - ilogbf(b)) : 1.f;
+}
+
+// Split rows of W [N, K], each scaled so that its largest value lies in [2^14,
+// 2^15), and winv[n] = 1 / (row scale x input scale), which undoes both. typ:
+// the typical sizes of the K inputs, as |g| and |b| (typ_b set) or their own.
+// One wavefront per row.
+__global__ void __launch_bounds__(256) k_split_w(const float* __restrict__ W,
+                                                 unsigned* __restrict__ Ws,
+                                                 float* __restrict__ winv, int N, int K,
+                                                 const float* __restrict__ typ,
+                                                 const float* __restrict__ typ_b,
+                                                 const float* __restrict__ bound,
+                                                 const float* __restrict__ xscale, int* bad) {
+    const int n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (n >= N) return;
+    const float* w = W + (long)n * K;
+    float mx = 0.f, s2 = 0.f, st = 0.f;
+    for (int k = 4 * lane; k < K; k += 256) {
+        const f32x4 v = *(const f32x4*)(w + k), t = *(const f32x4*)(typ + k);
+        f32x4 tb = {0.f, 0.f, 0.f, 0.f};
+        if (typ_b) tb = *(const f32x4*)(typ_b + k);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            mx = max_nan(mx, fabsf(v[e]));
+            s2 += v[e] * v[e];
+            st += (v[e] * v[e]) * (t[e] * t[e] + tb[e] * tb[e]);
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = max_nan(mx, __shfl_xor(mx, o, 64));
+    s2 = wave_sum(s2);
+    st = wave_sum(st);
+    // absolute error of inputs and weights too small for a full lo (2^-39 of
+    // the bound, and of the row's largest weight) against the output's
+    // typical size
+    const float x = *bound;
+    const float err = 0x1p-39f * (x * sqrtf(s2) + mx * sqrtf((float)K) * x);
+    const bool fits = (mx == 0.f || mx > 1e-15f) && mx < 1e15f && s2 < 1e30f && err <= 0x1p-24f * sqrtf(st);
+    const float sc = mx > 0.f && fits ? ldexpf(1.f, 14 - ilogbf(mx)) : 1.f;
+    if (lane == 0) {
+        winv[n] = 1.f / (sc * *xscale);
+        if (!fits) atomicOr(bad, 1);
+    }
+    unsigned* o = Ws + (long)n * K;
+    for (int k = 8 * lane; k < K; k += 512) {
+        u32x4 hi, lo;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const f32x4 v = *(const f32x4*)(w + k + 4 * h);
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                unsigned hp, lp;
+                split_pair(v[2 * e] * sc, v[2 * e + 1] * sc, hp, lp);
+                hi[2 * h + e] = hp;
+                lo[2 * h + e] = lp;
+            }
+        }
+        *(u32x4*)(o + k) = hi;
+        *(u32x4*)(o + k + 4) = lo;
+    }
+}
+
+// ---------------------------------------------------------------- dispatch
+
+// Tile shapes, by estimated time. A step of 16 k costs a workgroup sharing its
+// CU with w - 1 others step[w - 1] us (measured on launches that leave the chip
+// part-idle; 0.71 us for 256 x 256 is 2290 TFLOP/s of raw products, 92 % of
+// nominal), but a full chip is held by its power, the larger tiles with fewer
+// LDS bytes per product the least: all steps running at a time together take
+// no less than their raw products at rate TFLOP/s. start covers a workgroup's
+// first loads and its epilogue. Measured against it (us, best
+// shape first): 2048 x 2304 x 768 128x192 28.8, 128x128 32.8, 256x192 40.2;
+// 2048 x 768 x 768 64x128 15.7, 128x128 17.7, 128x192 21.7; 4096 x 1600 x 1600
+// 128x128 69.5, 256x192 73.7, 128x192 87.5; 16384 x 3072 x 768 256x256 209,
+// 256x192 220, 128x192 223. Splitting K pays where the tiles leave CUs idle
+// over a long K (2048 x 768 x 3072: 64x128 53.7, four splits of 128x192 39.3);
+// its partials cost about 0.25 us per MB written and summed.
+struct Shape {
+    int TM, TN, occ;
+    double step[4], start, rate;
+};
+constexpr Shape SHAPES[] = {{256, 256, 1, {0.71}, 11.0, 1310},
+                            {256, 192, 1, {0.565}, 8.0, 1250},
+                            {128, 192, 2, {0.42, 0.80}, 6.0, 1140},
+                            {128, 128, 3, {0.378, 0.60, 0.95}, 4.0, 970},
+                            {64, 128, 4, {0.256, 0.49, 0.65, 0.80}, 3.5, 900}};
+
+struct Plan {
+    int shape, KS, KR;
+};
+
+bool vec_ok(const SplitGemmArgs& a) {
+    return a.N % 4 == 0 && a.ldy % 4 == 0 && (size_t)a.Y % 16 == 0 && (size_t)a.bias % 16 == 0 &&
+           (size_t)a.winv % 16 == 0;
+}
+
+double round_us(const Shape& s, long wgs, int steps) {
+    const int w = (int)((wgs + 255) / 256);
+    const double raw = (double)wgs * s.TM * s.TN * SP_BK * 6 / (s.rate * 1e6);  // us a step
+    return s.start + steps * std::max(s.step[w - 1], raw);
+}
+
+Plan plan(const SplitGemmArgs& a) {
+    Plan best{0, 1, a.K};
+    double best_us = 1e30;
+    const int nk = a.K / SP_BK;
+    const int max_ks = a.part && vec_ok(a) && a.N % 8 == 0 ? std::min(8, nk / 8) : 1;
+    for (int i = 0; i < (int)(sizeof(SHAPES) / sizeof(SHAPES[0])); i++) {
+        const Shape& s = SHAPES[i];
+        const long tiles = (long)((a.M + s.TM - 1) / s.TM) * ((a.N + s.TN - 1) / s.TN);
+        for (int ks = 1; ks <= std::max(1, max_ks); ks++) {
+            const int per = (nk + ks - 1) / ks, kse = (nk + per - 1) / per;
+            if (kse != ks || (ks > 1 && (long)ks * a.M * a.N > a.part_cap)) continue;
+            const long wgs = tiles * ks, slots = 256L * s.occ;
+            double us = (wgs / slots) * round_us(s, slots, per);
+            if (wgs % slots) us += round_us(s, wgs % slots, per);
+            if (ks > 1) us += 2.0 + 1e-6 * ks * a.M * a.N;
+            if (us < best_us) {
+                best_us = us;
+                best = Plan{i, ks, per * SP_BK};
+            }
+        }
+    }
+    return best;
+}
+
+template <int EPI, bool VEC>
+hipError_t run_shape(const SplitGemmArgs& a, const Plan& p, hipStream_t s) {
+    const Shape& sh = SHAPES[p.shape];
+    const int tm = (a.M + sh.TM - 1) / sh.TM, tn = (a.N + sh.TN - 1) / sh.TN;
+    const unsigned grid = (unsigned)(tm * tn * p.KS);
+    switch (p.shape) {
+        case 0: k_gemm_split<EPI, 4, 2, 4, 4, 1, VEC><<<grid, 512, 0, s>>>(a, tm, tn, p.KR, p.KS); break;
+        case 1: k_gemm_split<EPI, 4, 2, 3, 4, 1, VEC><<<grid, 512, 0, s>>>(a, tm, tn, p.KR, p.KS); break;
+        case 2: k_gemm_split<EPI, 2, 2, 3, 3, 2, VEC><<<grid, 256, 0, s>>>(a, tm, tn, p.KR, p.KS); break;
+        case 3: k_gemm_split<EPI, 2, 2, 2, 3, 3, VEC><<<grid, 256, 0, s>>>(a, tm, tn, p.KR, p.KS); break;
+        default: k_gemm_split<EPI, 1, 2, 2, 3, 4, VEC><<<grid, 128, 0, s>>>(a, tm, tn, p.KR, p.KS); break;
+    }
+    return hipGetLastError();
+}
+
+template <int EPI>
+hipError_t reduce(const SplitGemmArgs& a, int KS, hipStream_t s) {
+    const long n = (long)a.M * (a.N / 8);
+    k_split_reduce<EPI><<<(unsigned)((n + 255) / 256), 256, 0, s>>>(a, KS);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+int launch_split_gemm_splits(const SplitGemmArgs& a) {
+    return a.M > 0 && a.N > 0 && a.K > 0 ? plan(a).KS : 1;
+}
+
+int launch_split_gemm_plan(const SplitGemmArgs& a) {
+    const Plan p = plan(a);
+    return p.KS + 256 * p.shape;
+}
+
+hipError_t launch_split_gemm(const SplitGemmArgs& a, hipStream_t s) {
+    if (a.M <= 0 || a.N <= 0) return hipSuccess;
+    if (a.K <= 0 || a.K % SP_BK || !a.winv) return hipErrorInvalidValue;
+    const bool vec = vec_ok(a);
+    if (a.epi != EPI_STORE && (!vec || !a.bias)) return hipErrorInvalidValue;
+    if ((a.epi == EPI_BIAS_GELU) != (a.out_scale != nullptr)) return hipErrorInvalidValue;
+    if (a.epi == EPI_BIAS_GELU && a.N % 8) return hipErrorInvalidValue;
+    if (!vec && a.seg) return hipErrorInvalidValue;
+    const Plan p = plan(a);
+    // the LayerNorm is formed by the split sum; without splits the caller
+    // launches it
+    if (a.ln_out && (p.KS == 1 || a.epi != EPI_RESID || a.seg)) return hipErrorInvalidValue;
+    if (p.KS > 1) {
+        const hipError_t e = run_shape<EPI_STORE, true>(a, p, s);
+        if (e != hipSuccess) return e;
+        if (a.ln_out) {
+            GemmArgs g{};
+            g.M = a.M; g.N = a.N; g.K = a.K;
+            g.bias = a.bias; g.Y = a.Y; g.ldy = a.ldy;
+            g.part = a.part; g.part_cap = a.part_cap;
+            g.ln_w = a.ln_w; g.ln_b = a.ln_b; g.ln_out = a.ln_out; g.ln_scale = a.ln_scale;
+            g.epi = EPI_RESID;
+            return launch_sum_heads(g, p.KS, s);
+        }
+        switch (a.epi) {
+            case EPI_STORE: return reduce<EPI_STORE>(a, p.KS, s);
+            case EPI_BIAS: return reduce<EPI_BIAS>(a, p.KS, s);
+            case EPI_BIAS_GELU: return reduce<EPI_BIAS_GELU>(a, p.KS, s);
+            case EPI_RESID: return reduce<EPI_RESID>(a, p.KS, s);
+        }
+        return hipErrorInvalidValue;
+    }
+    switch (a.epi) {
+        case EPI_STORE:
+            return vec ? run_shape<EPI_STORE, true>(a, p, s) : run_shape<EPI_STORE, false>(a, p, s);
+        case EPI_BIAS: return run_shape<EPI_BIAS, true>(a, p, s);
+        case EPI_BIAS_GELU: return run_shape<EPI_BIAS_GELU, true>(a, p, s);
+        case EPI_RESID: return run_shape<EPI_RESID, true>(a, p, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_split_scales(const LayerW* d_layers, const LayerW* layers, const float* lnf_w,
+                               const float* lnf_b, int L, int C, float* bound, float* scale,
+                               float* typ, int* bad, hipStream_t s) {
+    k_split_clear<<<1, 1, 0, s>>>(bad);
+    k_split_ln_bound<<<2 * L + 1, 256, 0, s>>>(d_layers, lnf_w, lnf_b, L, C, bound, bad);
+    for (int l = 0; l < L; l++) {
+        const LayerW& w = layers[l];
+        float* t = typ + (long)l * 5 * C;
+        // the v rows of the QKV product; fc
+        k_split_bound<<<(C + 3) / 4, 256, 0, s>>>(w.attn_w + 2L * C * C, w.ln1_w, w.ln1_b,
+                                                  w.attn_b + 2 * C, C, C, t, bound + 4 * l + 1, bad);
+        k_split_bound<<<C, 256, 0, s>>>(w.fc_w, w.ln2_w, w.ln2_b, w.fc_b, 4 * C, C, t + C,
+                                        bound + 4 * l + 3, bad);
+    }
+    k_split_scales<<<(4 * L + 64) / 64, 64, 0, s>>>(bound, scale, 4 * L + 1);
+    return hipGetLastError();
+}
+
+hipError_t launch_split_w(const float* W, const SplitWeights& o, int N, int K, const float* typ,
+                          const float* typ_b, const float* bound, const float* scale, int* bad,
+                          hipStream_t s) {
+    if (N <= 0 || K <= 0 || K % SP_BK) return hipErrorInvalidValue;
+    k_split_w<<<(N + 3) / 4, 256, 0, s>>>(W, (unsigned*)o.W, o.winv, N, K, typ, typ_b, bound, scale,
+                                          bad);
+    return hipGetLastError();
+}

@@ -1,0 +1,127 @@
+// split.cpp - test-only C entry points into the split-operand products
+// (split.hip): operands split on the device as the forward splits them, the
+// product through launch_split_gemm, split outputs joined again on the host.
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <cstring>
+#include <vector>
+
+#include "../../cngpt_amd/csrc/common.h"
+#include "../../cngpt_amd/csrc/kernels.h"
+
+namespace {
+
+struct Dev {
+    std::vector<void*> ptrs;
+    bool ok = true;
+    ~Dev() {
+        for (void* p : ptrs) (void)hipFree(p);
+    }
+    template <class T>
+    T* put(const T* host, size_t n) {
+        void* p = nullptr;
+        if (hipMalloc(&p, n * sizeof(T) + 16) != hipSuccess) return ok = false, nullptr;
+        ptrs.push_back(p);
+        const hipError_t e = host ? hipMemcpy(p, host, n * sizeof(T), hipMemcpyHostToDevice)
+                                  : hipMemset(p, 0, n * sizeof(T));
+        if (e != hipSuccess) ok = false;
+        return (T*)p;
+    }
+};
+
+float join(const _Float16* row, int c, float scale) {
+    const _Float16* g = row + c / 8 * 16 + c % 8;
+    return ((float)g[0] + (float)g[8]) / scale;
+}
+
+}  // namespace
+
+extern "C" {
+
+// K splits (low byte) and tile shape (second byte) that a plain product takes.
+int kat_split_plan(int M, int N, int K) {
+    SplitGemmArgs a{};
+    a.M = M; a.N = N; a.K = K; a.ldy = N;
+    a.part = (float*)16; a.part_cap = 1 << 24;
+    return launch_split_gemm_plan(a);
+}
+
+// Y = epi(X . W^T), rows of Y ldy floats apart at the row mapping of seg /
+// seg_stride (Y holds y_rows rows). xbound: the largest |X| the scales allow
+// for. With lnout, also LayerNorm(Y rows) (gains lnw, biases lnb): formed in
+// the split-K sum, or by the LayerNorm launch. Returns the verdict on W (0:
+// accurate), -1 on failure.
+int kat_split_gemm(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K,
+                   int ldy, int seg, int seg_stride, int y_rows, int epi, float xbound,
+                   const float* lnw, const float* lnb, float* lnout) {
+    Dev d;
+    std::vector<float> ones(K > N ? K : N, 1.f);
+    float* dw = d.put(W, (size_t)N * K);
+    float* db = d.put(bias, N);
+    float* dy = d.put(Y, (size_t)y_rows * ldy);
+    float* dxs = d.put<float>(nullptr, (size_t)M * K);
+    float* dws = d.put<float>(nullptr, (size_t)N * K);
+    float* winv = d.put<float>(nullptr, N);
+    float* typ = d.put(ones.data(), K);
+    const float scale = ldexpf(1.f, 14 - ilogbf(xbound));
+    const float oscale = 64.f;
+    float* bound = d.put(&xbound, 1);
+    float* xs = d.put(&scale, 1);
+    float* os = d.put(&oscale, 1);
+    int* bad = d.put<int>(nullptr, 2);
+    float* part = d.put<float>(nullptr, 1 << 24);
+    float* dlw = lnout ? d.put(lnw, N) : nullptr;
+    float* dlb = lnout ? d.put(lnb, N) : nullptr;
+    float* dln = lnout ? d.put<float>(nullptr, (size_t)M * N) : nullptr;
+    if (!d.ok) return -1;
+    SplitWeights o{dws, winv};
+    if (launch_split_w(dw, o, N, K, typ, nullptr, bound, xs, bad, nullptr) != hipSuccess) return -1;
+    std::vector<_Float16> split((size_t)M * K * 2);
+    for (int r = 0; r < M; r++)
+        for (int k = 0; k < K; k++) {
+            const float v = X[(size_t)r * K + k] * scale;
+            _Float16* g = &split[((size_t)r * K + k / 8 * 8) * 2 + k % 8];
+            g[0] = (_Float16)v;
+            g[8] = (_Float16)(v - (float)g[0]);
+        }
+    if (hipMemcpy(dxs, split.data(), split.size() * 2, hipMemcpyHostToDevice) != hipSuccess) return -1;
+    SplitGemmArgs a{};
+    a.X = dxs; a.W = dws; a.winv = winv; a.bias = db; a.Y = dy;
+    a.M = M; a.N = N; a.K = K;
+    a.ldy = ldy;
+    a.seg = seg; a.seg_stride = seg_stride;
+    a.epi = epi;
+    a.out_scale = epi == EPI_BIAS_GELU ? os : nullptr;
+    a.part = part; a.part_cap = 1 << 24;
+    const bool in_sum = lnout && launch_split_gemm_splits(a) > 1;
+    if (in_sum) {
+        a.ln_w = dlw; a.ln_b = dlb; a.ln_out = dln; a.ln_scale = os;
+    }
+    if (launch_split_gemm(a, nullptr) != hipSuccess) return -1;
+    if (lnout && !in_sum &&
+        launch_layernorm(dy, ldy, dlw, dlb, dln, N, M, N, nullptr, nullptr, nullptr, os) != hipSuccess)
+        return -1;
+    int verdict = 0;
+    if (hipDeviceSynchronize() != hipSuccess ||
+        hipMemcpy(&verdict, bad, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess ||
+        hipMemcpy(Y, dy, (size_t)y_rows * ldy * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess)
+        return -1;
+    std::vector<_Float16> row(2 * (size_t)N);
+    auto join_rows = [&](float* rows, int n, long stride) {
+        for (int r = 0; r < n; r++) {
+            float* p = rows + r * stride;
+            memcpy(row.data(), p, (size_t)N * sizeof(float));
+            for (int c = 0; c < N; c++) p[c] = join(row.data(), c, oscale);
+        }
+    };
+    if (epi == EPI_BIAS_GELU) join_rows(Y, M, ldy);
+    if (lnout) {
+        if (hipMemcpy(lnout, dln, (size_t)M * N * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess)
+            return -1;
+        join_rows(lnout, M, N);
+    }
+    return verdict;
+}
+
+}  // extern "C"
