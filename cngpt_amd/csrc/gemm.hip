@@ -1506,6 +1506,14 @@ int tile_splits(const GemmArgs& a, int tiles, int* KR) {
     return (a.K + *KR - 1) / *KR;
 }
 
+// Whether the tiles after the whole rounds give each of G stream-K workgroups
+// at least one step: the fixup adds a slot per range, and an empty range
+// leaves its slot unwritten.
+bool sk_fills(const GemmArgs& a, int tiles, int G) {
+    const int rest = tiles % G;
+    return rest == 0 || (long)rest * (a.K / 32) >= G;
+}
+
 // Stream-K instead of whole tiles in rounds of 2 x 256 when the last round
 // would leave more than a tenth of the slots idle (more than 256 tiles, K a
 // multiple of 32, partial slots for every workgroup within a.part_cap):
@@ -1520,14 +1528,15 @@ int sk_workgroups(const GemmArgs& a, int tiles) {
         // in one round of 2 or 3 tiles per CU, 132.0 us stream-K)
         const int per_cu = (tiles + cus - 1) / cus;
         if ((double)tiles / ((double)per_cu * cus) >= 0.9) return 0;
-        if (2L * cus * BM * BN > a.part_cap) return 0;
+        if (2L * cus * BM * BN > a.part_cap || !sk_fills(a, tiles, cus)) return 0;
         return cus;
     }
     const int rounds = (tiles + G - 1) / G;
     if ((double)tiles / ((double)rounds * G) >= 0.9) return 0;
     if (2L * G * BM * BN > a.part_cap || (long)tiles * (a.K / 32) < G) return 0;
     // fewer tiles than slots: one workgroup per CU (half the partial tiles)
-    return tiles < G ? cus : G;
+    const int g = tiles < G ? cus : G;
+    return sk_fills(a, tiles, g) ? g : 0;
 }
 
 // Rounds of whole tiles ahead of the stream-K part: every full round of G
