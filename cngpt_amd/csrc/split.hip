@@ -27,6 +27,7 @@
 // values that are not finite); a model with a flagged matrix keeps the fp32
 // kernels.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "common.h"
@@ -537,21 +538,40 @@ bool vec_ok(const SplitGemmArgs& a) {
 
 double round_us(const Shape& s, long wgs, int steps) {
     const int w = (int)((wgs + 255) / 256);
-    const double raw = (double)wgs * s.TM * s.TN * SP_BK * 6 / (s.rate * 1e6);  // us a step
+    // (a part-filled round draws its power at a higher clock and gets less for
+    // it: 192 of 256 workgroups of 256 x 256 ran at 1227, all of them at 1310)
+    const double rate = s.rate * (0.75 + 0.25 * wgs / (256.0 * s.occ));
+    const double raw = (double)wgs * s.TM * s.TN * SP_BK * 6 / (rate * 1e6);  // us a step
     return s.start + steps * std::max(s.step[w - 1], raw);
 }
 
+// Splits that keep the error no larger than the fp32 kernels' where those split
+// K over idle CUs, into sums of c k each. Measured (relative 2-norm, unit
+// inputs): an fp32 sum of c k 0.73e-7 + 0.155e-7 sqrt(c) (in quadrature), a
+// split one 0.90e-7 + 0.107e-7 sqrt(c), so sums of up to 2.1 c - 25 are as good
+// (K = 256, M = 384: 1.93e-7 whole, 1.50e-7 in fp32, whose 4 splits sum 64 k);
+// 1.5 c - 20 leaves a margin.
+int min_splits(const SplitGemmArgs& a) {
+    GemmArgs g{};
+    g.M = a.M; g.N = a.N; g.K = a.K;
+    g.part = a.part; g.part_cap = a.part_cap;
+    const int ks = launch_gemm_splits(g);
+    return ks <= 1 ? 1 : (int)std::ceil(a.K / (1.5 * a.K / ks - 20.0));
+}
+
 Plan plan(const SplitGemmArgs& a) {
-    Plan best{0, 1, a.K};
-    double best_us = 1e30;
     const int nk = a.K / SP_BK;
-    const int max_ks = a.part && vec_ok(a) && a.N % 8 == 0 ? std::min(8, nk / 8) : 1;
+    const bool can = a.part && vec_ok(a) && a.N % 8 == 0;
+    const int min_ks = can ? min_splits(a) : 1;
+    const int max_ks = can ? std::max(min_ks, std::min(8, nk / 8)) : 1;
+    Plan best{3, 1, a.K};
+    double best_us = 1e30;
     for (int i = 0; i < (int)(sizeof(SHAPES) / sizeof(SHAPES[0])); i++) {
         const Shape& s = SHAPES[i];
         const long tiles = (long)((a.M + s.TM - 1) / s.TM) * ((a.N + s.TN - 1) / s.TN);
-        for (int ks = 1; ks <= std::max(1, max_ks); ks++) {
-            const int per = (nk + ks - 1) / ks, kse = (nk + per - 1) / per;
-            if (kse != ks || (ks > 1 && (long)ks * a.M * a.N > a.part_cap)) continue;
+        for (int want = min_ks; want <= max_ks; want++) {
+            const int per = (nk + want - 1) / want, ks = (nk + per - 1) / per;
+            if (ks > 1 && (long)ks * a.M * a.N > a.part_cap) continue;
             const long wgs = tiles * ks, slots = 256L * s.occ;
             double us = (wgs / slots) * round_us(s, slots, per);
             if (wgs % slots) us += round_us(s, wgs % slots, per);
