@@ -410,10 +410,11 @@ __global__ void __launch_bounds__(256, 2)
             float* op = out + ((long)b * T + q0 + q) * C + h * HS;
             if (split_scale) {
                 const float y = v / l * *split_scale;
-                const _Float16 hi = (_Float16)y;
-                _Float16* oh = (_Float16*)(op + (d & ~7)) + (d & 7);
-                oh[0] = hi;
-                oh[8] = (_Float16)(y - (float)hi);
+                unsigned hi, lo;
+                split_pair(y, y, hi, lo);
+                unsigned short* oh = (unsigned short*)(op + (d & ~7)) + (d & 7);
+                oh[0] = (unsigned short)hi;
+                oh[8] = (unsigned short)lo;
             } else {
                 op[d] = v / l;
             }

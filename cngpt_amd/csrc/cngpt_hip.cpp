@@ -300,17 +300,17 @@ int run_ln(cngpt_hip_ctx* h, const float* x, long in_stride, const float* w, con
 // (split.hip); up to them the few-row products stream the weights.
 constexpr int SPLIT_MIN_ROWS = 128;
 
-// Y = epi(X . W^T) over split rows X. out_scale: the GELU epilogue's output
-// scale. With lnout, also LayerNorm(Y rows) as split rows times *lnscale.
+// Y = epi(X . W^T) over split rows X. out_scale: the GELU and QKV epilogues'
+// output scales, Ys: the latter's split rows. With lnout, also LayerNorm(Y rows) as split rows times *lnscale.
 int run_split(cngpt_hip_ctx* h, const float* X, const float* W, const float* bias, float* Y, int M,
               int N, int K, int epi, const float* out_scale = nullptr, int seg = 0,
               long seg_stride = 0, const float* lnw = nullptr, const float* lnb = nullptr,
-              float* lnout = nullptr, const float* lnscale = nullptr) {
+              float* lnout = nullptr, const float* lnscale = nullptr, float* Ys = nullptr) {
     const auto it = h->split_of.find(W);
     if (it == h->split_of.end()) return fail("no split copy of a weight matrix");
     SplitGemmArgs a{};
     a.X = X; a.W = it->second.W; a.winv = it->second.winv;
-    a.bias = bias; a.Y = Y;
+    a.bias = bias; a.Y = Y; a.Ys = Ys;
     a.M = M; a.N = N; a.K = K;
     a.ldy = N;
     a.seg = seg; a.seg_stride = seg_stride;
@@ -695,7 +695,13 @@ int enqueue_forward(cngpt_hip_ctx* h, int B, int T, int mode, bool kv, bool want
     // with sp, ln, aout and hid hold split rows (the same bytes), each scaled
     // by its slot's power of two
     const bool sp = h->split_state == 1 && rows > SPLIT_MIN_ROWS;
-    auto scale = [&](int l, int slot) { return sp ? h->sp_scale + 4 * l + slot : nullptr; };
+    auto scale = [&](int l, int slot) {
+        return sp ? h->sp_scale + SPLIT_SLOTS * l + slot : nullptr;
+    };
+    // and where the attention takes split rows, they come from the QKV product
+    // (beside the fp32 rows of the cache, in hid, which is free until fc)
+    const bool spa = sp && attention_split_takes(C / H);
+    float* qkvs = kv ? h->hid : h->qkv;
     {
         Timed t(h, CNGPT_K_EMBED, 0.0, 12.0 * C * rows);
         HIP_TRY(launch_embed(h->tok, h->wte, h->wpe, h->x, rows, T, C, c.vocab_size, 0, nullptr,
@@ -704,16 +710,20 @@ int enqueue_forward(cngpt_hip_ctx* h, int B, int T, int mode, bool kv, bool want
     // LayerNorm 1 of layer 0; every later LayerNorm over all rows is formed
     // by the residual product before it (while it sums its K splits, or in a
     // launch right after it), into ln
-    if (run_ln(h, h->x, C, h->layers[0].ln1_w, h->layers[0].ln1_b, h->ln, (int)rows, scale(0, 0)))
+    if (run_ln(h, h->x, C, h->layers[0].ln1_w, h->layers[0].ln1_b, h->ln, (int)rows, scale(0, SLOT_LN1)))
         return -1;
     for (int l = 0; l < L; l++) {
         const LayerW& w = h->layers[l];
         const bool last = (mode == CNGPT_LAST) && (l == L - 1);
         float* qkv = kv ? h->qkv + (size_t)l * B * h->capKV * 3 * C : h->qkv;
-        if (sp ? run_split(h, h->ln, w.attn_w, w.attn_b, qkv, (int)rows, 3 * C, C, EPI_BIAS,
-                           nullptr, kv ? T : 0, seq_stride)
-               : run_gemm(h, h->ln, w.attn_w, w.attn_b, qkv, (int)rows, 3 * C, C, EPI_BIAS,
-                          kv ? T : 0, seq_stride, 3L * C))
+        if (spa && !last
+                ? run_split(h, h->ln, w.attn_w, w.attn_b, kv ? qkv : nullptr, (int)rows, 3 * C, C,
+                            EPI_QKV, scale(l, SLOT_Q), kv ? T : 0, seq_stride, nullptr, nullptr,
+                            nullptr, nullptr, qkvs)
+            : sp ? run_split(h, h->ln, w.attn_w, w.attn_b, qkv, (int)rows, 3 * C, C, EPI_BIAS,
+                             nullptr, kv ? T : 0, seq_stride)
+                 : run_gemm(h, h->ln, w.attn_w, w.attn_b, qkv, (int)rows, 3 * C, C, EPI_BIAS,
+                            kv ? T : 0, seq_stride, 3L * C))
             return -1;
         if (!last) {
             // the next LayerNorm after the MLP: layer l+1's first, or the
@@ -744,16 +754,20 @@ int enqueue_forward(cngpt_hip_ctx* h, int B, int T, int mode, bool kv, bool want
                     double fl = 2.0 * C * (double)T * (T + 1) * B;
                     double by = 4.0 * rows * C * 4;  // q,k,v read + out written
                     Timed t(h, CNGPT_K_ATTN, fl, by);
-                    HIP_TRY(launch_attention_causal(qkv, seq_stride, h->aout, B, T, C, H,
-                                                    h->stream, nullptr, scale(l, 1)));
+                    if (spa)
+                        HIP_TRY(launch_attention_split(qkvs, h->aout, B, T, C, H, scale(l, SLOT_Q),
+                                                       h->stream));
+                    else
+                        HIP_TRY(launch_attention_causal(qkv, seq_stride, h->aout, B, T, C, H,
+                                                        h->stream, nullptr, scale(l, SLOT_V)));
                 }
                 if (sp) {
                     if (run_split(h, h->aout, w.proj_w, w.proj_b, h->x, (int)rows, C, C, EPI_RESID,
-                                  nullptr, 0, 0, w.ln2_w, w.ln2_b, h->ln, scale(l, 2)) ||
+                                  nullptr, 0, 0, w.ln2_w, w.ln2_b, h->ln, scale(l, SLOT_LN2)) ||
                         run_split(h, h->ln, w.fc_w, w.fc_b, h->hid, (int)rows, 4 * C, C,
-                                  EPI_BIAS_GELU, scale(l, 3)) ||
+                                  EPI_BIAS_GELU, scale(l, SLOT_HID)) ||
                         run_split(h, h->hid, w.mlp_w, w.mlp_b, h->x, (int)rows, C, 4 * C, EPI_RESID,
-                                  nullptr, 0, 0, nw, nb, h->ln, scale(l + 1, 0)))
+                                  nullptr, 0, 0, nw, nb, h->ln, scale(l + 1, SLOT_LN1)))
                         return -1;
                     continue;
                 }
@@ -1086,14 +1100,14 @@ size_t packed_bytes(const cngpt_hip_config* cfg) {
 }
 
 // Bytes of the split copies: the same matrices with a scale per row, the
-// 4 L + 1 input bounds and scales, the typical sizes and the verdict. The
+// input bounds and scales, the typical sizes and the verdict. The
 // split products take K in steps of 16.
 size_t split_bytes(const cngpt_hip_config* cfg) {
     const size_t C = cfg->n_embd, V = cfg->vocab_size, L = cfg->n_layer;
     if (C % 16) return 0;
     auto mat = [](size_t N, size_t K) { return align_up(4 * N * K) + align_up(4 * N); };
     return mat(V, C) + L * (mat(3 * C, C) + mat(C, C) + mat(4 * C, C) + mat(C, 4 * C)) +
-           2 * align_up(4 * (4 * L + 1)) + align_up(4 * 5 * C * L) + align_up(sizeof(int));
+           2 * align_up(4 * (size_t)split_slots(L)) + align_up(4 * 7 * C * L) + align_up(sizeof(int));
 }
 
 // Makes the packed and split copies of the weight matrices (again, after an
@@ -1108,8 +1122,8 @@ int fresh_packed(cngpt_hip_ctx* h, bool resolve = true) {
         if (!h->splits.empty()) {
             const int L = h->cfg.n_layer;
             HIP_TRY(launch_split_scales(h->d_layers, h->layers.data(), h->lnf_w, h->lnf_b, L,
-                                        h->cfg.n_embd, h->sp_bound, h->sp_scale, h->sp_typ,
-                                        h->sp_bad, h->stream));
+                                        h->cfg.n_embd, h->cfg.n_head, h->sp_bound, h->sp_scale,
+                                        h->sp_typ, h->sp_bad, h->stream));
             for (const cngpt_hip_ctx::SplitMat& m : h->splits)
                 HIP_TRY(launch_split_w(m.W, m.o, m.N, m.K, m.typ, m.typ_b, h->sp_bound + m.in,
                                        h->sp_scale + m.in, h->sp_bad, h->stream));
@@ -1219,9 +1233,9 @@ int params_commit(cngpt_hip_ctx* h, const cngpt_hip_config* cfg) {
     }
     if (h->use_split && split_bytes(cfg)) {
         const int L = cfg->n_layer;
-        h->sp_bound = (float*)take(4 * (4 * (size_t)L + 1));
-        h->sp_scale = (float*)take(4 * (4 * (size_t)L + 1));
-        h->sp_typ = (float*)take(4 * 5 * (size_t)C * L);
+        h->sp_bound = (float*)take(4 * (size_t)split_slots(L));
+        h->sp_scale = (float*)take(4 * (size_t)split_slots(L));
+        h->sp_typ = (float*)take(4 * 7 * (size_t)C * L);
         h->sp_bad = (int*)take(sizeof(int));
         auto add = [&](const float* W, int N, int K, int in, const float* typ, const float* typ_b) {
             SplitWeights o;
@@ -1230,14 +1244,15 @@ int params_commit(cngpt_hip_ctx* h, const cngpt_hip_config* cfg) {
             h->splits.push_back({W, o, N, K, in, typ, typ_b});
             h->split_of[W] = o;
         };
-        add(h->wte, (int)V, c, 4 * L, h->lnf_w, h->lnf_b);
+        add(h->wte, (int)V, c, SPLIT_SLOTS * L, h->lnf_w, h->lnf_b);
         for (int l = 0; l < L; l++) {
             const LayerW& w = h->layers[l];
-            const float* t = h->sp_typ + (size_t)l * 5 * C;
-            add(w.attn_w, 3 * c, c, 4 * l, w.ln1_w, w.ln1_b);
-            add(w.proj_w, c, c, 4 * l + 1, t, nullptr);
-            add(w.fc_w, 4 * c, c, 4 * l + 2, w.ln2_w, w.ln2_b);
-            add(w.mlp_w, c, 4 * c, 4 * l + 3, t + C, nullptr);
+            const float* t = h->sp_typ + (size_t)l * 7 * C;
+            const int in = SPLIT_SLOTS * l;
+            add(w.attn_w, 3 * c, c, in + SLOT_LN1, w.ln1_w, w.ln1_b);
+            add(w.proj_w, c, c, in + SLOT_V, t + 2 * C, nullptr);
+            add(w.fc_w, 4 * c, c, in + SLOT_LN2, w.ln2_w, w.ln2_b);
+            add(w.mlp_w, c, 4 * c, in + SLOT_HID, t + 3 * C, nullptr);
         }
     }
     if (fresh_packed(h)) return -1;

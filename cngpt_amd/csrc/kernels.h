@@ -87,20 +87,24 @@ hipError_t launch_pack_w(const float* W, float* Wp, int N, int K, hipStream_t s)
 
 // split.hip: the same products on the fp16 matrix cores, both operands split
 // rows (split.h) whose scales winv[n] undoes per output column (K a multiple of
-// 16). The GELU epilogue writes split rows scaled by *out_scale; with ln_out
+// 16). The GELU epilogue writes split rows scaled by *out_scale. EPI_QKV (split
+// products only) is EPI_BIAS into Y (may be null) and split rows of N values
+// into Ys, its three thirds scaled by out_scale[0], [1], [2]. With ln_out
 // (EPI_RESID) the LayerNorm of every row as split rows scaled by *ln_scale,
 // formed in the split-K sum (launch_split_gemm_splits > 1 only).
+constexpr int EPI_QKV = 4;
 struct SplitGemmArgs {
     const void* X;
     const void* W;
     const float* winv;
     const float* bias;
     float* Y;
+    float* Ys;
     int M, N, K;
     long ldy;
-    int seg;           // output row mapping as in GemmArgs
+    int seg;           // row mapping of Y as in GemmArgs
     long seg_stride;
-    int epi;
+    int epi;           // EpiMode or EPI_QKV
     const float* out_scale;
     float* part;
     long part_cap;
@@ -112,18 +116,21 @@ struct SplitGemmArgs {
 hipError_t launch_split_gemm(const SplitGemmArgs& a, hipStream_t s);
 int launch_split_gemm_splits(const SplitGemmArgs& a);
 int launch_split_gemm_plan(const SplitGemmArgs& a);  // splits + 256 x tile shape
-// Input scales and split weights of a model: bound and scale hold 4 L + 1
-// floats (slot 4 l: layer l's LayerNorm 1 output, + 1 attention output, + 2
-// LayerNorm 2 output, + 3 GELU output; 4 L the final LayerNorm's), typ L x 5 C
-// floats. *bad becomes non-zero where split products would be less accurate
-// than fp32 ones.
+// Input scales and split weights of a model: bound and scale hold
+// split_slots(L) floats, SPLIT_SLOTS per layer: LayerNorm 1's output, q, k, v
+// (and the attention's output), LayerNorm 2's output, GELU's output; then the
+// final LayerNorm's. typ holds 7 C floats per layer. *bad becomes non-zero where
+// split products would be less accurate than fp32 ones.
+constexpr int SPLIT_SLOTS = 6;
+constexpr int split_slots(int L) { return SPLIT_SLOTS * L + 1; }
+enum SplitSlot : int { SLOT_LN1 = 0, SLOT_Q = 1, SLOT_V = 3, SLOT_LN2 = 4, SLOT_HID = 5 };
 struct SplitWeights {
     void* W;      // split rows
     float* winv;  // per row
 };
 hipError_t launch_split_scales(const LayerW* d_layers, const LayerW* layers, const float* lnf_w,
-                               const float* lnf_b, int L, int C, float* bound, float* scale,
-                               float* typ, int* bad, hipStream_t s);
+                               const float* lnf_b, int L, int C, int H, float* bound,
+                               float* scale, float* typ, int* bad, hipStream_t s);
 hipError_t launch_split_w(const float* W, const SplitWeights& o, int N, int K, const float* typ,
                           const float* typ_b, const float* bound, const float* scale, int* bad,
                           hipStream_t s);
@@ -309,6 +316,12 @@ hipError_t launch_decode_persist(const PersistArgs& a, int G, hipStream_t s);
 hipError_t launch_attention_causal(const float* qkv, long seq_stride, float* out, int B, int T,
                                    int C, int H, hipStream_t s, float* lse = nullptr,
                                    const float* split_scale = nullptr);
+// The same with split products (attn_split.hip) over split qkv rows [B T][3 C],
+// out as split rows: q, k, v carry scales[0], [1], [2], the output scales[2];
+// for the head sizes of attention_split_takes.
+bool attention_split_takes(int HS);
+hipError_t launch_attention_split(const float* qkv, float* out, int B, int T, int C, int H,
+                                  const float* scales, hipStream_t s);
 // The same attention (64-wide heads, keys split over a workgroup's
 // wavefronts) with each head's share of the c_proj product applied in the
 // launch: part[(h * B * T + row) * C + n] = sum over d of out[row][h * 64 +

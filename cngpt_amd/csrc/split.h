@@ -15,11 +15,18 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 // hi and lo halves of two values (round to nearest, so that lo is at most
 // half a unit of hi's last place): |v - hi - lo| <= 2^-23 |v| while |v| <=
-// 2^15 and lo is a normal fp16, at most 2^-25 below that.
+// 2^15 and lo is a normal fp16, at most 2^-25 below that. The values are pinned
+// to their fp32 roundings first: a product that the compiler forms again,
+// rounded straight to fp16, for one of its two uses can round to the other side
+// of a tie, and hi would be off by a whole unit.
 __device__ __forceinline__ void split_pair(float x, float y, unsigned& hi, unsigned& lo) {
-    const f16x2 h = {(_Float16)x, (_Float16)y};
-    const f16x2 l = {(_Float16)(x - (float)h[0]), (_Float16)(y - (float)h[1])};
-    hi = __builtin_bit_cast(unsigned, h);
+    asm("" : "+v"(x), "+v"(y));
+    const f16x2 hp = {(_Float16)x, (_Float16)y};
+    hi = __builtin_bit_cast(unsigned, hp);
+    float dx, dy;  // v - hi: exact
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(dx) : "v"(hi), "v"(x));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(dy) : "v"(hi), "v"(y));
+    const f16x2 l = {(_Float16)dx, (_Float16)dy};
     lo = __builtin_bit_cast(unsigned, l);
 }
 

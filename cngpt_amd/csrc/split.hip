@@ -59,7 +59,7 @@ __device__ __forceinline__ void group_coords(int p, int tiles_m, int tiles_n, in
 template <int EPI>
 __device__ __forceinline__ float epi_value(float v, float b, float old) {
     if (EPI == EPI_STORE) return v;
-    if (EPI == EPI_BIAS) return v + b;
+    if (EPI == EPI_BIAS || EPI == EPI_QKV) return v + b;
     if (EPI == EPI_BIAS_GELU) return gelu_tanh(v + b);
     return (old + v) + b;
 }
@@ -86,8 +86,8 @@ __device__ __forceinline__ float epi_value(float v, float b, float old) {
 // VEC: the operands swapped, so that a lane holds four consecutive columns of
 // a row and moves them as 16 bytes (N, ldy and the pointers multiples of
 // four); without it 32 lanes cover 32 columns of a row, which takes any
-// alignment (the lm_head's odd row length). The GELU epilogue writes Y as split
-// rows scaled by *out_scale, the next product's operand. KS > 1 (EPI_STORE):
+// alignment (the lm_head's odd row length). The GELU and QKV epilogues write
+// split rows, the next product's or the attention's operands. KS > 1 (EPI_STORE):
 // K split over workgroups, partials to a.part + ks M N.
 template <int EPI, int WR, int WC, int CB, int S, int OCC, bool VEC>
 __global__ void __launch_bounds__(64 * WR * WC, OCC * WR * WC / 4)
@@ -96,7 +96,7 @@ __global__ void __launch_bounds__(64 * WR * WC, OCC * WR * WC / 4)
     constexpr int ROWS = (TM + TN + 16 * NW - 1) / (16 * NW) * 16 * NW;  // padded: whole loads
     constexpr int NI = ROWS / (16 * NW);  // load instructions per wavefront and stage
     constexpr int STAGE = ROWS * 64;      // bytes
-    constexpr bool OUT_SPLIT = EPI == EPI_BIAS_GELU;
+    constexpr bool OUT_SPLIT = EPI == EPI_BIAS_GELU || EPI == EPI_QKV;
     static_assert(S >= 2 && OCC * S * STAGE <= 160 * 1024, "LDS");
     __shared__ __attribute__((aligned(1024))) char sm[S * STAGE];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -230,14 +230,18 @@ __global__ void __launch_bounds__(64 * WR * WC, OCC * WR * WC / 4)
         // load after a store would wait for that store too (the vector-memory
         // counter counts both).
         const bool part = EPI == EPI_STORE && KS > 1;
-        float* yrow[2];
+        float *yrow[2], *srow[2];
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             const int row = min(m0 + wm + 32 * i + lr, a.M - 1);
+            srow[i] = EPI == EPI_QKV ? a.Ys + (long)row * a.N : nullptr;
             const long orow = a.seg ? (long)(row / a.seg) * a.seg_stride + row % a.seg : row;
             yrow[i] = part ? a.part + ((long)ks * a.M + row) * a.N : a.Y + orow * a.ldy;
         }
-        const float os = OUT_SPLIT ? *a.out_scale : 1.f;
+        const float os0 = OUT_SPLIT ? a.out_scale[0] : 1.f;
+        const float os1 = EPI == EPI_QKV ? a.out_scale[1] : 1.f;
+        const float os2 = EPI == EPI_QKV ? a.out_scale[2] : 1.f;
+        const int third = a.N / 3;
         constexpr bool AHEAD = EPI != EPI_RESID || OCC < 3;  // (three per CU: registers)
         f32x4 s[2][4], b[2][4], old[2][2][4];
         auto load = [&](int j, int t) {
@@ -274,12 +278,18 @@ __global__ void __launch_bounds__(64 * WR * WC, OCC * WR * WC / 4)
                         // lanes l and l + 32 hold columns 0-3 and 4-7 of an
                         // octet: the lower lane stores its hi granule, the
                         // upper its lo granule
+                        const float os = EPI == EPI_QKV && c >= third
+                                             ? (c >= 2 * third ? os2 : os1)
+                                             : os0;
                         unsigned h0, h1, l0, l1;
                         split_pair(v[0] * os, v[1] * os, h0, l0);
                         split_pair(v[2] * os, v[3] * os, h1, l1);
                         swap32(h0, l0);
                         swap32(h1, l1);
-                        if (rok && c < a.N) *(u32x4*)(yrow[i] + c) = u32x4{h0, h1, l0, l1};
+                        if (rok && c < a.N) {
+                            *(u32x4*)((EPI == EPI_QKV ? srow[i] : yrow[i]) + c) = u32x4{h0, h1, l0, l1};
+                            if (EPI == EPI_QKV && a.Y) *(f32x4*)(yrow[i] + c) = v;
+                        }
                     } else if (rok && c < a.N) {
                         *(f32x4*)(yrow[i] + c) = v;
                     }
@@ -308,8 +318,7 @@ __global__ void __launch_bounds__(64 * WR * WC, OCC * WR * WC / 4)
     }
 }
 
-// Y = epi(sum of the KS partials in order), eight columns per thread; with
-// out_scale split rows.
+// Y = epi(sum of the KS partials in order), eight columns per thread.
 template <int EPI>
 __global__ void __launch_bounds__(256) k_split_reduce(SplitGemmArgs a, int KS) {
     const int n8 = a.N >> 3;
@@ -343,8 +352,8 @@ __global__ void __launch_bounds__(256) k_split_reduce(SplitGemmArgs a, int KS) {
     for (int h = 0; h < 2; h++)
 #pragma unroll
         for (int e = 0; e < 4; e++) v[h][e] = epi_value<EPI>(v[h][e], b[h][e], old[h][e]);
-    if (a.out_scale) {
-        const float os = *a.out_scale;
+    if (EPI == EPI_BIAS_GELU || EPI == EPI_QKV) {
+        const float os = a.out_scale[EPI == EPI_QKV ? c / (a.N / 3) : 0];
         u32x4 hi, lo;
 #pragma unroll
         for (int h = 0; h < 2; h++)
@@ -355,9 +364,11 @@ __global__ void __launch_bounds__(256) k_split_reduce(SplitGemmArgs a, int KS) {
                 hi[2 * h + e] = hp;
                 lo[2 * h + e] = lp;
             }
-        *(u32x4*)y = hi;
-        *(u32x4*)(y + 4) = lo;
-    } else {
+        float* ys = EPI == EPI_QKV ? a.Ys + (long)row * a.N + c : y;
+        *(u32x4*)ys = hi;
+        *(u32x4*)(ys + 4) = lo;
+    }
+    if (EPI != EPI_BIAS_GELU && (EPI != EPI_QKV || a.Y)) {
         *(f32x4*)y = v[0];
         *(f32x4*)(y + 4) = v[1];
     }
@@ -376,8 +387,7 @@ __device__ __forceinline__ float block_max(float v, float* red) {
 // max that keeps a NaN (fmaxf drops it)
 __device__ __forceinline__ float max_nan(float m, float v) { return v <= m ? m : v; }
 
-// Bounds of the LayerNorm outputs: slot 4 l of layer l's LayerNorm 1, 4 l + 2
-// of its LayerNorm 2, 4 L of the final one; the other slots are cleared for
+// Bounds of the LayerNorm outputs; the other slots are cleared for
 // k_split_bound.
 __global__ void __launch_bounds__(256) k_split_ln_bound(const LayerW* layers, const float* lnf_w,
                                                         const float* lnf_b, int L, int C,
@@ -397,8 +407,9 @@ __global__ void __launch_bounds__(256) k_split_ln_bound(const LayerW* layers, co
     mb = block_max(mb, red);
     if (!fin) atomicOr(bad, 1);
     if (threadIdx.x == 0) {
-        bound[2 * i] = sqrtf((float)C) * mg + mb;
-        if (i < 2 * L) bound[2 * i + 1] = 0.f;
+        float* slot = bound + SPLIT_SLOTS * l;
+        slot[i & 1 ? SLOT_LN2 : SLOT_LN1] = sqrtf((float)C) * mg + mb;
+        if (i < 2 * L && !(i & 1)) slot[SLOT_Q] = slot[SLOT_Q + 1] = slot[SLOT_V] = slot[SLOT_HID] = 0.f;
     }
 }
 
@@ -406,12 +417,13 @@ __global__ void k_split_clear(int* bad) { *bad = 0; }
 
 // Of each row n of W [N, K] applied to a LayerNorm output (gains g, biases
 // b): typ[n], the output's size for inputs of unit variance, and the
-// largest possible |output| over all rows into *bound. One wavefront per row.
+// largest possible |output| over each `part` rows into bound[n / part]. One
+// wavefront per row.
 __global__ void __launch_bounds__(256) k_split_bound(const float* __restrict__ W,
                                                      const float* __restrict__ g,
                                                      const float* __restrict__ b,
                                                      const float* __restrict__ bias, int N, int K,
-                                                     float* __restrict__ typ, float* bound,
+                                                     int part, float* __restrict__ typ, float* bound,
                                                      int* bad) {
     const int n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (n >= N) return;
@@ -430,8 +442,29 @@ __global__ void __launch_bounds__(256) k_split_bound(const float* __restrict__ W
     if (lane) return;
     const float y = sqrtf((float)K) * sqrtf(s2) + fabsf(sb);
     typ[n] = sqrtf(s2 + sb * sb);
-    if (y < 1e30f) atomicMax((int*)bound, __float_as_int(y));  // non-negative: ordered as ints
+    if (y < 1e30f) atomicMax((int*)bound + n / part, __float_as_int(y));  // non-negative: ordered as ints
     else atomicOr(bad, 1);
+}
+
+// Per layer and head: whether scores keep their accuracy. q and k values too
+// small for a full lo are off by 2^-39 of their bounds, which must move a score
+// (in units of log2 e) by no more than its fp32 roundings would: 2^-24 of its
+// typical size, or of a quarter.
+__global__ void __launch_bounds__(64) k_split_scores(const float* __restrict__ typ,
+                                                     const float* __restrict__ bound, int C, int H,
+                                                     int* bad) {
+    const int l = blockIdx.x / H, hs = C / H, h = blockIdx.x % H, lane = threadIdx.x;
+    const float* t = typ + (long)l * 7 * C + h * hs;
+    float tq = 0.f, tk = 0.f;
+    for (int d = lane; d < hs; d += 64) {
+        tq = fmaxf(tq, t[d]);
+        tk = fmaxf(tk, t[C + d]);
+    }
+    tq = wave_max(tq);
+    tk = wave_max(tk);
+    const float bq = bound[SPLIT_SLOTS * l + SLOT_Q], bk = bound[SPLIT_SLOTS * l + SLOT_Q + 1];
+    const float err = 0x1p-39f * (bq * tk + bk * tq);  // sqrt(hs) terms, over sqrt(hs)
+    if (lane == 0 && !(err <= 0x1p-24f * fmaxf(0.25f, tq * tk))) atomicOr(bad, 1);
 }
 
 // scale = the power of two that takes the bound into [2^14, 2^15)
@@ -623,8 +656,10 @@ hipError_t launch_split_gemm(const SplitGemmArgs& a, hipStream_t s) {
     if (a.K <= 0 || a.K % SP_BK || !a.winv) return hipErrorInvalidValue;
     const bool vec = vec_ok(a);
     if (a.epi != EPI_STORE && (!vec || !a.bias)) return hipErrorInvalidValue;
-    if ((a.epi == EPI_BIAS_GELU) != (a.out_scale != nullptr)) return hipErrorInvalidValue;
-    if (a.epi == EPI_BIAS_GELU && a.N % 8) return hipErrorInvalidValue;
+    const bool split_out = a.epi == EPI_BIAS_GELU || a.epi == EPI_QKV;
+    if (split_out != (a.out_scale != nullptr)) return hipErrorInvalidValue;
+    if (split_out && a.N % (a.epi == EPI_QKV ? 24 : 8)) return hipErrorInvalidValue;
+    if (a.epi == EPI_QKV && (!a.Ys || (size_t)a.Ys % 16)) return hipErrorInvalidValue;
     if (!vec && a.seg) return hipErrorInvalidValue;
     const Plan p = plan(a);
     // the LayerNorm is formed by the split sum; without splits the caller
@@ -647,6 +682,7 @@ hipError_t launch_split_gemm(const SplitGemmArgs& a, hipStream_t s) {
             case EPI_BIAS: return reduce<EPI_BIAS>(a, p.KS, s);
             case EPI_BIAS_GELU: return reduce<EPI_BIAS_GELU>(a, p.KS, s);
             case EPI_RESID: return reduce<EPI_RESID>(a, p.KS, s);
+            case EPI_QKV: return reduce<EPI_QKV>(a, p.KS, s);
         }
         return hipErrorInvalidValue;
     }
@@ -656,25 +692,28 @@ hipError_t launch_split_gemm(const SplitGemmArgs& a, hipStream_t s) {
         case EPI_BIAS: return run_shape<EPI_BIAS, true>(a, p, s);
         case EPI_BIAS_GELU: return run_shape<EPI_BIAS_GELU, true>(a, p, s);
         case EPI_RESID: return run_shape<EPI_RESID, true>(a, p, s);
+        case EPI_QKV: return run_shape<EPI_QKV, true>(a, p, s);
     }
     return hipErrorInvalidValue;
 }
 
 hipError_t launch_split_scales(const LayerW* d_layers, const LayerW* layers, const float* lnf_w,
-                               const float* lnf_b, int L, int C, float* bound, float* scale,
-                               float* typ, int* bad, hipStream_t s) {
+                               const float* lnf_b, int L, int C, int H, float* bound,
+                               float* scale, float* typ, int* bad, hipStream_t s) {
     k_split_clear<<<1, 1, 0, s>>>(bad);
     k_split_ln_bound<<<2 * L + 1, 256, 0, s>>>(d_layers, lnf_w, lnf_b, L, C, bound, bad);
     for (int l = 0; l < L; l++) {
         const LayerW& w = layers[l];
-        float* t = typ + (long)l * 5 * C;
-        // the v rows of the QKV product; fc
-        k_split_bound<<<(C + 3) / 4, 256, 0, s>>>(w.attn_w + 2L * C * C, w.ln1_w, w.ln1_b,
-                                                  w.attn_b + 2 * C, C, C, t, bound + 4 * l + 1, bad);
-        k_split_bound<<<C, 256, 0, s>>>(w.fc_w, w.ln2_w, w.ln2_b, w.fc_b, 4 * C, C, t + C,
-                                        bound + 4 * l + 3, bad);
+        float* t = typ + (long)l * 7 * C;
+        float* slot = bound + SPLIT_SLOTS * l;
+        // the QKV product's three thirds; fc
+        k_split_bound<<<(3 * C + 3) / 4, 256, 0, s>>>(w.attn_w, w.ln1_w, w.ln1_b, w.attn_b, 3 * C, C,
+                                                      C, t, slot + SLOT_Q, bad);
+        k_split_bound<<<C, 256, 0, s>>>(w.fc_w, w.ln2_w, w.ln2_b, w.fc_b, 4 * C, C, 4 * C, t + 3 * C,
+                                        slot + SLOT_HID, bad);
     }
-    k_split_scales<<<(4 * L + 64) / 64, 64, 0, s>>>(bound, scale, 4 * L + 1);
+    k_split_scores<<<L * H, 64, 0, s>>>(typ, bound, C, H, bad);
+    k_split_scales<<<(split_slots(L) + 63) / 64, 64, 0, s>>>(bound, scale, split_slots(L));
     return hipGetLastError();
 }
 

@@ -65,7 +65,7 @@ int kat_split_gemm(const float* X, const float* W, const float* bias, float* Y, 
     float* winv = d.put<float>(nullptr, N);
     float* typ = d.put(ones.data(), K);
     const float scale = ldexpf(1.f, 14 - ilogbf(xbound));
-    const float oscale = 64.f;
+    const float oscale = 64.f, qkv_scale[3] = {64.f, 256.f, 32.f};
     float* bound = d.put(&xbound, 1);
     float* xs = d.put(&scale, 1);
     float* os = d.put(&oscale, 1);
@@ -92,14 +92,17 @@ int kat_split_gemm(const float* X, const float* W, const float* bias, float* Y, 
     a.ldy = ldy;
     a.seg = seg; a.seg_stride = seg_stride;
     a.epi = epi;
-    a.out_scale = epi == EPI_BIAS_GELU ? os : nullptr;
+    a.out_scale = epi == EPI_BIAS_GELU ? os : epi == EPI_QKV ? d.put(qkv_scale, 3) : nullptr;
+    if (epi == EPI_QKV) a.Ys = dln;
+    if (!d.ok) return -1;
     a.part = part; a.part_cap = 1 << 24;
-    const bool in_sum = lnout && launch_split_gemm_splits(a) > 1;
+    const bool ln = lnout && epi != EPI_QKV;
+    const bool in_sum = ln && launch_split_gemm_splits(a) > 1;
     if (in_sum) {
         a.ln_w = dlw; a.ln_b = dlb; a.ln_out = dln; a.ln_scale = os;
     }
     if (launch_split_gemm(a, nullptr) != hipSuccess) return -1;
-    if (lnout && !in_sum &&
+    if (ln && !in_sum &&
         launch_layernorm(dy, ldy, dlw, dlb, dln, N, M, N, nullptr, nullptr, nullptr, os) != hipSuccess)
         return -1;
     int verdict = 0;
@@ -112,7 +115,8 @@ int kat_split_gemm(const float* X, const float* W, const float* bias, float* Y, 
         for (int r = 0; r < n; r++) {
             float* p = rows + r * stride;
             memcpy(row.data(), p, (size_t)N * sizeof(float));
-            for (int c = 0; c < N; c++) p[c] = join(row.data(), c, oscale);
+            for (int c = 0; c < N; c++)
+                p[c] = join(row.data(), c, epi == EPI_QKV ? qkv_scale[c / (N / 3)] : oscale);
         }
     };
     if (epi == EPI_BIAS_GELU) join_rows(Y, M, ldy);
@@ -122,6 +126,37 @@ int kat_split_gemm(const float* X, const float* W, const float* bias, float* Y, 
         join_rows(lnout, M, N);
     }
     return verdict;
+}
+
+// Causal attention over qkv [B, T, 3C] through the split kernel: out [B, T, C].
+// smax: the largest magnitude of q, k and v the scales allow for.
+int kat_attention_split(const float* qkv, float* out, int B, int T, int C, int H, const float* smax) {
+    const size_t rows = (size_t)B * T;
+    float scale[3];
+    for (int i = 0; i < 3; i++) scale[i] = ldexpf(1.f, 14 - ilogbf(smax[i]));
+    std::vector<_Float16> split(rows * 3 * C * 2);
+    for (size_t r = 0; r < rows; r++)
+        for (int c = 0; c < 3 * C; c++) {
+            const float v = qkv[r * 3 * C + c] * scale[c / C];
+            _Float16* g = &split[(r * 3 * C + c / 8 * 8) * 2 + c % 8];
+            g[0] = (_Float16)v;
+            g[8] = (_Float16)(v - (float)g[0]);
+        }
+    Dev d;
+    _Float16* dq = d.put(split.data(), split.size());
+    float* ds = d.put(scale, 3);
+    float* dout = d.put<float>(nullptr, rows * C);
+    if (!d.ok) return -1;
+    if (launch_attention_split((const float*)dq, dout, B, T, C, H, ds, nullptr) != hipSuccess ||
+        hipDeviceSynchronize() != hipSuccess ||
+        hipMemcpy(out, dout, rows * C * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess)
+        return -1;
+    std::vector<_Float16> row(2 * (size_t)C);
+    for (size_t r = 0; r < rows; r++) {
+        memcpy(row.data(), out + r * C, (size_t)C * sizeof(float));
+        for (int c = 0; c < C; c++) out[r * C + c] = join(row.data(), c, scale[2]);
+    }
+    return 0;
 }
 
 }  // extern "C"

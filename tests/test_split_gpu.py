@@ -26,6 +26,8 @@ def kat():
     lib = ctypes.CDLL(LIB)
     lib.kat_split_gemm.argtypes = ([ctypes.POINTER(ctypes.c_float)] * 4 + [ctypes.c_int] * 8 +
                                    [ctypes.c_float] + [ctypes.POINTER(ctypes.c_float)] * 3)
+    lib.kat_attention_split.argtypes = ([ctypes.POINTER(ctypes.c_float)] * 2 + [ctypes.c_int] * 4 +
+                                        [ctypes.POINTER(ctypes.c_float)])
     return lib
 
 
@@ -117,6 +119,67 @@ def test_split_rows_into_a_cache(kat):
     Y = Y.reshape(B, cap, N)
     assert np.linalg.norm(Y[:, :T].reshape(-1, N) - want) <= 1e-6 * np.linalg.norm(want)
     assert (Y[:, T:] == 7).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(150, 144, 48), (129, 2304, 768), (2048, 2304, 768)])
+@pytest.mark.parametrize("fp32", [True, False])
+def test_split_qkv(kat, M, N, K, fp32):
+    """The QKV epilogue: split rows with a scale per third, and the fp32 rows
+    (of a cache) beside them."""
+    rng = np.random.default_rng(8)
+    X = rng.standard_normal((M, K)).astype(np.float32)
+    W = (0.05 * rng.standard_normal((N, K))).astype(np.float32)
+    b = rng.standard_normal(N).astype(np.float32)
+    Y = np.full((M, N), 7, np.float32)
+    Ys = np.zeros((M, N), np.float32)
+    z = np.zeros(N, np.float32)
+    v = kat.kat_split_gemm(fp(X), fp(W), fp(b), fp(Y), M, N, K, N, 0, 0, M, 4,
+                           float(np.abs(X).max()), fp(z), fp(z), fp(Ys))
+    assert v == 0
+    want = X.astype(np.float64) @ W.T.astype(np.float64) + b
+    assert np.linalg.norm(Y - want) <= 1e-6 * np.linalg.norm(want)
+    # two fp16 halves of a value hold it to one unit of fp32's last place
+    assert (np.abs(Ys - Y) <= 2 * U * np.abs(Y) + 2.0 ** -25 / 32).all()
+
+
+def attention64(qkv, H):
+    B, T, C3 = qkv.shape
+    q, k, v = (a.reshape(B, T, H, -1).transpose(0, 2, 1, 3) for a in np.split(qkv.astype(np.float64), 3, 2))
+    s = q @ k.transpose(0, 1, 3, 2) / np.sqrt(q.shape[-1])
+    s[:, :, np.triu(np.ones((T, T), bool), 1)] = -np.inf
+    p = np.exp(s - s.max(-1, keepdims=True))
+    return (p / p.sum(-1, keepdims=True) @ v).transpose(0, 2, 1, 3).reshape(B, T, C3 // 3)
+
+
+# head sizes; query and key tiles' edges; scores near zero, ordinary and far
+# apart (large ones, where most probabilities vanish, and rows whose maximum
+# grows from tile to tile)
+@pytest.mark.parametrize("B,T,H,hs", [(1, 1, 2, 64), (2, 31, 3, 32), (1, 64, 2, 64), (3, 65, 1, 128),
+                                      (1, 127, 2, 128), (2, 128, 2, 32), (1, 129, 3, 64), (1, 700, 2, 64)])
+@pytest.mark.parametrize("size", [1e-3, 1.0, 6.0])
+def test_split_attention(kat, B, T, H, hs, size):
+    rng = np.random.default_rng(T)
+    C = H * hs
+    qkv = rng.standard_normal((B, T, 3 * C)).astype(np.float32)
+    qkv[..., :C] *= size
+    qkv[..., C:2 * C] *= np.linspace(0.1, 2, T, dtype=np.float32)[None, :, None]
+    out = np.zeros((B, T, C), np.float32)
+    smax = np.array([np.abs(a).max() * 20 for a in np.split(qkv, 3, 2)], np.float32)
+    assert kat.kat_attention_split(fp(qkv), fp(out), B, T, C, H, fp(smax)) == 0
+    want = attention64(qkv, H)
+    # a score s is off by at most (3 hs + 8) u sum|q k| / sqrt(hs), its
+    # probability by that times itself; PV adds (3 T + 16) u of sum p |v|
+    q, k, v = np.split(np.abs(qkv.astype(np.float64)), 3, 2)
+    smag = max(np.einsum("td,sd->ts", q[b][:, h * hs:(h + 1) * hs], k[b][:, h * hs:(h + 1) * hs]).max()
+               for b in range(B) for h in range(H)) / np.sqrt(hs)
+    bound = ((3 * hs + 8) * smag + 3 * T + 32) * U * 2 * v.max()
+    err = np.abs(out - want)
+    assert (err <= bound).all(), (err.max(), bound)
+    rel = np.linalg.norm(out - want) / np.linalg.norm(want)
+    print(f"B{B} T{T} H{H} hs{hs} size {size}: rel {rel:.2e}, worst {err.max() / bound:.3f} of the bound")
+    # (a wrong half of any value would show as 2^-11 of it)
+    assert rel <= (5e-7 if size <= 1 else 4e-6)
+    assert err.max() <= 2.0 ** -16 * v.max()
 
 
 def test_verdict(kat):
