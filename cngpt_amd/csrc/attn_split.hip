@@ -9,9 +9,6 @@
 
 namespace {
 
-typedef __fp16 h16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) h16x4 lds_h16x4;
-
 // hi and lo operands of 8 values
 struct Pair8 {
     f16x8 h, l;
@@ -30,21 +27,6 @@ __device__ __forceinline__ Pair8 split8(const float (&v)[8]) {
 
 __device__ __forceinline__ f32x16 mfma(const f16x8& a, const f16x8& b, const f32x16& c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
-// Rows r and r + 4 of a 4-row x 16-lane corner turn: each lane reads 8 bytes
-// of its row (ds_read_b64_tr_b16: within 16 lanes, lane s reads row s / 4, four
-// halves from 4 (s % 4); lane i receives half i of the four rows).
-__device__ __forceinline__ f16x8 read_turned(const char* p, int second) {
-    const h16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_h16x4*)p);
-    const h16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_h16x4*)(p + second));
-    f16x8 r;
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        r[e] = (_Float16)a[e];
-        r[4 + e] = (_Float16)b[e];
-    }
-    return r;
 }
 
 // One workgroup = 4 wavefronts = 128 queries of one (sequence, head). The qkv

@@ -112,6 +112,14 @@ struct SplitGemmArgs {
     const float* ln_b;
     float* ln_out;
     const float* ln_scale;
+    // launch_split_train only (X and W with one scale each, winv unused): the
+    // bits of the operands' largest magnitudes; K-major operands as in GemmArgs
+    // (km 2 or 3, rows of ldx / ldw values, multiples of 8; K rows of each); the
+    // bits of the largest |Y|, raised in *amax (EPI_STORE; null: not wanted).
+    const unsigned *xmax, *wmax;
+    int km;
+    long ldx, ldw;
+    unsigned* amax;
 };
 hipError_t launch_split_gemm(const SplitGemmArgs& a, hipStream_t s);
 int launch_split_gemm_splits(const SplitGemmArgs& a);
@@ -134,6 +142,43 @@ hipError_t launch_split_scales(const LayerW* d_layers, const LayerW* layers, con
 hipError_t launch_split_w(const float* W, const SplitWeights& o, int N, int K, const float* typ,
                           const float* typ_b, const float* bound, const float* scale, int* bad,
                           hipStream_t s);
+
+// split_train.hip: the training backward's products over operands that carry one
+// scale each (a power of two from the tensor's largest magnitude): km 2 with
+// EPI_STORE, km 3 with EPI_RESID; odd rows of X, with km 3 also of W, negated.
+hipError_t launch_split_train(const SplitGemmArgs& a, hipStream_t s);
+// A tensor to be split: n values (a multiple of 8) of src into dst (may be src), the
+// bits of the largest magnitude at amax. alt: the row length of activations and
+// gradients, whose odd rows are stored negated (split_train.hip), 0 for weights;
+// for those also the row length and room for the columns' largest magnitudes.
+struct SplitTensor {
+    const float* src;
+    float* dst;
+    long n;
+    unsigned* amax;
+    int alt;
+    int K;
+    unsigned* colmax;
+};
+// `count` weight matrices described on the device (colmax: all their columns,
+// ncol in one array): raises each *amax (cleared before) to the largest magnitude,
+// then splits it. *bad becomes non-zero where a column is too far below the
+// largest for one scale.
+hipError_t launch_split_weights(const SplitTensor* d, int count, unsigned* colmax, long ncol, int* bad,
+                                hipStream_t s);
+// One tensor; without measure, *amax is known already.
+hipError_t launch_split_tensor(const SplitTensor& t, bool measure, hipStream_t s);
+// Clears n slots and sets slot `at` (-1: none) to the bits of v.
+hipError_t launch_split_slots(unsigned* slots, long n, int at, float v, hipStream_t s);
+// Bounds of every LayerNorm's outputs, as bits: layer l's at 2 l and 2 l + 1, the
+// last one's at 2 L.
+hipError_t launch_split_ln(const LayerW* layers, const float* lnf_w, const float* lnf_b, int L, int C,
+                           unsigned* amax, hipStream_t s);
+// The gradient through GELU: d (n values in rows of `cols`, a multiple of 8) in place
+// and as split rows (odd ones negated), *amax of the incoming gradient (the outgoing one is at most 1.13 times
+// larger, which the scale leaves room for).
+hipError_t launch_split_gelu_bwd(float* d, const float* x, float* ds, long n, int cols,
+                                 const unsigned* amax, hipStream_t s);
 
 // decode.hip
 // Partials of the split one-query attention, merged by their consumer:
@@ -340,14 +385,18 @@ hipError_t launch_attention_proj(const float* qkv, long seq_stride, const float*
 // [0, V) are clamped and reported through *err (bit 2).
 // dl != 0 (probs 0): the logits stay, and dl [rows][ldd] (ldd >= V, a
 // multiple of 4) gets the mean loss's gradient (p - onehot) / rows, zero in
-// columns V .. ldd-1.
+// columns V .. ldd-1; dl_split (may be null) gets it as split rows (odd ones negated; ldd
+// a multiple of 8, *dl_amax the bits of a bound of its magnitudes).
 hipError_t launch_cross_entropy(float* logits, long rows, int V, const int* targets,
                                 float* row_loss, float* loss, int probs, int* err, hipStream_t s,
-                                float* dl = nullptr, long ldd = 0);
+                                float* dl = nullptr, long ldd = 0,
+                                float* dl_split = nullptr, const unsigned* dl_amax = nullptr);
 
 // train.hip: the training step's elementwise, row and reduction kernels.
-// out = gelu(in); d = d * gelu'(x) (n a multiple of 4).
-hipError_t launch_gelu_fwd(const float* in, float* out, long n, hipStream_t s);
+// out = gelu(in) (with amax, *amax raised to the bits of the largest |out|); d = d *
+// gelu'(x) (n a multiple of 4).
+hipError_t launch_gelu_fwd(const float* in, float* out, long n, hipStream_t s,
+                           unsigned* amax = nullptr);
 hipError_t launch_gelu_bwd(float* d, const float* x, long n, hipStream_t s);
 // x[i] *= mask[i] ? scale : 0 (dropout_fwd / dropout_bwd's scaling, the
 // bytes of mask 0 or 1; n a multiple of 4, mask 4-byte aligned).

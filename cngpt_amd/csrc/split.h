@@ -51,3 +51,76 @@ __device__ __forceinline__ u32x4 split_quad(const f32x4& v, int lane) {
     const unsigned r1 = __builtin_amdgcn_mov_dpp(s1, 0xB1, 0xF, 0xF, false);
     return odd ? u32x4{r0, r1, l0, l1} : u32x4{h0, h1, r0, r1};
 }
+
+typedef __fp16 h16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) h16x4 lds_h16x4;
+
+// Rows r and r + 4 of a 4-row x 16-lane corner turn: each lane reads 8 bytes
+// of its row (ds_read_b64_tr_b16: within 16 lanes, lane s reads row s / 4, four
+// halves from 4 (s % 4); lane i receives half i of the four rows).
+__device__ __forceinline__ f16x8 read_turned(const char* p, int second) {
+    const h16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_h16x4*)p);
+    const h16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_h16x4*)(p + second));
+    f16x8 r;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        r[e] = (_Float16)a[e];
+        r[4 + e] = (_Float16)b[e];
+    }
+    return r;
+}
+
+// The scale of a tensor whose largest magnitude has the bits amax: the power of
+// two that takes it into [2^14, 2^15) (exponents held where the scale and its
+// inverse are normal), 1 for zero, infinity and NaN.
+__device__ __forceinline__ float split_scale(unsigned amax) {
+    if (amax == 0 || amax >= 0x7f800000u) return 1.f;
+    const int e = min(14 - ((int)(amax >> 23) - 127), 100);
+    return __builtin_bit_cast(float, (unsigned)(e + 127) << 23);
+}
+__device__ __forceinline__ float split_unscale(unsigned amax) {
+    return __builtin_bit_cast(float, (254u << 23) - __builtin_bit_cast(unsigned, split_scale(amax)));
+}
+
+// Largest magnitude of four values, as bits (ordered as the values are, NaN
+// above infinity), and the wavefront's into *dst (no order: a maximum).
+__device__ __forceinline__ unsigned abs_bits(const f32x4& v) {
+    unsigned m = 0;
+#pragma unroll
+    for (int e = 0; e < 4; e++) m = max(m, __builtin_bit_cast(unsigned, (float)v[e]) & 0x7fffffffu);
+    return m;
+}
+__device__ __forceinline__ void wave_atomic_max(unsigned* dst, unsigned v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = max(v, (unsigned)__shfl_xor((int)v, o, 64));
+    if ((threadIdx.x & 63) == 0 && v) atomicMax(dst, v);
+}
+// The same of a workgroup of NW wavefronts.
+template <int NW>
+__device__ __forceinline__ void block_atomic_max(unsigned* dst, unsigned v) {
+    __shared__ unsigned red[NW];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = max(v, (unsigned)__shfl_xor((int)v, o, 64));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < NW; w++) v = max(v, red[w]);
+        if (v) atomicMax(dst, v);
+    }
+}
+
+// Eight values times sc as the two granules of an octet.
+__device__ __forceinline__ void split_octet(const f32x4& a, const f32x4& b, float sc, u32x4& hi,
+                                            u32x4& lo) {
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+        unsigned h, l;
+        split_pair(a[2 * e] * sc, a[2 * e + 1] * sc, h, l);
+        hi[e] = h;
+        lo[e] = l;
+        split_pair(b[2 * e] * sc, b[2 * e + 1] * sc, h, l);
+        hi[2 + e] = h;
+        lo[2 + e] = l;
+    }
+}

@@ -7,8 +7,11 @@
 // formed as partial sums of fixed row chunks, then the chunks are summed in
 // order by a second launch (no atomics), so repeated steps give the same
 // bits.
+#include <algorithm>
+
 #include "common.h"
 #include "kernels.h"
+#include "split.h"
 
 namespace {
 
@@ -22,6 +25,21 @@ __global__ void __launch_bounds__(256) k_gelu_fwd(const f32x4* __restrict__ in,
     if (i >= n4) return;
     const f32x4 v = in[i];
     out[i] = f32x4{gelu_tanh(v.x), gelu_tanh(v.y), gelu_tanh(v.z), gelu_tanh(v.w)};
+}
+// The same over few large workgroups, with *amax raised to the largest |out|: one
+// atomic a workgroup (one a wavefront of the form above took 139 us for 50 MB, the
+// atomics to one word following each other).
+__global__ void __launch_bounds__(1024) k_gelu_fwd_max(const f32x4* __restrict__ in,
+                                                       f32x4* __restrict__ out, long n4,
+                                                       unsigned* __restrict__ amax) {
+    unsigned m = 0;
+    for (long i = (long)blockIdx.x * 1024 + threadIdx.x; i < n4; i += (long)gridDim.x * 1024) {
+        const f32x4 v = in[i];
+        const f32x4 g = {gelu_tanh(v.x), gelu_tanh(v.y), gelu_tanh(v.z), gelu_tanh(v.w)};
+        out[i] = g;
+        m = max(m, abs_bits(g));
+    }
+    block_atomic_max<16>(amax, m);
 }
 
 // x[i] *= mask[i] ? scale : 0, over n4 groups of 4: dropout_fwd's scaling
@@ -39,16 +57,6 @@ __global__ void __launch_bounds__(256) k_dropout(f32x4* __restrict__ x,
     v.z *= (m & 0xff0000u) ? scale : 0.0f;
     v.w *= (m & 0xff000000u) ? scale : 0.0f;
     x[i] = v;
-}
-
-// d gelu / dx of the tanh form (reference ops.c:347-355): 0.5 (1 + t) +
-// 0.5 x (1 - t^2) u'(x), t = tanh(u), u = sqrt(2/pi) (x + 0.044715 x^3).
-__device__ __forceinline__ float gelu_grad(float x) {
-    const float k0 = 0.7978845608028654f, k1 = 0.044715f;
-    const float u = k0 * (x + k1 * (x * x * x));
-    const float t = tanhf(u);
-    const float du = k0 * (1.0f + 3.0f * k1 * x * x);
-    return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * du;
 }
 
 // d[i] = d[i] * gelu'(x[i]) (gelu_bwd, ops.c:382-422, into the buffer that
@@ -345,11 +353,15 @@ __global__ void __launch_bounds__(256) k_adamw(float* __restrict__ p, float* __r
 
 // ---------------------------------------------------------------- launchers
 
-hipError_t launch_gelu_fwd(const float* in, float* out, long n, hipStream_t s) {
+hipError_t launch_gelu_fwd(const float* in, float* out, long n, hipStream_t s, unsigned* amax) {
     if (n <= 0) return hipSuccess;
     if (n & 3) return hipErrorInvalidValue;
     const long n4 = n >> 2;
-    k_gelu_fwd<<<(unsigned)((n4 + 255) / 256), 256, 0, s>>>((const f32x4*)in, (f32x4*)out, n4);
+    if (amax)
+        k_gelu_fwd_max<<<(unsigned)std::min((n4 + 1023) / 1024, 512l), 1024, 0, s>>>(
+            (const f32x4*)in, (f32x4*)out, n4, amax);
+    else
+        k_gelu_fwd<<<(unsigned)((n4 + 255) / 256), 256, 0, s>>>((const f32x4*)in, (f32x4*)out, n4);
     return hipGetLastError();
 }
 

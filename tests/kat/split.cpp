@@ -128,6 +128,52 @@ int kat_split_gemm(const float* X, const float* W, const float* bias, float* Y, 
     return verdict;
 }
 
+// The training backward's products (launch_split_train) in Y [M][N], and the fp32
+// product of the same operands in Y32: km 2, Y = X [M][K] . W [K][ldw]; km 3, Y
+// += X [K][ldx]^T . W [K][ldw]. Returns the largest |Y| that the launch reports as
+// bits (km 2), 0 otherwise; -1 on failure.
+long kat_split_train(const float* X, const float* W, float* Y, float* Y32, int M, int N, int K, int ldx,
+                     int ldw, int km) {
+    Dev d;
+    const long nx = km == 3 ? (long)K * ldx : (long)M * K, nw = (long)K * ldw;
+    std::vector<float> zero(N, 0.f);
+    float *dx = d.put(X, nx), *dw = d.put(W, nw), *dy = d.put(Y, (size_t)M * N), *dy2 = d.put(Y32, (size_t)M * N);
+    float *dxs = d.put<float>(nullptr, nx), *dws = d.put<float>(nullptr, nw), *db = d.put(zero.data(), N);
+    float* part = d.put<float>(nullptr, 1 << 24);
+    unsigned* slot = d.put<unsigned>(nullptr, 3);
+    if (!d.ok) return -1;
+    SplitTensor tx{}, tw{};
+    tx.src = dx; tx.dst = dxs; tx.n = nx; tx.amax = slot; tx.alt = km == 3 ? ldx : K;
+    tw.src = dw; tw.dst = dws; tw.n = nw; tw.amax = slot + 1; tw.alt = km == 3 ? ldw : 0;
+    if (launch_split_tensor(tx, true, nullptr) != hipSuccess || launch_split_tensor(tw, true, nullptr) != hipSuccess)
+        return -1;
+    SplitGemmArgs a{};
+    a.X = dxs; a.W = dws; a.Y = dy; a.bias = db;
+    a.M = M; a.N = N; a.K = K;
+    a.ldy = N; a.ldx = ldx; a.ldw = ldw; a.km = km;
+    a.epi = km == 3 ? EPI_RESID : EPI_STORE;
+    a.xmax = slot; a.wmax = slot + 1;
+    if (km == 2) a.amax = slot + 2;
+    a.part = part; a.part_cap = 1 << 24;
+    if (launch_split_train(a, nullptr) != hipSuccess) return -1;
+    if (K % 32 == 0 && M > SKINNY_MAX_M) {
+        GemmArgs g{};
+        g.X = dx; g.W = dw; g.Y = dy2; g.bias = db;
+        g.M = M; g.N = N; g.K = K;
+        g.ldy = N; g.ldx = ldx; g.ldw = ldw; g.km = km;
+        g.epi = a.epi;
+        g.part = part; g.part_cap = 1 << 24;
+        if (launch_gemm(g, nullptr) != hipSuccess) return -1;
+    }
+    unsigned top = 0;
+    if (hipDeviceSynchronize() != hipSuccess ||
+        hipMemcpy(Y, dy, (size_t)M * N * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess ||
+        hipMemcpy(Y32, dy2, (size_t)M * N * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess ||
+        hipMemcpy(&top, slot + 2, sizeof(top), hipMemcpyDeviceToHost) != hipSuccess)
+        return -1;
+    return top;
+}
+
 // Causal attention over qkv [B, T, 3C] through the split kernel: out [B, T, C].
 // smax: the largest magnitude of q, k and v the scales allow for.
 int kat_attention_split(const float* qkv, float* out, int B, int T, int C, int H, const float* smax) {
