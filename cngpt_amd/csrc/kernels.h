@@ -168,8 +168,8 @@ hipError_t launch_split_weights(const SplitTensor* d, int count, unsigned* colma
                                 hipStream_t s);
 // One tensor; without measure, *amax is known already.
 hipError_t launch_split_tensor(const SplitTensor& t, bool measure, hipStream_t s);
-// Clears n slots and sets slot `at` (-1: none) to the bits of v.
-hipError_t launch_split_slots(unsigned* slots, long n, int at, float v, hipStream_t s);
+// Clears n slots.
+hipError_t launch_split_slots(unsigned* slots, long n, hipStream_t s);
 // Bounds of every LayerNorm's outputs, as bits: layer l's at 2 l and 2 l + 1, the
 // last one's at 2 L.
 hipError_t launch_split_ln(const LayerW* layers, const float* lnf_w, const float* lnf_b, int L, int C,
@@ -385,12 +385,10 @@ hipError_t launch_attention_proj(const float* qkv, long seq_stride, const float*
 // [0, V) are clamped and reported through *err (bit 2).
 // dl != 0 (probs 0): the logits stay, and dl [rows][ldd] (ldd >= V, a
 // multiple of 4) gets the mean loss's gradient (p - onehot) / rows, zero in
-// columns V .. ldd-1; dl_split (may be null) gets it as split rows (odd ones negated; ldd
-// a multiple of 8, *dl_amax the bits of a bound of its magnitudes).
+// columns V .. ldd-1.
 hipError_t launch_cross_entropy(float* logits, long rows, int V, const int* targets,
                                 float* row_loss, float* loss, int probs, int* err, hipStream_t s,
-                                float* dl = nullptr, long ldd = 0,
-                                float* dl_split = nullptr, const unsigned* dl_amax = nullptr);
+                                float* dl = nullptr, long ldd = 0);
 
 // train.hip: the training step's elementwise, row and reduction kernels.
 // out = gelu(in) (with amax, *amax raised to the bits of the largest |out|); d = d *

@@ -16,7 +16,6 @@
 // taken one by one.
 #include "common.h"
 #include "kernels.h"
-#include "split.h"
 
 namespace {
 
@@ -69,16 +68,13 @@ __device__ __forceinline__ float rescale(float m, float M) {
 // exp(x - max) * (1 / sum) (ops.c:557-566); with dl, leaves the logits and
 // writes the gradient of the mean loss instead, dl[row][v] = gscale *
 // (p_v - [v == target]) (cross_entropy_bwd, ops.c:576-589, with gscale = 1 /
-// rows), zero for V <= v < ldd (rows of ldd floats, 16-byte aligned), also as split
-// rows (odd ones negated) into dls when that is set.
+// rows), zero for V <= v < ldd (rows of ldd floats, 16-byte aligned).
 __global__ void __launch_bounds__(CE_THREADS) k_ce_rows(float* __restrict__ logits, int V,
                                                          const int* __restrict__ targets,
                                                          float* __restrict__ row_loss, int probs,
                                                          int* __restrict__ err,
                                                          float* __restrict__ dl, long ldd,
-                                                         float gscale,
-                                                         float* __restrict__ dls,
-                                                         const unsigned* __restrict__ dl_amax) {
+                                                         float gscale) {
     __shared__ float sm[CE_WAVES], ss[CE_WAVES];
     __shared__ float s_max, s_inv;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -148,8 +144,6 @@ __global__ void __launch_bounds__(CE_THREADS) k_ce_rows(float* __restrict__ logi
     const float M = s_max, inv = s_inv;
     if (dl) {
         f32x4* d4 = (f32x4*)(dl + row * ldd);
-        f32x4* s4 = (f32x4*)(dls + row * ldd);
-        const float sc = dls ? (row & 1 ? -1.f : 1.f) * split_scale(*dl_amax) : 1.f;
         for (int k = tid; k < (int)(ldd >> 2); k += CE_THREADS) {
             f32x4 g;
 #pragma unroll
@@ -158,8 +152,6 @@ __global__ void __launch_bounds__(CE_THREADS) k_ce_rows(float* __restrict__ logi
                 const float x = lg[min(v, V - 1)];
                 g[e] = v < V ? gscale * (exp_of(x - M) * inv - (v == tg ? 1.0f : 0.0f)) : 0.f;
             }
-            // (neighbouring lanes hold neighbouring quads, both or neither inside)
-            if (dls) __builtin_nontemporal_store(__builtin_bit_cast(f32x4, split_quad(g * sc, lane)), s4 + k);
             __builtin_nontemporal_store(g, d4 + k);
         }
         return;
@@ -198,12 +190,12 @@ __global__ void __launch_bounds__(MEAN_THREADS) k_ce_mean(const float* __restric
 
 hipError_t launch_cross_entropy(float* logits, long rows, int V, const int* targets,
                                 float* row_loss, float* loss, int probs, int* err, hipStream_t s,
-                                float* dl, long ldd, float* dl_split, const unsigned* dl_amax) {
+                                float* dl, long ldd) {
     if (rows <= 0 || V <= 0) return hipErrorInvalidValue;
     if (rows > 0x7fffffffL) return hipErrorInvalidValue;
-    if (dl && (probs || ldd < V || (ldd & (dl_split ? 7 : 3)))) return hipErrorInvalidValue;
+    if (dl && (probs || ldd < V || (ldd & 3))) return hipErrorInvalidValue;
     k_ce_rows<<<(unsigned)rows, CE_THREADS, 0, s>>>(logits, V, targets, row_loss, probs, err, dl,
-                                                    ldd, 1.0f / (float)rows, dl_split, dl_amax);
+                                                    ldd, 1.0f / (float)rows);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     k_ce_mean<<<1, MEAN_THREADS, 0, s>>>(row_loss, rows, loss);

@@ -4,7 +4,7 @@
 // Weights, activations and gradients change with every step, so each tensor
 // carries one power-of-two scale taken from its own largest magnitude, found on
 // the device in the same step: by the kernel that writes the tensor, from a bound
-// that its producer implies (LayerNorm, GELU's gradient, the loss), or by a pass
+// that its producer implies (LayerNorm, GELU's gradient), or by a pass
 // over it. One scale per tensor, not per row, is what lets one split copy serve both
 // products it is in, with K along its rows in one and across them in the other. A
 // value loses bits of lo once it is 2^-16 below its tensor's largest (2^-39 of that
@@ -107,9 +107,9 @@ __global__ void __launch_bounds__(256) k_weights_split(const SplitTensor* d, int
 }
 __global__ void __launch_bounds__(256) k_tensor_split(SplitTensor t) { tensor_split(t); }
 
-__global__ void __launch_bounds__(256) k_split_slots(unsigned* slots, long n, int at, float v) {
+__global__ void __launch_bounds__(256) k_split_slots(unsigned* slots, long n) {
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) slots[i] = i == at ? __builtin_bit_cast(unsigned, v) : 0u;
+    if (i < n) slots[i] = 0u;
 }
 
 // |LayerNorm(x)| <= sqrt(C) max|g| + max|b|
@@ -207,7 +207,7 @@ hipError_t launch_split_train(const SplitGemmArgs& a, hipStream_t s) {
 hipError_t launch_split_weights(const SplitTensor* d, int count, unsigned* colmax, long ncol, int* bad,
                                 hipStream_t s) {
     if (count <= 0) return hipSuccess;
-    const hipError_t e = launch_split_slots(colmax, ncol, -1, 0.f, s);
+    const hipError_t e = launch_split_slots(colmax, ncol, s);
     if (e != hipSuccess) return e;
     k_weights_max<<<dim3(32, count), 256, 0, s>>>(d);
     k_weights_split<<<dim3(256, count), 256, 0, s>>>(d, bad);
@@ -222,8 +222,8 @@ hipError_t launch_split_tensor(const SplitTensor& t, bool measure, hipStream_t s
     return hipGetLastError();
 }
 
-hipError_t launch_split_slots(unsigned* slots, long n, int at, float v, hipStream_t s) {
-    k_split_slots<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(slots, n, at, v);
+hipError_t launch_split_slots(unsigned* slots, long n, hipStream_t s) {
+    k_split_slots<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(slots, n);
     return hipGetLastError();
 }
 

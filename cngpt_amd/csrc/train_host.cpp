@@ -19,7 +19,7 @@
 // rows padded with zeros to whole product steps), and dW accumulates into
 // the gradient through the residual epilogue with a zero bias. Larger steps
 // (split_takes) form dX and dW on the fp16 matrix cores from split copies
-// (split_train.hip), all but the lm_head's dX. LayerNorm,
+// (split_train.hip), all but the lm_head's. LayerNorm,
 // GELU, cross-entropy and embedding backwards are the kernels of
 // train.hip, attention's is attn_bwd.hip. Every sum is formed in a fixed
 // order, so a step is reproducible bit for bit.
@@ -66,9 +66,8 @@ struct TrainSlots {
     int weight(int i) const { return 2 * L + 1 + i; }        // 4 l ..
     int attn(int l) const { return 6 * L + 2 + 2 * l; }
     int gelu(int l) const { return 6 * L + 3 + 2 * l; }
-    int dlog() const { return 8 * L + 2; }
-    int grad(int l, int i) const { return 8 * L + 3 + 4 * l + i; }  // d_x, d_hid, d_res1, d_qkv
-    int count() const { return 12 * L + 3; }
+    int grad(int l, int i) const { return 8 * L + 2 + 4 * l + i; }  // d_x, d_hid, d_res1, d_qkv
+    int count() const { return 12 * L + 2; }
 };
 
 struct cngpt_hip_train {
@@ -107,10 +106,10 @@ struct cngpt_hip_train {
     // by the last forward; allowed until a forward finds weights that need the
     // fp32 products. `slot` holds the tensors' largest magnitudes (TrainSlots),
     // sp_x, sp_hid and sp_qkv a layer's gradients as split rows (one per width:
-    // the padding rows of each stay zero), dlog_sp dlog's.
+    // the padding rows of each stay zero).
     bool split = false, can_split = false;
     unsigned *slot = nullptr, *colmax = nullptr;
-    float *wsp = nullptr, *sp_x = nullptr, *sp_hid = nullptr, *sp_qkv = nullptr, *dlog_sp = nullptr;
+    float *wsp = nullptr, *sp_x = nullptr, *sp_hid = nullptr, *sp_qkv = nullptr;
     SplitTensor* weights = nullptr;        // device: 4 per layer
     std::vector<SplitTensor> hweights;
 
@@ -282,7 +281,7 @@ int forward_pass(cngpt_hip_train* t, const CtxView& v) {
         return t->split ? launch_split_tensor(d, measure, s) : hipSuccess;
     };
     if (t->split) {
-        TRY(launch_split_slots(t->slot, k.count(), k.dlog(), 1.0f / (float)N, s));
+        TRY(launch_split_slots(t->slot, k.count(), s));
         TRY(launch_split_ln(v.d_layers, v.lnf_w, v.lnf_b, c.n_layer, C, t->slot, s));
         TRY(launch_split_weights(t->weights, 4 * c.n_layer, t->colmax, 7l * c.n_layer * C,
                                  t->err + 1, s));
@@ -318,12 +317,11 @@ int forward_pass(cngpt_hip_train* t, const CtxView& v) {
     TRY(launch_layernorm(x, C, v.lnf_w, v.lnf_b, t->lnf_out, C, (int)N, C, s, t->lnf_mean,
                          t->lnf_rstd));
     if (gemm(t, s, t->lnf_out, v.wte, nullptr, t->logits, N, V, C, EPI_STORE)) return -1;
-    TRY(split_rows(t->lnf_out, t->lnf_out, C, k.ln(2 * c.n_layer), false));
     // the loss, and the gradient of the mean loss for the backward
     // (cross_entropy_bwd) into the padded dlogits rows, from one read of the
     // logits
     TRY(launch_cross_entropy(t->logits, N, V, t->tgt, t->row_loss, t->loss, 0, t->err, s, t->dlog,
-                             t->Vp, t->split ? t->dlog_sp : nullptr, t->slot + k.dlog()));
+                             t->Vp));
     return 0;
 }
 
@@ -408,13 +406,15 @@ int backward_split(cngpt_hip_train* t, const CtxView& v) {
         g.src = d; g.dst = o; g.n = N * cols; g.alt = cols; g.amax = t->slot + slot;
         return launch_split_tensor(g, true, s);
     };
-    TRY(launch_split_slots(t->slot + k.grad(0, 0), 4 * L, -1, 0.f, s));
-    // the tied lm_head; its dX stays in fp32, whose sum of V products is the
+    TRY(launch_split_slots(t->slot + k.grad(0, 0), 4 * L, s));
+    // the tied lm_head stays in fp32: its dX, whose sum of V products is the
     // more accurate (gradient of the last LayerNorm's bias, V = 50257, against
-    // float64: 3.6e-6, split 6.2e-6)
+    // float64: 3.6e-6, split 6.2e-6), and its dW, whose rows are as far apart as the
+    // tokens' probabilities (one scale for all of dlogits holds a token of p = 1e-8
+    // to 9e-5 of its row, of 1e-12 not at all; fp32 to 4e-7)
     TRY(launch_transpose(v.wte, C, V, C, t->tW, t->Vp, (int)t->Vp, C, s));
     if (gemm(t, s, t->dlog, t->tW, nullptr, t->d_ln, N, C, t->Vp, EPI_STORE) ||
-        sdw(t, s, t->dlog_sp, t->Vp, k.dlog(), t->lnf_out, k.ln(2 * L), grad_of(t, v, v.wte), V, C))
+        linear_dw(t, s, t->dlog, t->Vp, t->lnf_out, grad_of(t, v, v.wte), nullptr, V, C))
         return -1;
     TRY(hipMemsetAsync(t->d_x, 0, xbytes, s));
     const float* x_last = L > 0 ? t->acts[L - 1].res2 : t->emb;
@@ -532,7 +532,6 @@ int cngpt_hip_train_create(cngpt_hip_ctx* h, int B, int T, cngpt_hip_train** out
         fl(slots.count());                    // slot
         fl(L * 7 * C);                        // colmax (columns: 3 x C and 4 C a layer)
         fl(L * 12 * C * C);                   // wsp
-        fl(Np * Vp);                          // dlog_sp
         fl(Np * C); fl(Np * 4 * C); fl(Np * 3 * C);       // sp_x, sp_hid, sp_qkv
         sz.push_back(4 * L * sizeof(SplitTensor) + 1);  // weights
         for (long l = 0; l < L; l++) fl(Np * C);          // attn_sp
@@ -577,7 +576,7 @@ int cngpt_hip_train_create(cngpt_hip_ctx* h, int B, int T, cngpt_hip_train** out
     t->part = (float*)take(); t->red = (float*)take(); t->zeros = (float*)take();
     if (t->can_split) {
         t->slot = (unsigned*)take();
-        t->colmax = (unsigned*)take(); t->wsp = (float*)take(); t->dlog_sp = (float*)take();
+        t->colmax = (unsigned*)take(); t->wsp = (float*)take();
         t->sp_x = (float*)take(); t->sp_hid = (float*)take(); t->sp_qkv = (float*)take();
         t->weights = (SplitTensor*)take();
         for (auto& a : t->acts) a.attn_sp = (float*)take();
