@@ -1481,7 +1481,6 @@ int ctx_view(cngpt_hip_ctx* h, CtxView* v) {
     v->lnf_w = h->lnf_w;
     v->lnf_b = h->lnf_b;
     v->layers = h->layers.data();
-    v->d_layers = h->d_layers;
     v->use_split = h->use_split;
     return 0;
 }

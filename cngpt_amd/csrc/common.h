@@ -121,16 +121,6 @@ __device__ __forceinline__ float gelu_tanh(float x) {
     return x * __builtin_amdgcn_rcpf(1.0f + __expf(-2.0f * u));
 }
 
-// d gelu / dx of the tanh form (reference ops.c:347-355): 0.5 (1 + t) +
-// 0.5 x (1 - t^2) u'(x), t = tanh(u), u = sqrt(2/pi) (x + 0.044715 x^3).
-__device__ __forceinline__ float gelu_grad(float x) {
-    const float k0 = 0.7978845608028654f, k1 = 0.044715f;
-    const float u = k0 * (x + k1 * (x * x * x));
-    const float t = tanhf(u);
-    const float du = k0 * (1.0f + 3.0f * k1 * x * x);
-    return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * du;
-}
-
 // Epilogues shared by the GEMM and GEMV kernels.
 enum EpiMode : int {
     EPI_STORE = 0,      // Y = acc

@@ -15,7 +15,6 @@ struct CtxView {
     long n_params;
     const float *wte, *wpe, *lnf_w, *lnf_b;
     const LayerW* layers;  // host array of n_layer views into params
-    const LayerW* d_layers;  // the same on the device
     bool use_split;          // products on the fp16 matrix cores allowed
 };
 

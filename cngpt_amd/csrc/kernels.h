@@ -112,11 +112,13 @@ struct SplitGemmArgs {
     const float* ln_b;
     float* ln_out;
     const float* ln_scale;
-    // launch_split_train only (X and W with one scale each, winv unused): the
-    // bits of the operands' largest magnitudes; K-major operands as in GemmArgs
-    // (km 2 or 3, rows of ldx / ldw values, multiples of 8; K rows of each); the
-    // bits of the largest |Y|, raised in *amax (EPI_STORE; null: not wanted).
+    // launch_split_train only (winv unused): the bits of the operands' largest
+    // magnitudes, of each whole (xstep, wstep 0) or one for each of the M rows and N
+    // columns of Y (1); K-major operands as in GemmArgs (km 2 or 3, rows of ldx / ldw
+    // values, multiples of 8; K rows of each); the bits of the largest |Y|, raised in
+    // *amax (EPI_STORE; null: not wanted).
     const unsigned *xmax, *wmax;
+    int xstep, wstep;
     int km;
     long ldx, ldw;
     unsigned* amax;
@@ -143,14 +145,13 @@ hipError_t launch_split_w(const float* W, const SplitWeights& o, int N, int K, c
                           const float* typ_b, const float* bound, const float* scale, int* bad,
                           hipStream_t s);
 
-// split_train.hip: the training backward's products over operands that carry one
-// scale each (a power of two from the tensor's largest magnitude): km 2 with
-// EPI_STORE, km 3 with EPI_RESID; odd rows of X, with km 3 also of W, negated.
+// split_train.hip: the training backward's products: km 2 with EPI_STORE, km 3
+// with EPI_RESID; odd rows of X, with km 3 also of W, negated.
 hipError_t launch_split_train(const SplitGemmArgs& a, hipStream_t s);
-// A tensor to be split: n values (a multiple of 8) of src into dst (may be src), the
-// bits of the largest magnitude at amax. alt: the row length of activations and
-// gradients, whose odd rows are stored negated (split_train.hip), 0 for weights;
-// for those also the row length and room for the columns' largest magnitudes.
+// A tensor to be split under one scale: n values (a multiple of 8) of src into dst (may
+// be src), the bits of the largest magnitude at amax. alt: the row length of
+// activations and gradients, whose odd rows are stored negated (split_train.hip), 0
+// for weights; for those also the row length and the columns' largest magnitudes.
 struct SplitTensor {
     const float* src;
     float* dst;
@@ -160,25 +161,29 @@ struct SplitTensor {
     int K;
     unsigned* colmax;
 };
-// `count` weight matrices described on the device (colmax: all their columns,
-// ncol in one array): raises each *amax (cleared before) to the largest magnitude,
-// then splits it. *bad becomes non-zero where a column is too far below the
-// largest for one scale.
-hipError_t launch_split_weights(const SplitTensor* d, int count, unsigned* colmax, long ncol, int* bad,
-                                hipStream_t s);
+// `count` weight matrices described on the device: raises each *amax and colmax
+// (cleared before) to the largest magnitudes, then splits it. *bad becomes non-zero
+// where a row or column is too far below the largest for one scale.
+hipError_t launch_split_weights(const SplitTensor* d, int count, int* bad, hipStream_t s);
 // One tensor; without measure, *amax is known already.
 hipError_t launch_split_tensor(const SplitTensor& t, bool measure, hipStream_t s);
-// Clears n slots.
-hipError_t launch_split_slots(unsigned* slots, long n, hipStream_t s);
-// Bounds of every LayerNorm's outputs, as bits: layer l's at 2 l and 2 l + 1, the
-// last one's at 2 L.
-hipError_t launch_split_ln(const LayerW* layers, const float* lnf_w, const float* lnf_b, int L, int C,
-                           unsigned* amax, hipStream_t s);
-// The gradient through GELU: d (n values in rows of `cols`, a multiple of 8) in place
-// and as split rows (odd ones negated), *amax of the incoming gradient (the outgoing one is at most 1.13 times
-// larger, which the scale leaves room for).
-hipError_t launch_split_gelu_bwd(float* d, const float* x, float* ds, long n, int cols,
-                                 const unsigned* amax, hipStream_t s);
+// Split copies of src [rows][cols] (cols a multiple of 8), odd rows negated: by_col
+// [rows_p][cols] with the scales of its columns' largest magnitudes (rows and up of it
+// zero), and by_row (null: none) with those of its rows', which go to rowmax.
+struct SplitRows {
+    const float* src;
+    int rows, rows_p, cols;
+    const unsigned* colmax;
+    float* by_col;
+    float* by_row;
+    unsigned* rowmax;
+};
+hipError_t launch_split_rows(const SplitRows& a, hipStream_t s);
+// Raises colmax[c] to the largest magnitude of column c of x [rows][cols] (cols a
+// multiple of 4).
+hipError_t launch_cols_max(const float* x, int rows, int cols, unsigned* colmax, hipStream_t s);
+// Clears n magnitudes.
+hipError_t launch_clear_max(unsigned* slots, long n, hipStream_t s);
 
 // decode.hip
 // Partials of the split one-query attention, merged by their consumer:
@@ -391,10 +396,8 @@ hipError_t launch_cross_entropy(float* logits, long rows, int V, const int* targ
                                 float* dl = nullptr, long ldd = 0);
 
 // train.hip: the training step's elementwise, row and reduction kernels.
-// out = gelu(in) (with amax, *amax raised to the bits of the largest |out|); d = d *
-// gelu'(x) (n a multiple of 4).
-hipError_t launch_gelu_fwd(const float* in, float* out, long n, hipStream_t s,
-                           unsigned* amax = nullptr);
+// out = gelu(in); d = d * gelu'(x) (n a multiple of 4).
+hipError_t launch_gelu_fwd(const float* in, float* out, long n, hipStream_t s);
 hipError_t launch_gelu_bwd(float* d, const float* x, long n, hipStream_t s);
 // x[i] *= mask[i] ? scale : 0 (dropout_fwd / dropout_bwd's scaling, the
 // bytes of mask 0 or 1; n a multiple of 4, mask 4-byte aligned).
@@ -405,10 +408,11 @@ hipError_t launch_dropout(float* x, const unsigned char* mask, long n, float sca
 hipError_t launch_transpose(const float* src, long lds, int rows, int cols, float* dst, long ldd,
                             int rows_p, int cols_p, hipStream_t s);
 // out[c] += sum over rows of Y[r][c] (partials of colsum_part_floats floats
-// at part, summed in row-chunk order).
+// at part, summed in row-chunk order). With colmax, colmax[c] is raised to the bits
+// of the largest magnitude of column c.
 long colsum_part_floats(int rows, int cols);
 hipError_t launch_colsum_add(const float* Y, long ldy, int rows, int cols, float* part,
-                             float* out, hipStream_t s);
+                             float* out, hipStream_t s, unsigned* colmax = nullptr);
 // The same transpose, and out[c] += the column sums of src over its rows
 // (partials of transpose_colsum_floats floats at part, summed in row order).
 long transpose_colsum_floats(int rows, int cols);

@@ -70,16 +70,14 @@ __device__ __forceinline__ f16x8 read_turned(const char* p, int second) {
     return r;
 }
 
-// The scale of a tensor whose largest magnitude has the bits amax: the power of
-// two that takes it into [2^14, 2^15) (exponents held where the scale and its
-// inverse are normal), 1 for zero, infinity and NaN.
-__device__ __forceinline__ float split_scale(unsigned amax) {
-    if (amax == 0 || amax >= 0x7f800000u) return 1.f;
-    const int e = min(14 - ((int)(amax >> 23) - 127), 100);
-    return __builtin_bit_cast(float, (unsigned)(e + 127) << 23);
+// The scale of values whose largest magnitude has the bits amax, 2 to the
+// power of this: it takes that into [2^14, 2^15) (held where the scale is a normal
+// float); 0 for zero, infinity and NaN.
+__device__ __forceinline__ int split_exp(unsigned amax) {
+    return amax - 1u < 0x7f7fffffu ? min(141 - (int)(amax >> 23), 127) : 0;
 }
-__device__ __forceinline__ float split_unscale(unsigned amax) {
-    return __builtin_bit_cast(float, (254u << 23) - __builtin_bit_cast(unsigned, split_scale(amax)));
+__device__ __forceinline__ float split_scale(unsigned amax) {
+    return __builtin_bit_cast(float, (unsigned)(split_exp(amax) + 127) << 23);
 }
 
 // Largest magnitude of four values, as bits (ordered as the values are, NaN
@@ -110,16 +108,15 @@ __device__ __forceinline__ void block_atomic_max(unsigned* dst, unsigned v) {
     }
 }
 
-// Eight values times sc as the two granules of an octet.
-__device__ __forceinline__ void split_octet(const f32x4& a, const f32x4& b, float sc, u32x4& hi,
-                                            u32x4& lo) {
+// Eight values as the two granules of an octet.
+__device__ __forceinline__ void split_octet(const f32x4& a, const f32x4& b, u32x4& hi, u32x4& lo) {
 #pragma unroll
     for (int e = 0; e < 2; e++) {
         unsigned h, l;
-        split_pair(a[2 * e] * sc, a[2 * e + 1] * sc, h, l);
+        split_pair(a[2 * e], a[2 * e + 1], h, l);
         hi[e] = h;
         lo[e] = l;
-        split_pair(b[2 * e] * sc, b[2 * e + 1] * sc, h, l);
+        split_pair(b[2 * e], b[2 * e + 1], h, l);
         hi[2 + e] = h;
         lo[2 + e] = l;
     }

@@ -65,7 +65,8 @@ __device__ __forceinline__ float epi_value(float v, float b, float old) {
 // K split over workgroups, partials to a.part + ks M N.
 //
 // KM >= 0 (the training backward): each operand carries one scale, that of
-// split_scale of *a.xmax and *a.wmax, and a K-major operand (KM & 1: X, KM & 2:
+// split_scale of *a.xmax and *a.wmax, or (xstep, wstep 1) one for each row and
+// column of Y, and a K-major operand (KM & 1: X, KM & 2:
 // W; rows of ldx / ldw values, one per k) is used as it is stored: a stage
 // holds 16 of its rows, TM / 4 (TN / 4) granules each, and the reads turn 4 x 16
 // corners of it (read_turned) into the lanes' eight k. Granules are XORed with
@@ -241,12 +242,6 @@ __global__ void __launch_bounds__(64 * WR * WC, OCC * WR * WC / 4)
     }
     if (kt < nk) step(kt, o0, o1, std::false_type{});
 
-    float inv_x = 1.f, inv_w = 1.f;
-    if constexpr (KM >= 0) {
-        inv_x = split_unscale(*a.xmax);
-        if (KM == 2 && (lr & 1)) inv_x = -inv_x;  // (odd rows are stored negated)
-        inv_w = split_unscale(*a.wmax);
-    }
     if constexpr (VEC) {
         unsigned top = 0;
         // acc[i][j][4 g + e]: row m0 + wm + 32 i + lane % 32, column n0 + wn
@@ -256,25 +251,38 @@ __global__ void __launch_bounds__(64 * WR * WC, OCC * WR * WC / 4)
         // counter counts both).
         const bool part = EPI == EPI_STORE && KS > 1;
         float *yrow[2], *srow[2];
+        const float sign = KM == 2 && (lr & 1) ? -1.f : 1.f;  // (odd rows are stored negated)
+        int ex[2] = {0, 0};                                   // exponents that undo the scales
+        int ew[2][4][4];
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             const int row = min(m0 + wm + 32 * i + lr, a.M - 1);
             srow[i] = EPI == EPI_QKV ? a.Ys + (long)row * a.N : nullptr;
             const long orow = a.seg ? (long)(row / a.seg) * a.seg_stride + row % a.seg : row;
             yrow[i] = part ? a.part + ((long)ks * a.M + row) * a.N : a.Y + orow * a.ldy;
+            if (KM >= 0) ex[i] = -split_exp(a.xmax[row * a.xstep]);
         }
         const float os0 = OUT_SPLIT ? a.out_scale[0] : 1.f;
         const float os1 = EPI == EPI_QKV ? a.out_scale[1] : 1.f;
         const float os2 = EPI == EPI_QKV ? a.out_scale[2] : 1.f;
         const int third = a.N / 3;
+        constexpr bool BIAS = EPI != EPI_STORE && KM < 0;  // (the backward's is zero)
         constexpr bool AHEAD = EPI != EPI_RESID || OCC < 3;  // (three per CU: registers)
         f32x4 s[2][4], b[2][4], old[2][2][4];
         auto load = [&](int j, int t) {
 #pragma unroll
             for (int g = 0; g < 4; g++) {
                 const int c = min(n0 + wn + 32 * j + 4 * lh + 8 * g, a.N - 4);
-                if (KM < 0) s[t][g] = *(const f32x4*)(a.winv + c);
-                if (EPI != EPI_STORE) b[t][g] = *(const f32x4*)(a.bias + c);
+                if constexpr (KM < 0) {
+                    s[t][g] = *(const f32x4*)(a.winv + c);
+                } else {
+                    u32x4 u;
+                    if (a.wstep) u = *(const u32x4*)(a.wmax + c);
+                    else u = u32x4{*a.wmax, *a.wmax, *a.wmax, *a.wmax};
+#pragma unroll
+                    for (int e = 0; e < 4; e++) ew[t][g][e] = -split_exp(u[e]);
+                }
+                if (BIAS) b[t][g] = *(const f32x4*)(a.bias + c);
                 if (EPI == EPI_RESID)
 #pragma unroll
                     for (int i = 0; i < 2; i++) old[t][i][g] = *(const f32x4*)(yrow[i] + c);
@@ -295,9 +303,10 @@ __global__ void __launch_bounds__(64 * WR * WC, OCC * WR * WC / 4)
                     f32x4 v;
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        const float y = KM >= 0 ? acc[i][j][4 * g + e] * inv_x * inv_w
+                        const float y = KM >= 0 ? __builtin_amdgcn_ldexpf(acc[i][j][4 * g + e] * sign,
+                                                                          ex[i] + ew[t][g][e])
                                                 : acc[i][j][4 * g + e] * s[t][g][e];
-                        v[e] = epi_value<EPI>(y, EPI == EPI_STORE ? 0.f : b[t][g][e],
+                        v[e] = epi_value<EPI>(y, BIAS ? b[t][g][e] : 0.f,
                                               EPI == EPI_RESID ? old[t][i][g][e] : 0.f);
                     }
                     if constexpr (OUT_SPLIT) {

@@ -7,11 +7,8 @@
 // formed as partial sums of fixed row chunks, then the chunks are summed in
 // order by a second launch (no atomics), so repeated steps give the same
 // bits.
-#include <algorithm>
-
 #include "common.h"
 #include "kernels.h"
-#include "split.h"
 
 namespace {
 
@@ -25,21 +22,6 @@ __global__ void __launch_bounds__(256) k_gelu_fwd(const f32x4* __restrict__ in,
     if (i >= n4) return;
     const f32x4 v = in[i];
     out[i] = f32x4{gelu_tanh(v.x), gelu_tanh(v.y), gelu_tanh(v.z), gelu_tanh(v.w)};
-}
-// The same over few large workgroups, with *amax raised to the largest |out|: one
-// atomic a workgroup (one a wavefront of the form above took 139 us for 50 MB, the
-// atomics to one word following each other).
-__global__ void __launch_bounds__(1024) k_gelu_fwd_max(const f32x4* __restrict__ in,
-                                                       f32x4* __restrict__ out, long n4,
-                                                       unsigned* __restrict__ amax) {
-    unsigned m = 0;
-    for (long i = (long)blockIdx.x * 1024 + threadIdx.x; i < n4; i += (long)gridDim.x * 1024) {
-        const f32x4 v = in[i];
-        const f32x4 g = {gelu_tanh(v.x), gelu_tanh(v.y), gelu_tanh(v.z), gelu_tanh(v.w)};
-        out[i] = g;
-        m = max(m, abs_bits(g));
-    }
-    block_atomic_max<16>(amax, m);
 }
 
 // x[i] *= mask[i] ? scale : 0, over n4 groups of 4: dropout_fwd's scaling
@@ -57,6 +39,16 @@ __global__ void __launch_bounds__(256) k_dropout(f32x4* __restrict__ x,
     v.z *= (m & 0xff0000u) ? scale : 0.0f;
     v.w *= (m & 0xff000000u) ? scale : 0.0f;
     x[i] = v;
+}
+
+// d gelu / dx of the tanh form (reference ops.c:347-355): 0.5 (1 + t) +
+// 0.5 x (1 - t^2) u'(x), t = tanh(u), u = sqrt(2/pi) (x + 0.044715 x^3).
+__device__ __forceinline__ float gelu_grad(float x) {
+    const float k0 = 0.7978845608028654f, k1 = 0.044715f;
+    const float u = k0 * (x + k1 * (x * x * x));
+    const float t = tanhf(u);
+    const float du = k0 * (1.0f + 3.0f * k1 * x * x);
+    return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * du;
 }
 
 // d[i] = d[i] * gelu'(x[i]) (gelu_bwd, ops.c:382-422, into the buffer that
@@ -117,14 +109,16 @@ __global__ void __launch_bounds__(256) k_transpose(const float* __restrict__ src
 constexpr int CS_ROWS = 64;  // rows per partial column sum
 
 // part[chunk][c] = sum of Y[r][c] over the chunk's CS_ROWS rows, in order
-// (eight loads in flight per thread).
+// (eight loads in flight per thread), and the chunk's largest magnitude into colmax[c].
 __global__ void __launch_bounds__(256) k_colsum_part(const float* __restrict__ Y, long ldy,
                                                      int rows, int cols,
-                                                     float* __restrict__ part) {
+                                                     float* __restrict__ part,
+                                                     unsigned* __restrict__ colmax) {
     const int c = blockIdx.x * 256 + threadIdx.x;
     if (c >= cols) return;
     const int r0 = blockIdx.y * CS_ROWS, r1 = min(rows, r0 + CS_ROWS);
     float s = 0.f;
+    unsigned m = 0;
     for (int r = r0; r < r1; r += 8) {
         float v[8];
 #pragma unroll
@@ -132,8 +126,11 @@ __global__ void __launch_bounds__(256) k_colsum_part(const float* __restrict__ Y
 #pragma unroll
         for (int j = 0; j < 8; j++)
             if (r + j < r1) s += v[j];
+#pragma unroll
+        for (int j = 0; j < 8; j++) m = max(m, __builtin_bit_cast(unsigned, v[j]) & 0x7fffffffu);
     }
     part[(long)blockIdx.y * cols + c] = s;
+    if (colmax && m) atomicMax(colmax + c, m);
 }
 
 // out[c] += sum over the nparts partials of column c: eight threads per
@@ -353,15 +350,11 @@ __global__ void __launch_bounds__(256) k_adamw(float* __restrict__ p, float* __r
 
 // ---------------------------------------------------------------- launchers
 
-hipError_t launch_gelu_fwd(const float* in, float* out, long n, hipStream_t s, unsigned* amax) {
+hipError_t launch_gelu_fwd(const float* in, float* out, long n, hipStream_t s) {
     if (n <= 0) return hipSuccess;
     if (n & 3) return hipErrorInvalidValue;
     const long n4 = n >> 2;
-    if (amax)
-        k_gelu_fwd_max<<<(unsigned)std::min((n4 + 1023) / 1024, 512l), 1024, 0, s>>>(
-            (const f32x4*)in, (f32x4*)out, n4, amax);
-    else
-        k_gelu_fwd<<<(unsigned)((n4 + 255) / 256), 256, 0, s>>>((const f32x4*)in, (f32x4*)out, n4);
+    k_gelu_fwd<<<(unsigned)((n4 + 255) / 256), 256, 0, s>>>((const f32x4*)in, (f32x4*)out, n4);
     return hipGetLastError();
 }
 
@@ -413,10 +406,10 @@ long colsum_part_floats(int rows, int cols) {
 }
 
 hipError_t launch_colsum_add(const float* Y, long ldy, int rows, int cols, float* part,
-                             float* out, hipStream_t s) {
+                             float* out, hipStream_t s, unsigned* colmax) {
     if (rows <= 0 || cols <= 0) return hipSuccess;
     const int nparts = (rows + CS_ROWS - 1) / CS_ROWS;
-    k_colsum_part<<<dim3((cols + 255) / 256, nparts), 256, 0, s>>>(Y, ldy, rows, cols, part);
+    k_colsum_part<<<dim3((cols + 255) / 256, nparts), 256, 0, s>>>(Y, ldy, rows, cols, part, colmax);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     k_colsum_fin<<<(cols + 31) / 32, 256, 0, s>>>(part, nparts, cols, out);

@@ -18,8 +18,8 @@
 // is a row index is transposed first (W for dX; dY and X for dW, their
 // rows padded with zeros to whole product steps), and dW accumulates into
 // the gradient through the residual epilogue with a zero bias. Larger steps
-// (split_takes) form dX and dW on the fp16 matrix cores from split copies
-// (split_train.hip), all but the lm_head's. LayerNorm,
+// (split_takes) form the layers' dX and dW on the fp16 matrix cores from split copies
+// (split_train.hip). LayerNorm,
 // GELU, cross-entropy and embedding backwards are the kernels of
 // train.hip, attention's is attn_bwd.hip. Every sum is formed in a fixed
 // order, so a step is reproducible bit for bit.
@@ -56,18 +56,6 @@ long round_up(long n, long m) { return (n + m - 1) / m * m; }
 struct TrainLayer {
     float *ln1_out, *ln1_mean, *ln1_rstd, *qkv, *lse, *attn_out, *res1;
     float *ln2_out, *ln2_mean, *ln2_rstd, *fc_out, *gelu, *res2;
-    float* attn_sp;  // attn_out as split rows
-};
-
-// Places in cngpt_hip_train::slot for L layers (LayerNorms' first: launch_split_ln)
-struct TrainSlots {
-    int L;
-    int ln(int i) const { return i; }                        // 2 l, 2 l + 1, 2 L
-    int weight(int i) const { return 2 * L + 1 + i; }        // 4 l ..
-    int attn(int l) const { return 6 * L + 2 + 2 * l; }
-    int gelu(int l) const { return 6 * L + 3 + 2 * l; }
-    int grad(int l, int i) const { return 8 * L + 2 + 4 * l + i; }  // d_x, d_hid, d_res1, d_qkv
-    int count() const { return 12 * L + 2; }
 };
 
 struct cngpt_hip_train {
@@ -102,16 +90,21 @@ struct cngpt_hip_train {
     float *norm = nullptr, *coef = nullptr;
     bool have_fwd = false;
 
-    // The backward's products on the fp16 matrix cores (split_train.hip): prepared
-    // by the last forward; allowed until a forward finds weights that need the
-    // fp32 products. `slot` holds the tensors' largest magnitudes (TrainSlots),
-    // sp_x, sp_hid and sp_qkv a layer's gradients as split rows (one per width:
-    // the padding rows of each stay zero).
-    bool split = false, can_split = false;
-    unsigned *slot = nullptr, *colmax = nullptr;
-    float *wsp = nullptr, *sp_x = nullptr, *sp_hid = nullptr, *sp_qkv = nullptr;
-    SplitTensor* weights = nullptr;        // device: 4 per layer
+    // The backward's products on the fp16 matrix cores (split_train.hip), until a
+    // backward finds weights that need the fp32 products. wsp holds the layers'
+    // weights as split rows (weights / hweights: 4 a layer); y_col, y_row and x_col the
+    // operands of the products being formed, rmax the rows' largest magnitudes of
+    // y_row. maxima, cleared by each backward: of the weights, of their columns (7 C a
+    // layer) and, from colmax on, of the columns of the gradients and activations (16 C
+    // a layer).
+    bool can_split = false;
+    unsigned *maxima = nullptr, *colmax = nullptr, *rmax = nullptr;
+    long n_maxima = 0;
+    float *wsp = nullptr, *y_col = nullptr, *y_row = nullptr, *x_col = nullptr;
+    SplitTensor* weights = nullptr;
     std::vector<SplitTensor> hweights;
+    int* verdict = nullptr;        // pinned: not zero where the weights do not fit
+    hipEvent_t judged = nullptr;   // it has arrived
 
     // GPTConfig.dropout (model.h:43): the keep masks of the last forward,
     // [1 + 2 L][B T C] bytes (the embedding, then res1 and res2 of each
@@ -153,53 +146,47 @@ int gemm(cngpt_hip_train* t, hipStream_t s, const float* X, const float* W, cons
     return 0;
 }
 
-// Split products (launch_split_train), the operands' largest magnitudes at two
-// slots. dX [rows, in] = dY [rows, out] . W [out, in], W read K-major.
-int sdx(cngpt_hip_train* t, hipStream_t s, const float* dY, int y, const float* W, int w, float* dX,
-        long out, long in, unsigned* amax = nullptr) {
+// A linear layer's backward by split products (launch_split_train): from dY [N, out]
+// and X [N, in], dX [N, in] = dY . W (the split weights w, K-major), dW [out, in] +=
+// dY^T . X (both K-major) and db += column sums of dY. col: the columns' largest
+// magnitudes, of dY (found with its sums) and then of X; takes out + in of them.
+int slinear_bwd(cngpt_hip_train* t, hipStream_t s, const float* dY, const float* X,
+                const SplitTensor& w, float* dX, float* dW, float* db, long out, long in,
+                unsigned*& col) {
+    const int N = (int)t->N, Np = (int)t->Np;
+    unsigned *ymax = col, *xmax = col + out;
+    col += out + in;
+    TRY(launch_colsum_add(dY, out, N, (int)out, t->red, db, s, ymax));
+    TRY(launch_split_rows({dY, N, Np, (int)out, ymax, t->y_col, t->y_row, t->rmax}, s));
+    TRY(launch_cols_max(X, N, (int)in, xmax, s));
+    TRY(launch_split_rows({X, N, Np, (int)in, xmax, t->x_col, nullptr, nullptr}, s));
     SplitGemmArgs a{};
-    a.X = dY; a.W = W; a.Y = dX;
-    a.M = (int)t->N; a.N = (int)in; a.K = (int)out;
+    a.X = t->y_row; a.W = w.dst; a.Y = dX;
+    a.M = N; a.N = (int)in; a.K = (int)out;
     a.ldy = in; a.ldw = in; a.km = 2;
     a.epi = EPI_STORE;
-    a.xmax = t->slot + y; a.wmax = t->slot + w;
-    a.amax = amax;
+    a.xmax = t->rmax; a.xstep = 1;
+    a.wmax = w.amax;
     a.part = t->part; a.part_cap = PART_FLOATS;
     TRY(launch_split_train(a, s));
+    SplitGemmArgs d{};
+    d.X = t->y_col; d.W = t->x_col; d.Y = dW; d.bias = t->zeros;
+    d.M = (int)out; d.N = (int)in; d.K = Np;
+    d.ldy = in; d.ldx = out; d.ldw = in; d.km = 3;
+    d.epi = EPI_RESID;
+    d.xmax = ymax; d.wmax = xmax;
+    d.xstep = d.wstep = 1;
+    d.part = t->part; d.part_cap = PART_FLOATS;
+    TRY(launch_split_train(d, s));
     return 0;
-}
-// dW [out, in] += dY^T . X, both read K-major (rows of ldy and `in` values, N ..
-// Np-1 of them zero).
-int sdw(cngpt_hip_train* t, hipStream_t s, const float* dY, long ldy, int y, const float* X, int x,
-        float* dW, long out, long in) {
-    SplitGemmArgs a{};
-    a.X = dY; a.W = X; a.Y = dW; a.bias = t->zeros;
-    a.M = (int)out; a.N = (int)in; a.K = (int)t->Np;
-    a.ldy = in; a.ldx = ldy; a.ldw = in; a.km = 3;
-    a.epi = EPI_RESID;
-    a.xmax = t->slot + y; a.wmax = t->slot + x;
-    a.part = t->part; a.part_cap = PART_FLOATS;
-    TRY(launch_split_train(a, s));
-    return 0;
-}
-// A linear layer's backward: dY (fp32, for the bias gradient, and as split rows)
-// to dX, dW and db.
-int slinear_bwd(cngpt_hip_train* t, hipStream_t s, const float* dY, const float* dYs, int y,
-                const float* X, int x, int w, float* dX, float* dW, float* db, long out, long in,
-                unsigned* amax = nullptr) {
-    const float* Ws = t->hweights[w - TrainSlots{t->cfg.n_layer}.weight(0)].dst;
-    TRY(launch_colsum_add(dY, out, (int)t->N, (int)out, t->red, db, s));
-    return sdx(t, s, dYs, y, Ws, w, dX, out, in, amax) || sdw(t, s, dYs, out, y, X, x, dW, out, in)
-               ? -1
-               : 0;
 }
 
 // Whether the backward's products go to the fp16 matrix cores: rows of whole octets
 // and steps, and enough work to pay for the splits' launches (a forward and
-// backward of 3 layers, us, fp32 against split: C = 512, 768 rows 1537 / 1574, 1536
-// rows 1894 / 1844; C = 768, 384 rows 1696 / 1704, 768 rows 2097 / 1948, 4096 rows
-// 5949 / 4588; C = 1600, 256 rows 2547 / 2574, 384 rows 3296 / 3024, 4096 rows 21949
-// / 13777; C = 256 at no size up to 4096 rows).
+// backward of 3 layers, us, fp32 against split: C = 512, 768 rows 1607 / 1609, 1152
+// rows 1768 / 1766-1784, 1536 rows 1949 / 1929; C = 768, 384 rows 1635 / 1632, 768 rows
+// 2177 / 2080, 4096 rows 6450 / 5550; C = 1600, 256 rows 2566 / 2561, 384 rows 3273 /
+// 3162, 1024 rows 6700 / 5420; C = 256, 4096 rows 2012 / 2010).
 bool split_takes(const CtxView& v, long N) {
     const long C = v.cfg.n_embd;
     return v.use_split && C % 16 == 0 && C >= 512 && N * C >= 768l * 768;
@@ -255,206 +242,21 @@ int linear_dw(cngpt_hip_train* t, hipStream_t s, const float* dY, long ldy, cons
     return gemm(t, s, t->tA, t->tB, t->zeros, dW, out, in, Np, EPI_RESID);
 }
 
+// The split copies of the layers' weights for this backward, and the verdict on
+// them (split_train.hip) on its way to the host.
+int split_weights(cngpt_hip_train* t, hipStream_t s) {
+    TRY(launch_clear_max(t->maxima, t->n_maxima, s));
+    TRY(launch_split_weights(t->weights, (int)t->hweights.size(), t->err + 1, s));
+    TRY(hipMemcpyAsync(t->verdict, t->err + 1, sizeof(int), hipMemcpyDeviceToHost, s));
+    TRY(hipEventRecord(t->judged, s));
+    return 0;
+}
+
 int check_ids(const int* ids, long n, int V, const char* what) {
     if (!ids) return ctx_fail("null %s", what);
     for (long i = 0; i < n; i++)
         if (ids[i] < 0 || ids[i] >= V)
             return ctx_fail("%s %d at index %ld outside [0, %d)", what, ids[i], i, V);
-    return 0;
-}
-
-// The forward from the tokens to the loss and dlogits. With t->split, also the
-// operands of the backward's products as split rows: the weights', LayerNorm's and
-// GELU's outputs in place once the forward's own product has read them, and copies
-// of those that are read again in fp32.
-int forward_pass(cngpt_hip_train* t, const CtxView& v) {
-    const cngpt_hip_config& c = t->cfg;
-    const int B = t->B, T = t->T, C = c.n_embd, V = c.vocab_size, H = c.n_head;
-    const long N = t->N, NC = N * C;
-    hipStream_t s = v.stream;
-    const bool drop = t->dropped;
-    const float dscale = drop ? 1.0f / (1.0f - t->dropout) : 1.0f;
-    const TrainSlots k{c.n_layer};
-    auto split_rows = [&](float* x, float* o, int cols, int slot, bool measure) {
-        SplitTensor d{};
-        d.src = x; d.dst = o; d.n = N * cols; d.alt = cols; d.amax = t->slot + slot;
-        return t->split ? launch_split_tensor(d, measure, s) : hipSuccess;
-    };
-    if (t->split) {
-        TRY(launch_split_slots(t->slot, k.count(), s));
-        TRY(launch_split_ln(v.d_layers, v.lnf_w, v.lnf_b, c.n_layer, C, t->slot, s));
-        TRY(launch_split_weights(t->weights, 4 * c.n_layer, t->colmax, 7l * c.n_layer * C,
-                                 t->err + 1, s));
-    }
-
-    TRY(launch_embed(t->tok, v.wte, v.wpe, t->emb, N, T, C, V, 0, nullptr, t->err, nullptr, 0, s));
-    if (drop) TRY(launch_dropout(t->emb, t->masks, NC, dscale, s));   // model.c:471-472
-    const float* x = t->emb;
-    const size_t xbytes = (size_t)N * C * sizeof(float);
-    for (int l = 0; l < c.n_layer; l++) {
-        const LayerW& w = v.layers[l];
-        TrainLayer& a = t->acts[l];
-        TRY(launch_layernorm(x, C, w.ln1_w, w.ln1_b, a.ln1_out, C, (int)N, C, s, a.ln1_mean,
-                             a.ln1_rstd));
-        if (gemm(t, s, a.ln1_out, w.attn_w, w.attn_b, a.qkv, N, 3 * C, C, EPI_BIAS)) return -1;
-        TRY(split_rows(a.ln1_out, a.ln1_out, C, k.ln(2 * l), false));
-        TRY(launch_attention_causal(a.qkv, T, a.attn_out, B, T, C, H, s, a.lse));
-        TRY(split_rows(a.attn_out, a.attn_sp, C, k.attn(l), true));
-        TRY(hipMemcpyAsync(a.res1, x, xbytes, hipMemcpyDeviceToDevice, s));
-        if (gemm(t, s, a.attn_out, w.proj_w, w.proj_b, a.res1, N, C, C, EPI_RESID)) return -1;
-        if (drop) TRY(launch_dropout(a.res1, t->masks + (1 + 2 * l) * NC, NC, dscale, s));
-        TRY(launch_layernorm(a.res1, C, w.ln2_w, w.ln2_b, a.ln2_out, C, (int)N, C, s, a.ln2_mean,
-                             a.ln2_rstd));
-        if (gemm(t, s, a.ln2_out, w.fc_w, w.fc_b, a.fc_out, N, 4 * C, C, EPI_BIAS)) return -1;
-        TRY(split_rows(a.ln2_out, a.ln2_out, C, k.ln(2 * l + 1), false));
-        TRY(launch_gelu_fwd(a.fc_out, a.gelu, N * 4 * C, s, t->split ? t->slot + k.gelu(l) : nullptr));
-        TRY(hipMemcpyAsync(a.res2, a.res1, xbytes, hipMemcpyDeviceToDevice, s));
-        if (gemm(t, s, a.gelu, w.mlp_w, w.mlp_b, a.res2, N, C, 4 * C, EPI_RESID)) return -1;
-        TRY(split_rows(a.gelu, a.gelu, 4 * C, k.gelu(l), false));
-        if (drop) TRY(launch_dropout(a.res2, t->masks + (2 + 2 * l) * NC, NC, dscale, s));
-        x = a.res2;
-    }
-    TRY(launch_layernorm(x, C, v.lnf_w, v.lnf_b, t->lnf_out, C, (int)N, C, s, t->lnf_mean,
-                         t->lnf_rstd));
-    if (gemm(t, s, t->lnf_out, v.wte, nullptr, t->logits, N, V, C, EPI_STORE)) return -1;
-    // the loss, and the gradient of the mean loss for the backward
-    // (cross_entropy_bwd) into the padded dlogits rows, from one read of the
-    // logits
-    TRY(launch_cross_entropy(t->logits, N, V, t->tgt, t->row_loss, t->loss, 0, t->err, s, t->dlog,
-                             t->Vp));
-    return 0;
-}
-
-// From dlogits to the gradient of the embedding.
-int backward_fp32(cngpt_hip_train* t, const CtxView& v) {
-    const cngpt_hip_config& c = t->cfg;
-    const int B = t->B, T = t->T, C = c.n_embd, V = c.vocab_size, H = c.n_head;
-    const long N = t->N, NC = N * C;
-    hipStream_t s = v.stream;
-    const size_t xbytes = (size_t)NC * sizeof(float);
-    const bool drop = t->dropped;
-    const float dscale = drop ? 1.0f / (1.0f - t->dropout) : 1.0f;
-    // dlogits = (probs - onehot) / (B T) (model.c:660-666) was formed by the
-    // forward's loss pass; the tied lm_head: d ln_f = dlogits . wte,
-    // d wte += dlogits^T . ln_f_out
-    TRY(launch_transpose(v.wte, C, V, C, t->tW, t->Vp, (int)t->Vp, C, s));
-    if (gemm(t, s, t->dlog, t->tW, nullptr, t->d_ln, N, C, t->Vp, EPI_STORE)) return -1;
-    if (linear_dw(t, s, t->dlog, t->Vp, t->lnf_out, grad_of(t, v, v.wte), nullptr, V, C))
-        return -1;
-    // the final LayerNorm (its input gradient into a cleared d_x)
-    TRY(hipMemsetAsync(t->d_x, 0, xbytes, s));
-    const float* x_last = c.n_layer > 0 ? t->acts[c.n_layer - 1].res2 : t->emb;
-    TRY(launch_layernorm_bwd(t->d_ln, x_last, v.lnf_w, t->lnf_mean, t->lnf_rstd, t->d_x,
-                             grad_of(t, v, v.lnf_w), grad_of(t, v, v.lnf_b), (int)N, C, t->red, s));
-
-    for (int l = c.n_layer - 1; l >= 0; l--) {
-        const LayerW& w = v.layers[l];
-        const TrainLayer& a = t->acts[l];
-        const float* x_in = l > 0 ? t->acts[l - 1].res2 : t->emb;
-        // dropout_bwd (ops.c:620-625) of res2 (model.c:699-700)
-        if (drop) TRY(launch_dropout(t->d_x, t->masks + (2 + 2 * l) * NC, NC, dscale, s));
-        TRY(hipMemcpyAsync(t->d_res1, t->d_x, xbytes, hipMemcpyDeviceToDevice, s));
-        // proj: Y = gelu . mlp_w^T + b
-        if (linear_dx(t, s, t->d_x, w.mlp_w, t->d_hid, C, 4 * C) ||
-            linear_dw(t, s, t->d_x, C, a.gelu, grad_of(t, v, w.mlp_w), grad_of(t, v, w.mlp_b), C,
-                      4 * C))
-            return -1;
-        TRY(launch_gelu_bwd(t->d_hid, a.fc_out, N * 4 * C, s));
-        // fc: Y = ln2_out . fc_w^T + b
-        if (linear_dx(t, s, t->d_hid, w.fc_w, t->d_ln, 4 * C, C) ||
-            linear_dw(t, s, t->d_hid, 4 * C, a.ln2_out, grad_of(t, v, w.fc_w), grad_of(t, v, w.fc_b),
-                      4 * C, C))
-            return -1;
-        TRY(launch_layernorm_bwd(t->d_ln, a.res1, w.ln2_w, a.ln2_mean, a.ln2_rstd, t->d_res1,
-                                 grad_of(t, v, w.ln2_w), grad_of(t, v, w.ln2_b), (int)N, C, t->red,
-                                 s));
-        // and of res1 (model.c:732-733)
-        if (drop) TRY(launch_dropout(t->d_res1, t->masks + (1 + 2 * l) * NC, NC, dscale, s));
-        // c_proj: Y = attn_out . proj_w^T + b
-        if (linear_dx(t, s, t->d_res1, w.proj_w, t->d_attn, C, C) ||
-            linear_dw(t, s, t->d_res1, C, a.attn_out, grad_of(t, v, w.proj_w),
-                      grad_of(t, v, w.proj_b), C, C))
-            return -1;
-        TRY(launch_attention_bwd(a.qkv, a.attn_out, t->d_attn, a.lse, t->Dbuf, t->d_qkv, B, T, C, H,
-                                 s));
-        // QKV: Y = ln1_out . attn_w^T + b
-        if (linear_dx(t, s, t->d_qkv, w.attn_w, t->d_ln, 3 * C, C) ||
-            linear_dw(t, s, t->d_qkv, 3 * C, a.ln1_out, grad_of(t, v, w.attn_w), grad_of(t, v, w.attn_b),
-                      3 * C, C))
-            return -1;
-        TRY(hipMemcpyAsync(t->d_x, t->d_res1, xbytes, hipMemcpyDeviceToDevice, s));
-        TRY(launch_layernorm_bwd(t->d_ln, x_in, w.ln1_w, a.ln1_mean, a.ln1_rstd, t->d_x,
-                                 grad_of(t, v, w.ln1_w), grad_of(t, v, w.ln1_b), (int)N, C, t->red,
-                                 s));
-    }
-    return 0;
-}
-
-// The same with split products.
-int backward_split(cngpt_hip_train* t, const CtxView& v) {
-    const cngpt_hip_config& c = t->cfg;
-    const int B = t->B, T = t->T, C = c.n_embd, V = c.vocab_size, H = c.n_head;
-    const long N = t->N, NC = N * C;
-    hipStream_t s = v.stream;
-    const size_t xbytes = (size_t)NC * sizeof(float);
-    const bool drop = t->dropped;
-    const float dscale = drop ? 1.0f / (1.0f - t->dropout) : 1.0f;
-    const int L = c.n_layer;
-    const TrainSlots k{L};
-    auto split_grad = [&](const float* d, float* o, int cols, int slot) {
-        SplitTensor g{};
-        g.src = d; g.dst = o; g.n = N * cols; g.alt = cols; g.amax = t->slot + slot;
-        return launch_split_tensor(g, true, s);
-    };
-    TRY(launch_split_slots(t->slot + k.grad(0, 0), 4 * L, s));
-    // the tied lm_head stays in fp32: its dX, whose sum of V products is the
-    // more accurate (gradient of the last LayerNorm's bias, V = 50257, against
-    // float64: 3.6e-6, split 6.2e-6), and its dW, whose rows are as far apart as the
-    // tokens' probabilities (one scale for all of dlogits holds a token of p = 1e-8
-    // to 9e-5 of its row, of 1e-12 not at all; fp32 to 4e-7)
-    TRY(launch_transpose(v.wte, C, V, C, t->tW, t->Vp, (int)t->Vp, C, s));
-    if (gemm(t, s, t->dlog, t->tW, nullptr, t->d_ln, N, C, t->Vp, EPI_STORE) ||
-        linear_dw(t, s, t->dlog, t->Vp, t->lnf_out, grad_of(t, v, v.wte), nullptr, V, C))
-        return -1;
-    TRY(hipMemsetAsync(t->d_x, 0, xbytes, s));
-    const float* x_last = L > 0 ? t->acts[L - 1].res2 : t->emb;
-    TRY(launch_layernorm_bwd(t->d_ln, x_last, v.lnf_w, t->lnf_mean, t->lnf_rstd, t->d_x,
-                             grad_of(t, v, v.lnf_w), grad_of(t, v, v.lnf_b), (int)N, C, t->red, s));
-    for (int l = L - 1; l >= 0; l--) {
-        const LayerW& w = v.layers[l];
-        const TrainLayer& a = t->acts[l];
-        const float* x_in = l > 0 ? t->acts[l - 1].res2 : t->emb;
-        if (drop) TRY(launch_dropout(t->d_x, t->masks + (2 + 2 * l) * NC, NC, dscale, s));
-        TRY(hipMemcpyAsync(t->d_res1, t->d_x, xbytes, hipMemcpyDeviceToDevice, s));
-        TRY(split_grad(t->d_x, t->sp_x, C, k.grad(l, 0)));
-        if (slinear_bwd(t, s, t->d_x, t->sp_x, k.grad(l, 0), a.gelu, k.gelu(l), k.weight(4 * l + 3),
-                        t->d_hid, grad_of(t, v, w.mlp_w), grad_of(t, v, w.mlp_b), C, 4 * C,
-                        t->slot + k.grad(l, 1)))
-            return -1;
-        TRY(launch_split_gelu_bwd(t->d_hid, a.fc_out, t->sp_hid, N * 4 * C, 4 * C, t->slot + k.grad(l, 1), s));
-        if (slinear_bwd(t, s, t->d_hid, t->sp_hid, k.grad(l, 1), a.ln2_out, k.ln(2 * l + 1),
-                        k.weight(4 * l + 2), t->d_ln, grad_of(t, v, w.fc_w), grad_of(t, v, w.fc_b),
-                        4 * C, C))
-            return -1;
-        TRY(launch_layernorm_bwd(t->d_ln, a.res1, w.ln2_w, a.ln2_mean, a.ln2_rstd, t->d_res1,
-                                 grad_of(t, v, w.ln2_w), grad_of(t, v, w.ln2_b), (int)N, C, t->red,
-                                 s));
-        if (drop) TRY(launch_dropout(t->d_res1, t->masks + (1 + 2 * l) * NC, NC, dscale, s));
-        TRY(split_grad(t->d_res1, t->sp_x, C, k.grad(l, 2)));
-        if (slinear_bwd(t, s, t->d_res1, t->sp_x, k.grad(l, 2), a.attn_sp, k.attn(l), k.weight(4 * l + 1),
-                        t->d_attn, grad_of(t, v, w.proj_w), grad_of(t, v, w.proj_b), C, C))
-            return -1;
-        TRY(launch_attention_bwd(a.qkv, a.attn_out, t->d_attn, a.lse, t->Dbuf, t->d_qkv, B, T, C, H,
-                                 s));
-        TRY(split_grad(t->d_qkv, t->sp_qkv, 3 * C, k.grad(l, 3)));
-        if (slinear_bwd(t, s, t->d_qkv, t->sp_qkv, k.grad(l, 3), a.ln1_out, k.ln(2 * l), k.weight(4 * l),
-                        t->d_ln, grad_of(t, v, w.attn_w), grad_of(t, v, w.attn_b), 3 * C, C))
-            return -1;
-        TRY(hipMemcpyAsync(t->d_x, t->d_res1, xbytes, hipMemcpyDeviceToDevice, s));
-        TRY(launch_layernorm_bwd(t->d_ln, x_in, w.ln1_w, a.ln1_mean, a.ln1_rstd, t->d_x,
-                                 grad_of(t, v, w.ln1_w), grad_of(t, v, w.ln1_b), (int)N, C, t->red,
-                                 s));
-    }
     return 0;
 }
 
@@ -527,14 +329,12 @@ int cngpt_hip_train_create(cngpt_hip_ctx* h, int B, int T, cngpt_hip_train** out
                  ln_bwd_part_floats((int)N, (int)C)}));
     fl(4 * C);                                // zeros
     t->can_split = split_takes(v, N);
-    const TrainSlots slots{(int)L};
     if (t->can_split) {
-        fl(slots.count());                    // slot
-        fl(L * 7 * C);                        // colmax (columns: 3 x C and 4 C a layer)
+        t->n_maxima = L * (4 + 7 * C + 16 * C);
+        fl(t->n_maxima); fl(N);               // maxima, rmax
         fl(L * 12 * C * C);                   // wsp
-        fl(Np * C); fl(Np * 4 * C); fl(Np * 3 * C);       // sp_x, sp_hid, sp_qkv
-        sz.push_back(4 * L * sizeof(SplitTensor) + 1);  // weights
-        for (long l = 0; l < L; l++) fl(Np * C);          // attn_sp
+        fl(Np * 4 * C); fl(N * 4 * C); fl(Np * 4 * C);  // y_col, y_row, x_col
+        sz.push_back(4 * L * sizeof(SplitTensor));      // weights
     }
     sz.push_back((size_t)grad_norm_parts(n) * sizeof(double));
     fl(1); fl(1);                             // norm, coef
@@ -575,29 +375,28 @@ int cngpt_hip_train_create(cngpt_hip_ctx* h, int B, int T, cngpt_hip_train** out
     t->tA = (float*)take(); t->tB = (float*)take(); t->tW = (float*)take();
     t->part = (float*)take(); t->red = (float*)take(); t->zeros = (float*)take();
     if (t->can_split) {
-        t->slot = (unsigned*)take();
-        t->colmax = (unsigned*)take(); t->wsp = (float*)take();
-        t->sp_x = (float*)take(); t->sp_hid = (float*)take(); t->sp_qkv = (float*)take();
+        t->maxima = (unsigned*)take(); t->rmax = (unsigned*)take();
+        t->wsp = (float*)take();
+        t->y_col = (float*)take(); t->y_row = (float*)take(); t->x_col = (float*)take();
         t->weights = (SplitTensor*)take();
-        for (auto& a : t->acts) a.attn_sp = (float*)take();
         float* o = t->wsp;
-        unsigned* col = t->colmax;
+        unsigned* col = t->maxima + 4 * L;
         auto add = [&](const float* W, long rows, long K) {
             SplitTensor d{};
             d.src = W; d.dst = o; d.n = rows * K; d.K = (int)K;
-            d.amax = t->slot + slots.weight((int)t->hweights.size());
+            d.amax = t->maxima + t->hweights.size();
             d.colmax = col;
             t->hweights.push_back(d);
             o += rows * K;
             col += K;
         };
-        for (int l = 0; l < (int)L; l++) {
-            const LayerW& w = v.layers[l];
-            add(w.attn_w, 3 * C, C);
-            add(w.proj_w, C, C);
-            add(w.fc_w, 4 * C, C);
-            add(w.mlp_w, C, 4 * C);
+        for (const LayerW* w = v.layers; w < v.layers + L; w++) {
+            add(w->attn_w, 3 * C, C);
+            add(w->proj_w, C, C);
+            add(w->fc_w, 4 * C, C);
+            add(w->mlp_w, C, 4 * C);
         }
+        t->colmax = col;
     }
     t->nparts = (double*)take();
     t->norm = (float*)take(); t->coef = (float*)take();
@@ -621,16 +420,17 @@ int cngpt_hip_train_create(cngpt_hip_ctx* h, int B, int T, cngpt_hip_train** out
     int rc = 0;
     // everything starts at zero: gradients, moments, the zero bias, the
     // error flags and the padding rows
-    if (hipMemsetAsync(t->arena, 0, total, s) != hipSuccess ||
+    if ((t->can_split && (hipHostMalloc(&t->verdict, sizeof(int)) != hipSuccess ||
+                          hipEventCreateWithFlags(&t->judged, hipEventDisableTiming) != hipSuccess)) ||
+        hipMemsetAsync(t->arena, 0, total, s) != hipSuccess ||
         hipMemcpyAsync(t->decay, mask.data(), (size_t)n, hipMemcpyHostToDevice, s) != hipSuccess ||
-        (!t->hweights.empty() &&
+        (t->can_split &&
          hipMemcpyAsync(t->weights, t->hweights.data(), t->hweights.size() * sizeof(SplitTensor),
                         hipMemcpyHostToDevice, s) != hipSuccess) ||
         hipStreamSynchronize(s) != hipSuccess)
         rc = ctx_fail("trainer set-up failed: %s", hipGetErrorString(hipGetLastError()));
     if (rc) {
-        (void)hipFree(t->arena);
-        delete t;
+        cngpt_hip_train_destroy(t);
         return -1;
     }
     *out = t;
@@ -643,6 +443,8 @@ void cngpt_hip_train_destroy(cngpt_hip_train* t) {
     (void)hipDeviceSynchronize();
     if (t->arena) (void)hipFree(t->arena);
     if (t->masks) (void)hipFree(t->masks);
+    if (t->verdict) (void)hipHostFree(t->verdict);
+    if (t->judged) (void)hipEventDestroy(t->judged);
     delete t;
 }
 
@@ -669,7 +471,7 @@ int cngpt_hip_train_forward(cngpt_hip_train* t, const int* tokens, const int* ta
     CtxView v;
     if (view_of(t, &v)) return -1;
     const cngpt_hip_config& c = t->cfg;
-    const int V = c.vocab_size;
+    const int B = t->B, T = t->T, C = c.n_embd, V = c.vocab_size, H = c.n_head;
     const long N = t->N;
     if (check_ids(tokens, N, V, "token") || check_ids(targets, N, V, "target")) return -1;
     hipStream_t s = v.stream;
@@ -701,6 +503,8 @@ int cngpt_hip_train_forward(cngpt_hip_train* t, const int* tokens, const int* ta
     // and res2 of each layer; then the keep masks go to the device
     const float p = t->dropout;
     const bool drop = p > 0.f;
+    const long NC = N * C;
+    const float dscale = drop ? 1.0f / (1.0f - p) : 1.0f;
     if (drop) {
         unsigned char* hm = t->hmasks.data();
         const size_t n = t->hmasks.size();
@@ -711,25 +515,48 @@ int cngpt_hip_train_forward(cngpt_hip_train* t, const int* tokens, const int* ta
         TRY(hipMemcpyAsync(t->masks, hm, n, hipMemcpyHostToDevice, s));
     }
     t->dropped = drop;
-
     t->have_fwd = false;
-    for (;;) {
-        t->split = t->can_split;
-        if (forward_pass(t, v)) return -1;
-        float lv = 0.f;
-        int e[2] = {0, 0};  // error flags, the verdict on the split weights
-        TRY(hipMemcpyAsync(&lv, t->loss, sizeof(float), hipMemcpyDeviceToHost, s));
-        TRY(hipMemcpyAsync(e, t->err, sizeof(e), hipMemcpyDeviceToHost, s));
-        TRY(hipStreamSynchronize(s));
-        if (e[0]) return ctx_fail("device reported error flags 0x%x in the training forward", e[0]);
-        if (t->split && e[1]) {  // these weights take the fp32 products from now on
-            t->can_split = false;
-            continue;
-        }
-        t->have_fwd = true;
-        if (loss) *loss = lv;
-        return 0;
+
+    TRY(launch_embed(t->tok, v.wte, v.wpe, t->emb, N, T, C, V, 0, nullptr, t->err, nullptr, 0, s));
+    if (drop) TRY(launch_dropout(t->emb, t->masks, NC, dscale, s));   // model.c:471-472
+    const float* x = t->emb;
+    const size_t xbytes = (size_t)N * C * sizeof(float);
+    for (int l = 0; l < c.n_layer; l++) {
+        const LayerW& w = v.layers[l];
+        TrainLayer& a = t->acts[l];
+        TRY(launch_layernorm(x, C, w.ln1_w, w.ln1_b, a.ln1_out, C, (int)N, C, s, a.ln1_mean,
+                             a.ln1_rstd));
+        if (gemm(t, s, a.ln1_out, w.attn_w, w.attn_b, a.qkv, N, 3 * C, C, EPI_BIAS)) return -1;
+        TRY(launch_attention_causal(a.qkv, T, a.attn_out, B, T, C, H, s, a.lse));
+        TRY(hipMemcpyAsync(a.res1, x, xbytes, hipMemcpyDeviceToDevice, s));
+        if (gemm(t, s, a.attn_out, w.proj_w, w.proj_b, a.res1, N, C, C, EPI_RESID)) return -1;
+        if (drop) TRY(launch_dropout(a.res1, t->masks + (1 + 2 * l) * NC, NC, dscale, s));
+        TRY(launch_layernorm(a.res1, C, w.ln2_w, w.ln2_b, a.ln2_out, C, (int)N, C, s, a.ln2_mean,
+                             a.ln2_rstd));
+        if (gemm(t, s, a.ln2_out, w.fc_w, w.fc_b, a.fc_out, N, 4 * C, C, EPI_BIAS)) return -1;
+        TRY(launch_gelu_fwd(a.fc_out, a.gelu, N * 4 * C, s));
+        TRY(hipMemcpyAsync(a.res2, a.res1, xbytes, hipMemcpyDeviceToDevice, s));
+        if (gemm(t, s, a.gelu, w.mlp_w, w.mlp_b, a.res2, N, C, 4 * C, EPI_RESID)) return -1;
+        if (drop) TRY(launch_dropout(a.res2, t->masks + (2 + 2 * l) * NC, NC, dscale, s));
+        x = a.res2;
     }
+    TRY(launch_layernorm(x, C, v.lnf_w, v.lnf_b, t->lnf_out, C, (int)N, C, s, t->lnf_mean,
+                         t->lnf_rstd));
+    if (gemm(t, s, t->lnf_out, v.wte, nullptr, t->logits, N, V, C, EPI_STORE)) return -1;
+    // the loss, and the gradient of the mean loss for the backward
+    // (cross_entropy_bwd) into the padded dlogits rows, from one read of the
+    // logits
+    TRY(launch_cross_entropy(t->logits, N, V, t->tgt, t->row_loss, t->loss, 0, t->err, s, t->dlog,
+                             t->Vp));
+    float lv = 0.f;
+    int e = 0;
+    TRY(hipMemcpyAsync(&lv, t->loss, sizeof(float), hipMemcpyDeviceToHost, s));
+    TRY(hipMemcpyAsync(&e, t->err, sizeof(int), hipMemcpyDeviceToHost, s));
+    TRY(hipStreamSynchronize(s));
+    if (e) return ctx_fail("device reported error flags 0x%x in the training forward", e);
+    t->have_fwd = true;
+    if (loss) *loss = lv;
+    return 0;
 }
 
 int cngpt_hip_train_backward(cngpt_hip_train* t) {
@@ -737,13 +564,75 @@ int cngpt_hip_train_backward(cngpt_hip_train* t) {
     if (view_of(t, &v)) return -1;
     if (!t->have_fwd) return ctx_fail("no training forward to differentiate");
     const cngpt_hip_config& c = t->cfg;
-    const int B = t->B, T = t->T, C = c.n_embd;
-    const long NC = t->N * C;
+    const int B = t->B, T = t->T, C = c.n_embd, V = c.vocab_size, H = c.n_head;
+    const long N = t->N;
     hipStream_t s = v.stream;
+    const size_t xbytes = (size_t)N * C * sizeof(float);
+    const long NC = N * C;
     const bool drop = t->dropped;
     const float dscale = drop ? 1.0f / (1.0f - t->dropout) : 1.0f;
 
-    if (t->split ? backward_split(t, v) : backward_fp32(t, v)) return -1;
+    if (t->can_split && split_weights(t, s)) return -1;
+    // dlogits = (probs - onehot) / (B T) (model.c:660-666) was formed by the
+    // forward's loss pass; the tied lm_head: d ln_f = dlogits . wte,
+    // d wte += dlogits^T . ln_f_out. Both stay in fp32: the dX, whose sum of V products
+    // is the more accurate (gradient of the last LayerNorm's bias, V = 50257, against
+    // float64: 3.6e-6, split 6.2e-6), and the dW (one scale for all of dlogits held the
+    // row of a token of p = 1e-8 to 9e-5, of 1e-12 not at all; one per column takes
+    // another copy of dlogits).
+    TRY(launch_transpose(v.wte, C, V, C, t->tW, t->Vp, (int)t->Vp, C, s));
+    if (gemm(t, s, t->dlog, t->tW, nullptr, t->d_ln, N, C, t->Vp, EPI_STORE)) return -1;
+    if (linear_dw(t, s, t->dlog, t->Vp, t->lnf_out, grad_of(t, v, v.wte), nullptr, V, C))
+        return -1;
+    // the final LayerNorm (its input gradient into a cleared d_x)
+    TRY(hipMemsetAsync(t->d_x, 0, xbytes, s));
+    const float* x_last = c.n_layer > 0 ? t->acts[c.n_layer - 1].res2 : t->emb;
+    TRY(launch_layernorm_bwd(t->d_ln, x_last, v.lnf_w, t->lnf_mean, t->lnf_rstd, t->d_x,
+                             grad_of(t, v, v.lnf_w), grad_of(t, v, v.lnf_b), (int)N, C, t->red, s));
+
+    // weights that do not fit take the fp32 products from now on (the device works on
+    // the lm_head meanwhile)
+    if (t->can_split) {
+        TRY(hipEventSynchronize(t->judged));
+        t->can_split = *t->verdict == 0;
+    }
+    unsigned* col = t->colmax;
+    // layer l's i-th matrix (attn, proj, fc, mlp), Y = X . W^T + b: dX, dW and db
+    auto linear_bwd = [&](int l, int i, const float* dY, const float* X, const float* W,
+                          const float* b, float* dX, long out, long in) {
+        float *dW = grad_of(t, v, W), *db = grad_of(t, v, b);
+        if (t->can_split)
+            return slinear_bwd(t, s, dY, X, t->hweights[4 * l + i], dX, dW, db, out, in, col);
+        return linear_dx(t, s, dY, W, dX, out, in) || linear_dw(t, s, dY, out, X, dW, db, out, in) ? -1 : 0;
+    };
+    for (int l = c.n_layer - 1; l >= 0; l--) {
+        const LayerW& w = v.layers[l];
+        const TrainLayer& a = t->acts[l];
+        const float* x_in = l > 0 ? t->acts[l - 1].res2 : t->emb;
+        // dropout_bwd (ops.c:620-625) of res2 (model.c:699-700)
+        if (drop) TRY(launch_dropout(t->d_x, t->masks + (2 + 2 * l) * NC, NC, dscale, s));
+        TRY(hipMemcpyAsync(t->d_res1, t->d_x, xbytes, hipMemcpyDeviceToDevice, s));
+        // proj: Y = gelu . mlp_w^T + b
+        if (linear_bwd(l, 3, t->d_x, a.gelu, w.mlp_w, w.mlp_b, t->d_hid, C, 4 * C)) return -1;
+        TRY(launch_gelu_bwd(t->d_hid, a.fc_out, N * 4 * C, s));
+        // fc: Y = ln2_out . fc_w^T + b
+        if (linear_bwd(l, 2, t->d_hid, a.ln2_out, w.fc_w, w.fc_b, t->d_ln, 4 * C, C)) return -1;
+        TRY(launch_layernorm_bwd(t->d_ln, a.res1, w.ln2_w, a.ln2_mean, a.ln2_rstd, t->d_res1,
+                                 grad_of(t, v, w.ln2_w), grad_of(t, v, w.ln2_b), (int)N, C, t->red,
+                                 s));
+        // and of res1 (model.c:732-733)
+        if (drop) TRY(launch_dropout(t->d_res1, t->masks + (1 + 2 * l) * NC, NC, dscale, s));
+        // c_proj: Y = attn_out . proj_w^T + b
+        if (linear_bwd(l, 1, t->d_res1, a.attn_out, w.proj_w, w.proj_b, t->d_attn, C, C)) return -1;
+        TRY(launch_attention_bwd(a.qkv, a.attn_out, t->d_attn, a.lse, t->Dbuf, t->d_qkv, B, T, C, H,
+                                 s));
+        // QKV: Y = ln1_out . attn_w^T + b
+        if (linear_bwd(l, 0, t->d_qkv, a.ln1_out, w.attn_w, w.attn_b, t->d_ln, 3 * C, C)) return -1;
+        TRY(hipMemcpyAsync(t->d_x, t->d_res1, xbytes, hipMemcpyDeviceToDevice, s));
+        TRY(launch_layernorm_bwd(t->d_ln, x_in, w.ln1_w, a.ln1_mean, a.ln1_rstd, t->d_x,
+                                 grad_of(t, v, w.ln1_w), grad_of(t, v, w.ln1_b), (int)N, C, t->red,
+                                 s));
+    }
     // and of the embedding (model.c:849-850)
     if (drop) TRY(launch_dropout(t->d_x, t->masks, NC, dscale, s));
     TRY(launch_embed_bwd(t->d_x, B, T, C, grad_of(t, v, v.wpe), grad_of(t, v, v.wte), t->uniq,

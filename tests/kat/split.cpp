@@ -174,6 +174,51 @@ long kat_split_train(const float* X, const float* W, float* Y, float* Y32, int M
     return top;
 }
 
+// The same products with the scales of the training step: km 2, a scale per row of X
+// [M][K] and one for W [K][ldw]; km 3, one per column of X [K][ldx] and of W. X holds
+// K - pad rows (M - pad with km 2), which launch_split_rows pads with zero rows.
+int kat_split_train_rows(const float* X, const float* W, float* Y, int M, int N, int K, int ldx, int ldw,
+                         int km, int pad) {
+    Dev d;
+    const int xrows = km == 3 ? K : M, xcols = km == 3 ? ldx : K;
+    std::vector<float> zero(N, 0.f);
+    float *dx = d.put(X, (size_t)(xrows - pad) * xcols), *dw = d.put(W, (size_t)K * ldw);
+    float *dy = d.put(Y, (size_t)M * N), *db = d.put(zero.data(), N);
+    std::vector<unsigned> ff((size_t)xrows * xcols, 0xffffffffu);  // (padding must be written)
+    float* xcol = (float*)d.put(ff.data(), ff.size());
+    float *xrow = d.put<float>(nullptr, (size_t)xrows * xcols), *wcol = d.put<float>(nullptr, (size_t)K * ldw);
+    float* part = d.put<float>(nullptr, 1 << 24);
+    unsigned *xmax = d.put<unsigned>(nullptr, xcols), *wmax = d.put<unsigned>(nullptr, ldw);
+    unsigned* rmax = d.put<unsigned>(nullptr, xrows);
+    if (!d.ok) return -1;
+    if (launch_cols_max(dx, xrows - pad, xcols, xmax, nullptr) != hipSuccess ||
+        launch_split_rows({dx, xrows - pad, xrows, xcols, xmax, xcol, km == 2 ? xrow : nullptr,
+                           km == 2 ? rmax : nullptr}, nullptr) != hipSuccess)
+        return -1;
+    SplitGemmArgs a{};
+    a.Y = dy; a.bias = db;
+    a.M = M; a.N = N; a.K = K;
+    a.ldy = N; a.ldx = ldx; a.ldw = ldw; a.km = km;
+    a.X = km == 3 ? xcol : xrow; a.W = wcol;
+    a.xmax = km == 3 ? xmax : rmax; a.wmax = wmax;
+    a.xstep = 1; a.wstep = km == 3;
+    a.epi = km == 3 ? EPI_RESID : EPI_STORE;
+    a.part = part; a.part_cap = 1 << 24;
+    if (km == 3) {
+        if (launch_cols_max(dw, K - pad, ldw, wmax, nullptr) != hipSuccess ||
+            launch_split_rows({dw, K - pad, K, ldw, wmax, wcol, nullptr, nullptr}, nullptr) != hipSuccess)
+            return -1;
+    } else {
+        SplitTensor t{};
+        t.src = dw; t.dst = wcol; t.n = (long)K * ldw; t.amax = wmax;
+        if (launch_split_tensor(t, true, nullptr) != hipSuccess) return -1;
+    }
+    if (launch_split_train(a, nullptr) != hipSuccess || hipDeviceSynchronize() != hipSuccess ||
+        hipMemcpy(Y, dy, (size_t)M * N * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess)
+        return -1;
+    return 0;
+}
+
 // Causal attention over qkv [B, T, 3C] through the split kernel: out [B, T, C].
 // smax: the largest magnitude of q, k and v the scales allow for.
 int kat_attention_split(const float* qkv, float* out, int B, int T, int C, int H, const float* smax) {

@@ -2,12 +2,14 @@
 tensor's norm does not show, and AdamW divides by. Steps of the size that takes the
 fp16 matrix cores, against float64 autograd and against the fp32 step
 (CNGPT_HIP_SPLIT=0) of the same weights."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import cngpt_amd
-from test_kat_gpu import U
+from test_kat_gpu import LIB, U, fp
 from test_parity_gpu import randomize, say
 from test_train_gpu import tensors
 
@@ -57,6 +59,44 @@ def step(cfg, params, tok, tgt):
         return loss, tr.grads
 
 
+# one step, tiles' edges, padding rows, K split, the tile shapes
+@pytest.mark.parametrize("M,N,K,pad", [(65, 16, 32, 1), (130, 72, 64, 30), (768, 776, 1216, 25),
+                                       (1000, 264, 992, 0), (4096, 3072, 768, 0), (4099, 768, 3072, 3)])
+@pytest.mark.parametrize("km", [2, 3])
+def test_product_of_far_apart_rows_and_columns(M, N, K, pad, km):
+    """Each element within the bound of a product (test_split_gpu) of its own row's and
+    column's sizes, 2^60 apart, where values too small for a full lo are off by
+    2^-40 of the largest that shares their scale."""
+    lib = ctypes.CDLL(LIB)
+    lib.kat_split_train_rows.argtypes = [ctypes.POINTER(ctypes.c_float)] * 3 + [ctypes.c_int] * 7
+    rng = np.random.default_rng(M + N + K + km)
+    ldx, ldw = (M + 7) // 8 * 8, N + 8
+    X = rng.standard_normal((K, ldx) if km == 3 else (M, K), dtype=np.float32)
+    W = rng.standard_normal((K, ldw), dtype=np.float32)
+    if km == 3:
+        X *= np.exp2(rng.integers(-30, 30, ldx)).astype(np.float32)
+        W *= np.exp2(rng.integers(-30, 30, ldw)).astype(np.float32)
+        X[:, 3], W[:, 5] = 0, 0
+        X[K - pad:], W[K - pad:] = 0, 0
+    else:
+        X *= np.exp2(rng.integers(-30, 30, (M, 1))).astype(np.float32)
+        X[3] = 0
+        X[M - pad:] = 0
+    Y = np.zeros((M, N), np.float32)
+    assert lib.kat_split_train_rows(fp(X), fp(W), fp(Y), M, N, K, ldx, ldw, km, pad) == 0
+    x = (X[:, :M].T if km == 3 else X)[: M - (pad if km == 2 else 0)].astype(np.float64)
+    Y = Y[: x.shape[0]]
+    w = W[:, :N].astype(np.float64)
+    ref, mag = x @ w, np.abs(x) @ np.abs(w)
+    wtop = np.abs(w).max(0) if km == 3 else np.abs(w).max()
+    bound = (3 * K + 16) * U * mag + 2.0 ** -38 * K * np.abs(x).max(1, keepdims=True) * wtop
+    err = np.abs(Y - ref)
+    assert (err <= bound).all()
+    ok = mag > 0
+    say(f"  {M} x {N} x {K} km {km}: at most {(err[ok] / mag[ok]).max():.1e} of the sum of magnitudes")
+    assert (err[ok] <= 2.0 ** -20 * mag[ok]).all()  # (a wrong half of a value: 2^-11)
+
+
 def test_improbable_tokens():
     """Tokens of probability 1e-2 down to 1e-18 in every row that appear nowhere in
     the batch: their embeddings' gradients are (p / N) . x summed over the rows, at
@@ -81,3 +121,65 @@ def test_improbable_tokens():
     xn = np.sqrt(CFG.n_embd) * np.abs(w["ln_f_w"]).max() + np.linalg.norm(w["ln_f_b"])
     bound = 2 * (CFG.n_embd + 8) * U * xn * np.linalg.norm(w["wte"], axis=1).max()
     assert (err <= bound).all(), (err.max(), bound)
+
+
+def test_far_apart_rows_and_columns(monkeypatch):
+    """Activations and gradients whose columns and rows are far apart under ordinary
+    weights: LayerNorm gains 2^-28 of the others, hidden units that never open, a
+    head of small queries and keys, rows whose token is certain. Every row and
+    column of every matrix's gradient is that of the fp32 step (whose forward is the
+    same to the bit) within what the two sums of up to Np rows may be off,
+    (Np + 16) u each, compounded over the layers' own few."""
+    params = randomize(CFG, cngpt_amd.init_weights(CFG, 61), 62)
+    w = named(CFG, params)
+    C = CFG.n_embd
+    rng = np.random.default_rng(63)
+    for n in ("h0.ln1", "h1.ln2"):
+        w[n + "_w"][::2] *= 2.0 ** -28
+        w[n + "_b"][::2] *= 2.0 ** -28
+    w["h0.fc_b"][:64] = -7
+    w["h1.fc_b"][64:128] = -5
+    w["h1.mlp_w"][:, 64:128] *= 2.0 ** -11
+    for third in (0, C):
+        w["h1.attn_w"][third + 192:third + 256] *= 2.0 ** -9
+        w["h1.attn_b"][third + 192:third + 256] *= 2.0 ** -9
+    tok, tgt = (rng.integers(0, 300, (B, T), dtype=np.int32) for _ in range(2))
+    sure = rng.standard_normal(C)
+    sure /= np.linalg.norm(sure)
+    w["wpe"][T - 1] = 40 * sure
+    w["wte"][300] = 0.85 * sure
+    tgt[:, -1] = 300
+    got = []
+    for split in ("1", "0"):
+        monkeypatch.setenv("CNGPT_HIP_SPLIT", split)
+        got.append(step(CFG, params, tok, tgt))
+    assert got[0][0] == got[1][0]
+    assert not np.array_equal(got[0][1], got[1][1])  # (the step took the split products)
+    tol = 4 * (1216 + 16) * U
+    a, b = (named(CFG, g[1]) for g in got)
+    worst = {}
+    for n in a:
+        if a[n].ndim < 2:
+            continue
+        x, y = a[n].astype(np.float64), b[n].astype(np.float64)
+        for axis in (0, 1):
+            size = np.linalg.norm(y, axis=axis)
+            err = np.linalg.norm(x - y, axis=axis)[size > 0] / size[size > 0]
+            worst[n, "columns" if axis == 0 else "rows"] = err.max()
+            say(f"  {n} {'columns' if axis == 0 else 'rows'}: of size {size[size > 0].min():.1e} .. {size.max():.1e}, "
+                f"off by {np.median(err):.1e}, at most {err.max():.1e}")
+    assert max(worst.values()) <= tol, (worst, tol)
+
+
+def test_weights_with_small_rows_keep_fp32(monkeypatch):
+    """Rows of a weight matrix 2^-20 of the others, whose outputs' gradients could be
+    that much larger under the same scale: the step is the fp32 one, to the bit."""
+    params = randomize(CFG, cngpt_amd.init_weights(CFG, 71), 72)
+    named(CFG, params)["h1.fc_w"][100:110] *= 2.0 ** -20
+    rng = np.random.default_rng(73)
+    tok, tgt = (rng.integers(0, 301, (B, T), dtype=np.int32) for _ in range(2))
+    got = []
+    for split in ("1", "0"):
+        monkeypatch.setenv("CNGPT_HIP_SPLIT", split)
+        got.append(step(CFG, params, tok, tgt))
+    assert got[0][0] == got[1][0] and np.array_equal(got[0][1], got[1][1])
