@@ -160,10 +160,12 @@ struct cngpt_hip_ctx {
     std::unordered_map<const float*, const float*> packed_of;
     // Split copies (split.h) of the same matrices and the input scales of
     // their products (launch_split_scales), in the same allocation, for the
-    // forwards over more than SPLIT_MIN_ROWS rows. Made with the packed copies
-    // and stale when they are; split_state is 1 where the split products are
-    // as accurate as fp32 ones, -1 where they are not, 0 while the device's
-    // verdict has not been read. CNGPT_HIP_SPLIT=0 at create time: none.
+    // forwards over more than SPLIT_MIN_ROWS rows. split_state is 1 where the split
+    // products are as accurate as fp32 ones, -1 where they are not, 0 while the
+    // copies are stale (fresh_weights makes them for the forwards that need
+    // them). split_ok is off while a forward is captured for a caller, whose
+    // replays would read copies that an AdamW update leaves behind.
+    // CNGPT_HIP_SPLIT=0 at create time: none.
     struct SplitMat {
         const float* W;
         SplitWeights o;
@@ -172,7 +174,7 @@ struct cngpt_hip_ctx {
         const float* typ;  // typical sizes of its inputs (launch_split_w)
         const float* typ_b;
     };
-    bool use_split = true;
+    bool use_split = true, split_ok = true;
     int split_state = 0;
     std::vector<SplitMat> splits;
     std::unordered_map<const float*, SplitWeights> split_of;
@@ -228,7 +230,8 @@ struct cngpt_hip_ctx {
     // cngpt_hip_forward_resident replay it; captured on the first call of a
     // shape, again after the arena or the parameters moved)
     hipGraphExec_t fwd_exec = nullptr;
-    int fwd_B = 0, fwd_T = 0, fwd_mode = -1, fwd_split = 0;
+    int fwd_B = 0, fwd_T = 0, fwd_mode = -1;
+    bool fwd_split = false;
     const void *fwd_act = nullptr, *fwd_par = nullptr;
 
     // state of the last forward / decode
@@ -299,6 +302,11 @@ int run_ln(cngpt_hip_ctx* h, const float* x, long in_stride, const float* w, con
 // Rows above which a forward's layer products take the split operands
 // (split.hip); up to them the few-row products stream the weights.
 constexpr int SPLIT_MIN_ROWS = 128;
+
+// Whether a forward over `rows` rows takes them.
+bool split_forward(const cngpt_hip_ctx* h, long rows) {
+    return h->split_state == 1 && h->split_ok && rows > SPLIT_MIN_ROWS;
+}
 
 // Y = epi(X . W^T) over split rows X. out_scale: the GELU and QKV epilogues'
 // output scales, Ys: the latter's split rows. With lnout, also LayerNorm(Y rows) as split rows times *lnscale.
@@ -694,7 +702,7 @@ int enqueue_forward(cngpt_hip_ctx* h, int B, int T, int mode, bool kv, bool want
     const long seq_stride = kv ? h->capKV : T;
     // with sp, ln, aout and hid hold split rows (the same bytes), each scaled
     // by its slot's power of two
-    const bool sp = h->split_state == 1 && rows > SPLIT_MIN_ROWS;
+    const bool sp = split_forward(h, rows);
     auto scale = [&](int l, int slot) {
         return sp ? h->sp_scale + SPLIT_SLOTS * l + slot : nullptr;
     };
@@ -816,8 +824,9 @@ int enqueue_forward(cngpt_hip_ctx* h, int B, int T, int mode, bool kv, bool want
 // outlasts the kernels, one graph launch does not.
 int run_forward(cngpt_hip_ctx* h, int B, int T, int mode) {
     if (h->prof || !h->use_graph) return enqueue_forward(h, B, T, mode, false, false);
+    const bool split = split_forward(h, (long)B * T);
     if (!h->fwd_exec || h->fwd_B != B || h->fwd_T != T || h->fwd_mode != mode ||
-        h->fwd_split != h->split_state ||
+        h->fwd_split != split ||
         h->fwd_act != h->d_act || h->fwd_par != h->d_params) {
         drop_fwd_graph(h);
         hipGraph_t g = nullptr;
@@ -835,7 +844,7 @@ int run_forward(cngpt_hip_ctx* h, int B, int T, int mode) {
         if (ei != hipSuccess) return fail("forward graph instantiate: %s", hipGetErrorString(ei));
         h->fwd_exec = ex;
         h->fwd_B = B; h->fwd_T = T; h->fwd_mode = mode;
-        h->fwd_split = h->split_state;
+        h->fwd_split = split;
         h->fwd_act = h->d_act;
         h->fwd_par = h->d_params;
     }
@@ -1110,34 +1119,35 @@ size_t split_bytes(const cngpt_hip_config* cfg) {
            2 * align_up(4 * (size_t)split_slots(L)) + align_up(4 * 7 * C * L) + align_up(sizeof(int));
 }
 
-// Makes the packed and split copies of the weight matrices (again, after an
-// AdamW update marked them stale: ctx_params_written) in kernels on the
-// handle's stream, ordered before what follows. resolve: also read the
-// verdict on the split products, if it is not known (this synchronises).
-int fresh_packed(cngpt_hip_ctx* h, bool resolve = true) {
+// Makes the packed copies of the weight matrices, and for a forward over `rows` rows
+// that takes them the split ones (each again, after an AdamW update marked them
+// stale: ctx_params_written), in kernels on the handle's stream, ordered before
+// what follows; then reads the verdict on the split copies (this synchronises). Under
+// `capture` the packing becomes part of the graph and runs with its replays only.
+int fresh_weights(cngpt_hip_ctx* h, long rows, bool capture = false) {
+    HIP_TRY(hipSetDevice(h->device));
     if (!h->packed_fresh) {
-        HIP_TRY(hipSetDevice(h->device));
         for (const cngpt_hip_ctx::Packed& p : h->packs)
             HIP_TRY(launch_pack_w(p.W, p.Wp, p.N, p.K, h->stream));
-        if (!h->splits.empty()) {
-            const int L = h->cfg.n_layer;
-            HIP_TRY(launch_split_scales(h->d_layers, h->layers.data(), h->lnf_w, h->lnf_b, L,
-                                        h->cfg.n_embd, h->cfg.n_head, h->sp_bound, h->sp_scale,
-                                        h->sp_typ, h->sp_bad, h->stream));
-            for (const cngpt_hip_ctx::SplitMat& m : h->splits)
-                HIP_TRY(launch_split_w(m.W, m.o, m.N, m.K, m.typ, m.typ_b, h->sp_bound + m.in,
-                                       h->sp_scale + m.in, h->sp_bad, h->stream));
-            h->split_state = 0;
-        }
-        h->packed_fresh = true;
+        h->packed_fresh = !capture;
     }
-    if (resolve && !h->splits.empty() && h->split_state == 0) {
-        int bad = 0;
-        HIP_TRY(hipSetDevice(h->device));
-        HIP_TRY(hipMemcpyAsync(&bad, h->sp_bad, sizeof(int), hipMemcpyDeviceToHost, h->stream));
-        HIP_TRY(hipStreamSynchronize(h->stream));
-        h->split_state = bad ? -1 : 1;
-    }
+    if (h->splits.empty() || h->split_state != 0 || rows <= SPLIT_MIN_ROWS || capture) return 0;
+    HIP_TRY(launch_split_scales(h->d_layers, h->layers.data(), h->lnf_w, h->lnf_b, h->cfg.n_layer,
+                                h->cfg.n_embd, h->cfg.n_head, h->sp_bound, h->sp_scale, h->sp_typ,
+                                h->sp_bad, h->stream));
+    for (const cngpt_hip_ctx::SplitMat& m : h->splits)
+        HIP_TRY(launch_split_w(m.W, m.o, m.N, m.K, m.typ, m.typ_b, h->sp_bound + m.in,
+                               h->sp_scale + m.in, h->sp_bad, h->stream));
+    // (a thread that captures another stream may wait for this one in relaxed
+    // mode only)
+    int bad = 0;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+    hipError_t e = hipMemcpyAsync(&bad, h->sp_bad, sizeof(int), hipMemcpyDeviceToHost, h->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+    HIP_TRY(e);
+    h->split_state = bad ? -1 : 1;
     return 0;
 }
 
@@ -1255,7 +1265,7 @@ int params_commit(cngpt_hip_ctx* h, const cngpt_hip_config* cfg) {
             add(w.mlp_w, c, 4 * c, in + SLOT_HID, t + 3 * C, nullptr);
         }
     }
-    if (fresh_packed(h)) return -1;
+    if (fresh_weights(h, SPLIT_MIN_ROWS + 1)) return -1;
     h->have_params = true;
     return 0;
 }
@@ -1486,7 +1496,9 @@ int ctx_view(cngpt_hip_ctx* h, CtxView* v) {
 }
 
 void ctx_params_written(cngpt_hip_ctx* h) {
-    if (h) h->packed_fresh = false;
+    if (!h) return;
+    h->packed_fresh = false;
+    h->split_state = 0;
 }
 
 int ctx_fail(const char* fmt, ...) {
@@ -1628,7 +1640,7 @@ int cngpt_hip_upload_tokens(cngpt_hip_ctx* h, const int* tokens, int B, int T) {
 }
 
 int cngpt_hip_forward_resident(cngpt_hip_ctx* h, int B, int T, int mode) {
-    if (need_params(h) || fresh_packed(h)) return -1;
+    if (need_params(h) || fresh_weights(h, (long)B * T)) return -1;
     if (mode != CNGPT_LAST && mode != CNGPT_ALL) return fail("bad mode %d", mode);
     if (B > h->capB || T > h->capT || (mode == CNGPT_ALL && !h->capAll))
         return fail("forward_resident: arena not reserved for B=%d T=%d mode=%d", B, T, mode);
@@ -1639,9 +1651,11 @@ int cngpt_hip_forward_resident(cngpt_hip_ctx* h, int B, int T, int mode) {
 
 int cngpt_hip_forward_noalloc(cngpt_hip_ctx* h, const int* tokens, int B, int T, int mode,
                               float* logits, int* err) {
-    // (without a synchronisation: until another entry point has read the
-    // verdict on copies made here, the fp32 products run)
-    if (need_params(h) || fresh_packed(h, false)) return -1;
+    if (need_params(h)) return -1;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(h->stream, &cap));
+    const bool capture = cap != hipStreamCaptureStatusNone;
+    if (fresh_weights(h, (long)B * T, capture)) return -1;
     if (mode != CNGPT_LAST && mode != CNGPT_ALL) return fail("bad mode %d", mode);
     if (!tokens || !logits) return fail("forward_noalloc: null device pointer");
     if (B <= 0 || T <= 0) return fail("B=%d T=%d must be positive", B, T);
@@ -1664,14 +1678,16 @@ int cngpt_hip_forward_noalloc(cngpt_hip_ctx* h, const int* tokens, int B, int T,
     HIP_TRY(hipGetLastError());
     const FwdBufs saved = fwd_bufs(h);
     set_fwd_bufs(h, f);
+    h->split_ok = !capture;
     const int rc = enqueue_forward(h, B, T, mode, false, false);
+    h->split_ok = true;
     set_fwd_bufs(h, saved);
     return rc;
 }
 
 int cngpt_hip_forward(cngpt_hip_ctx* h, const int* tokens, int B, int T, int mode,
                       float* logits_out) {
-    if (need_params(h) || fresh_packed(h)) return -1;
+    if (need_params(h) || fresh_weights(h, (long)B * T)) return -1;
     if (mode != CNGPT_LAST && mode != CNGPT_ALL) return fail("bad mode %d", mode);
     if (!tokens) return fail("null tokens");
     if (B <= 0 || T <= 0) return fail("B=%d T=%d must be positive", B, T);
@@ -1771,7 +1787,7 @@ int cngpt_hip_cross_entropy(cngpt_hip_ctx* h, const int* targets, int B, int T, 
 
 int cngpt_hip_decode_begin(cngpt_hip_ctx* h, const int* prompt, int B, int T, int capacity,
                            float* logits_out) {
-    if (need_params(h) || fresh_packed(h)) return -1;
+    if (need_params(h) || fresh_weights(h, (long)B * T)) return -1;
     if (!prompt) return fail("null prompt");
     if (B <= 0 || T <= 0) return fail("B=%d T=%d must be positive", B, T);
     if (capacity <= T || capacity > h->cfg.block_size)
@@ -1800,7 +1816,7 @@ int cngpt_hip_decode_begin(cngpt_hip_ctx* h, const int* prompt, int B, int T, in
 }
 
 int cngpt_hip_decode_step(cngpt_hip_ctx* h, const int* tokens, float* logits_out) {
-    if (need_params(h) || fresh_packed(h)) return -1;
+    if (need_params(h) || fresh_weights(h, 0)) return -1;
     if (h->kvB == 0) return fail("decode_step before decode_begin");
     if (h->kvLen >= h->capKV)
         return fail("KV cache full (%d positions)", h->capKV);
@@ -1831,7 +1847,7 @@ int cngpt_hip_decode_step(cngpt_hip_ctx* h, const int* tokens, float* logits_out
 
 int cngpt_hip_generate(cngpt_hip_ctx* h, int n_new, float temperature, int top_k,
                        const float* draws, int* out_tokens) {
-    if (need_params(h) || fresh_packed(h)) return -1;
+    if (need_params(h) || fresh_weights(h, 0)) return -1;
     if (h->kvB == 0) return fail("generate before decode_begin");
     if (!out_tokens) return fail("null output");
     if (n_new <= 0) return fail("n_new=%d must be positive", n_new);

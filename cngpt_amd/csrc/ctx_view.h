@@ -1,6 +1,6 @@
 // ctx_view.h - what the training step (train_host.cpp) reads of a handle of
 // cngpt_hip.cpp: its device, stream, shape and parameter views. Internal to
-// the library (hidden symbols).
+// the library (hidden symbols, but for ctx_view).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -18,8 +18,9 @@ struct CtxView {
     bool use_split;          // products on the fp16 matrix cores allowed
 };
 
-// Fills v from h; -1 (message set) when h is null or holds no parameters.
-__attribute__((visibility("hidden"))) int ctx_view(cngpt_hip_ctx* h, CtxView* v);
+// Fills v from h; -1 (message set) when h is null or holds no parameters. Exported for the
+// test library, which captures on the handle's stream.
+int ctx_view(cngpt_hip_ctx* h, CtxView* v);
 // Marks the packed weight copies stale after the parameters were updated
 // in place (the next forward or decode entry point packs them again).
 __attribute__((visibility("hidden"))) void ctx_params_written(cngpt_hip_ctx* h);

@@ -127,7 +127,12 @@ int  cngpt_hip_synchronize(cngpt_hip_ctx *h);
  * use until the process ends (a 1024-token window of GPT-2 small or medium
  * fits; larger B * T * n_embd is refused with an error). Needs parameters
  * (cngpt_hip_load_params or _load_file) but no cngpt_hip_reserve. Enqueues
- * on the handle's stream and returns without waiting. Token ids outside
+ * on the handle's stream and returns without waiting (as forward_resident
+ * does; only the first forward of more than 128 rows after an optimizer step
+ * waits, for the verdict on the updated weights' split copies). Captured
+ * into a graph of the handle's stream, forwards of more than 128 rows read
+ * the parameters themselves through the fp32 products, so that replays
+ * follow later updates. Token ids outside
  * [0, vocab_size) are clamped and set *err (device int, may be NULL), which
  * the call zeroes first. All calls on one device share its scratch and it
  * keeps the last call's contents: calls that overlap on one device (other

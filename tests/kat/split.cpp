@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../cngpt_amd/csrc/common.h"
+#include "../../cngpt_amd/csrc/ctx_view.h"
 #include "../../cngpt_amd/csrc/kernels.h"
 
 namespace {
@@ -249,5 +250,30 @@ int kat_attention_split(const float* qkv, float* out, int B, int T, int C, int H
     }
     return 0;
 }
+
+// cngpt_hip_forward_noalloc captured on the handle's stream (device pointers as there):
+// the graph, null on failure.
+hipGraphExec_t kat_capture_noalloc(cngpt_hip_ctx* h, const int* tokens, int B, int T, int mode, float* logits) {
+    CtxView v;
+    if (ctx_view(h, &v) || hipStreamBeginCapture(v.stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
+        return nullptr;
+    const int rc = cngpt_hip_forward_noalloc(h, tokens, B, T, mode, logits, nullptr);
+    hipGraph_t g = nullptr;
+    hipGraphExec_t ex = nullptr;
+    if (hipStreamEndCapture(v.stream, &g) != hipSuccess || rc) return nullptr;
+    if (hipGraphInstantiate(&ex, g, nullptr, nullptr, 0) != hipSuccess) ex = nullptr;
+    (void)hipGraphDestroy(g);
+    return ex;
+}
+
+int kat_replay(cngpt_hip_ctx* h, hipGraphExec_t ex) {
+    CtxView v;
+    return ctx_view(h, &v) || hipGraphLaunch(ex, v.stream) != hipSuccess ||
+                   hipStreamSynchronize(v.stream) != hipSuccess
+               ? -1
+               : 0;
+}
+
+void kat_drop(hipGraphExec_t ex) { (void)hipGraphExecDestroy(ex); }
 
 }  // extern "C"
