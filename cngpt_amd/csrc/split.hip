@@ -137,12 +137,16 @@ __global__ void __launch_bounds__(64) k_split_scores(const float* __restrict__ t
     if (lane == 0 && !(err <= 0x1p-24f * fmaxf(0.25f, tq * tk))) atomicOr(bad, 1);
 }
 
-// scale = the power of two that takes the bound into [2^14, 2^15)
-__global__ void k_split_scales(const float* bound, float* scale, int n) {
+// scale = the power of two that takes the bound into [2^14, 2^15), 1 where the
+// values are all zero. Bounds within 2^40 of 1 keep the products of two scales (a weight
+// row's is within 2^65 of 1), and what undoes them, normal floats.
+__global__ void k_split_scales(const float* bound, float* scale, int n, int* bad) {
     const int i = blockIdx.x * 64 + threadIdx.x;
     if (i >= n) return;
     const float b = bound[i];
-    scale[i] = b > 1e-30f && b < 1e30f ? ldexpf(1.f, 14 - ilogbf(b)) : 1.f;
+    const bool fits = b >= 0x1p-40f && b <= 0x1p40f;
+    scale[i] = fits ? ldexpf(1.f, 14 - ilogbf(b)) : 1.f;
+    if (!fits && b != 0.f) atomicOr(bad, 1);
 }
 
 // Split rows of W [N, K], each scaled so that its largest value lies in [2^14,
@@ -383,7 +387,7 @@ hipError_t launch_split_scales(const LayerW* d_layers, const LayerW* layers, con
                                         slot + SLOT_HID, bad);
     }
     k_split_scores<<<L * H, 64, 0, s>>>(typ, bound, C, H, bad);
-    k_split_scales<<<(split_slots(L) + 63) / 64, 64, 0, s>>>(bound, scale, split_slots(L));
+    k_split_scales<<<(split_slots(L) + 63) / 64, 64, 0, s>>>(bound, scale, split_slots(L), bad);
     return hipGetLastError();
 }
 

@@ -224,3 +224,29 @@ def test_unsuited_model_keeps_the_fp32_products(monkeypatch):
     assert not np.array_equal(split, plain)
     assert np.abs(split - plain).max() <= 2e-6 * np.abs(plain).max()
     assert np.array_equal(got, logits(wild))
+
+
+@pytest.mark.parametrize("gain", [1e-9, 1e-16, 1e-25, 1e14])
+def test_gains_far_from_one(monkeypatch, gain):
+    """Small and large gains of a whole LayerNorm: a product of two scales must not
+    leave fp32's range (q and k's together, a weight row's and its input's); gains too
+    far from 1 for that keep the fp32 products, bit for bit."""
+    cfg = cngpt_amd.Config(2, 2, 64, 300, 256)
+    p = cngpt_amd.init_weights(cfg, 3)
+    at = 300 * 64 + 256 * 64
+    p[at:at + 64] = gain  # layer 0, ln1_w
+    tokens = np.random.default_rng(1).integers(0, 300, (1, 200), dtype=np.int32)
+
+    def logits():
+        with cngpt_amd.Model(cfg, p) as m:
+            return m.forward(tokens, cngpt_amd.ALL)
+
+    got = logits()
+    monkeypatch.setenv("CNGPT_HIP_SPLIT", "0")
+    want = logits()
+    assert np.isfinite(got).all()
+    if gain == 1e-9:
+        assert not np.array_equal(got, want)
+        assert np.abs(got - want).max() <= 2e-6 * np.abs(want).max()
+    else:
+        assert np.array_equal(got, want)
