@@ -119,22 +119,27 @@ __global__ void __launch_bounds__(256) k_split_bound(const float* __restrict__ W
 // Per layer and head: whether scores keep their accuracy. q and k values too
 // small for a full lo are off by 2^-39 of their bounds, which must move a score
 // (in units of log2 e) by no more than its fp32 roundings would: 2^-24 of its
-// typical size, or of a quarter.
+// typical size, or of a quarter. And whether a score can be so large that its rounding
+// takes a probability out of fp16's range: k_attn_split's exponents reach 15 and
+// half a unit of the maximum's last place (0.25 at 2^22, 1 at 2^24) and must stay
+// below 16. |q| <= sqrt(C) |w g| + |w b + c| <= sqrt(C + 1) of its typical size.
 __global__ void __launch_bounds__(64) k_split_scores(const float* __restrict__ typ,
                                                      const float* __restrict__ bound, int C, int H,
                                                      int* bad) {
     const int l = blockIdx.x / H, hs = C / H, h = blockIdx.x % H, lane = threadIdx.x;
     const float* t = typ + (long)l * 7 * C + h * hs;
-    float tq = 0.f, tk = 0.f;
+    float tq = 0.f, tk = 0.f, top = 0.f;
     for (int d = lane; d < hs; d += 64) {
         tq = fmaxf(tq, t[d]);
         tk = fmaxf(tk, t[C + d]);
+        top += t[d] * t[C + d];
     }
     tq = wave_max(tq);
     tk = wave_max(tk);
+    top = wave_sum(top) * (C + 1.f) * (1.4426950408889634f / sqrtf((float)hs));
     const float bq = bound[SPLIT_SLOTS * l + SLOT_Q], bk = bound[SPLIT_SLOTS * l + SLOT_Q + 1];
     const float err = 0x1p-39f * (bq * tk + bk * tq);  // sqrt(hs) terms, over sqrt(hs)
-    if (lane == 0 && !(err <= 0x1p-24f * fmaxf(0.25f, tq * tk))) atomicOr(bad, 1);
+    if (lane == 0 && !(err <= 0x1p-24f * fmaxf(0.25f, tq * tk) && top <= 0x1p22f)) atomicOr(bad, 1);
 }
 
 // scale = the power of two that takes the bound into [2^14, 2^15), 1 where the
