@@ -175,6 +175,7 @@ struct cngpt_hip_ctx {
         const float* typ_b;
     };
     bool use_split = true, split_ok = true;
+    bool split_room = false;  // the parameter allocation holds the copies
     int split_state = 0;
     std::vector<SplitMat> splits;
     std::unordered_map<const float*, SplitWeights> split_of;
@@ -1177,9 +1178,12 @@ int params_prepare(cngpt_hip_ctx* h, const cngpt_hip_config* cfg) {
     const long want = params_of(cfg);
     const size_t bytes = align_up((size_t)want * sizeof(float)) +
                          align_up((size_t)cfg->n_layer * sizeof(LayerW)) +
-                         (h->use_packed ? packed_bytes(cfg) : 0) +
-                         (h->use_split ? split_bytes(cfg) : 0);
-    if (hipMalloc(&h->d_params, bytes) != hipSuccess) {
+                         (h->use_packed ? packed_bytes(cfg) : 0);
+    const size_t split = h->use_split ? split_bytes(cfg) : 0;
+    // (without the split copies, whose products the fp32 ones replace, if only that fits)
+    h->split_room = split && hipMalloc(&h->d_params, bytes + split) == hipSuccess;
+    if (!h->split_room) (void)hipGetLastError();
+    if (!h->split_room && hipMalloc(&h->d_params, bytes) != hipSuccess) {
         (void)hipGetLastError();
         h->d_params = nullptr;
         return fail("parameter allocation of %ld floats failed", want);
@@ -1241,7 +1245,7 @@ int params_commit(cngpt_hip_ctx* h, const cngpt_hip_config* cfg) {
             add(w.mlp_w, c, 4 * c);
         }
     }
-    if (h->use_split && split_bytes(cfg)) {
+    if (h->split_room) {
         const int L = cfg->n_layer;
         h->sp_bound = (float*)take(4 * (size_t)split_slots(L));
         h->sp_scale = (float*)take(4 * (size_t)split_slots(L));

@@ -329,6 +329,7 @@ int cngpt_hip_train_create(cngpt_hip_ctx* h, int B, int T, cngpt_hip_train** out
                  ln_bwd_part_floats((int)N, (int)C)}));
     fl(4 * C);                                // zeros
     t->can_split = split_takes(v, N);
+    const size_t split_at = sz.size();
     if (t->can_split) {
         t->n_maxima = L * (4 + 7 * C + 16 * C);
         fl(t->n_maxima); fl(N);               // maxima, rmax
@@ -336,12 +337,25 @@ int cngpt_hip_train_create(cngpt_hip_ctx* h, int B, int T, cngpt_hip_train** out
         fl(Np * 4 * C); fl(N * 4 * C); fl(Np * 4 * C);  // y_col, y_row, x_col
         sz.push_back(4 * L * sizeof(SplitTensor));      // weights
     }
+    const size_t split_end = sz.size();
     sz.push_back((size_t)grad_norm_parts(n) * sizeof(double));
     fl(1); fl(1);                             // norm, coef
     size_t total = 0;
-    for (size_t b : sz) total += (b + 255) & ~(size_t)255;
-    if (hipMalloc(&t->arena, total) != hipSuccess) {
+    auto allocate = [&] {
+        total = 0;
+        for (size_t b : sz) total += (b + 255) & ~(size_t)255;
+        if (hipMalloc(&t->arena, total) == hipSuccess) return true;
         (void)hipGetLastError();
+        t->arena = nullptr;
+        return false;
+    };
+    bool got = allocate();
+    if (!got && t->can_split) {  // only the fp32 products' buffers may fit
+        t->can_split = false;
+        sz.erase(sz.begin() + split_at, sz.begin() + split_end);
+        got = allocate();
+    }
+    if (!got) {
         delete t;
         return ctx_fail("training allocation of %zu bytes failed", total);
     }
