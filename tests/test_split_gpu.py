@@ -51,7 +51,14 @@ def gelu64(x):
 # odd row length
 SHAPES = [(129, 48, 16), (129, 256, 48), (300, 304, 80), (1, 8, 32), (2100, 304, 112), (130, 71, 32),
           (700, 2304, 768), (2047, 776, 3072), (1025, 768, 3072), (4095, 1608, 112),
-          (4097, 3064, 176), (4100, 6392, 1600), (513, 4099, 256), (2049, 2312, 768)]
+          (4097, 3064, 176), (4100, 6392, 1600), (513, 4099, 256), (2049, 2312, 768),
+          (5121, 2305, 144), (2049, 3073, 512), (5121, 769, 400)]
+
+
+def test_shapes_reach_every_tile(kat):
+    """Both forms of a store (16 bytes a lane; odd row lengths) on every tile shape."""
+    for odd in (0, 1):
+        assert {kat.kat_split_plan(*s) >> 8 for s in SHAPES if s[1] % 2 == odd} == set(range(5))
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)

@@ -61,7 +61,8 @@ def step(cfg, params, tok, tgt):
 
 # one step, tiles' edges, padding rows, K split, the tile shapes
 @pytest.mark.parametrize("M,N,K,pad", [(65, 16, 32, 1), (130, 72, 64, 30), (768, 776, 1216, 25),
-                                       (1000, 264, 992, 0), (4096, 3072, 768, 0), (4099, 768, 3072, 3)])
+                                       (1000, 264, 992, 0), (4096, 3072, 768, 0), (4099, 768, 3072, 3),
+                                       (5121, 2312, 144, 5)])
 @pytest.mark.parametrize("km", [2, 3])
 def test_product_of_far_apart_rows_and_columns(M, N, K, pad, km):
     """Each element within the bound of a product (test_split_gpu) of its own row's and

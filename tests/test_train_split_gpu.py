@@ -15,10 +15,16 @@ from test_train_gpu import batch, compare_grads, tensors
 
 pytestmark = pytest.mark.gpu
 
-# one step, fewer steps than the ring's stages, K split; ragged rows and columns; the
-# whole-K tiles of each shape
+# one step, fewer steps than the ring's stages, K split; ragged rows and columns; every
+# tile shape (test_products_reach_every_tile)
 PRODUCTS = [(65, 16, 32), (130, 72, 64), (768, 768, 4096), (3072, 768, 4096), (2304, 768, 1024),
-            (1000, 264, 992), (4096, 3072, 768), (4099, 768, 3072), (6400, 1600, 320)]
+            (1000, 264, 992), (4096, 3072, 768), (4099, 768, 3072), (6400, 1600, 320), (5121, 2312, 144)]
+
+
+def test_products_reach_every_tile():
+    lib = ctypes.CDLL(LIB)
+    assert {lib.kat_split_plan(*s) >> 8 for s in PRODUCTS} == set(range(5))
+
 
 
 @pytest.mark.parametrize("M,N,K", PRODUCTS)
@@ -57,6 +63,8 @@ CASES = {
     "c528": (cngpt_amd.Config(1, 33, 528, 97, 256), 5, 241),
     # many rows, so that the larger tiles are taken
     "rows": (cngpt_amd.Config(1, 12, 768, 1000, 512), 5, 509),
+    # GPT-2's vocabulary (the lm_head beside the split layers)
+    "vocab": (cngpt_amd.Config(1, 12, 768, 50257, 400), 2, 400),
 }
 
 
@@ -84,9 +92,9 @@ def test_step_vs_oracle(name):
 
 
 def test_far_apart_gains_keep_fp32(monkeypatch):
-    """Gains 2^-20 of their neighbours, on columns whose weights make up for it:
-    one scale would cost those columns their bits, so the step is the fp32 one,
-    to the bit."""
+    """Gains 2^-20 of their neighbours, on columns whose weights make up for it: the
+    weights' one scale would cost those columns their bits, so the step is the fp32 one,
+    to the bit. (Gains alone: test_train_precision_gpu.)"""
     cfg, B, T = CASES["ragged"]
     params = randomize(cfg, cngpt_amd.init_weights(cfg, 41), 42)
     at = {n: (o, k) for n, o, k in tensors(cfg)}
