@@ -1189,7 +1189,7 @@ __global__ void __launch_bounds__(256) k_stream_reduce(GemmArgs a, int KS) {
 // a.ln_out: the residual stream and the next product's input in one pass.
 // Only the residual epilogue forms a LayerNorm (the residual stream feeds the
 // next sub-layer); rows of up to 2048 floats (NCH = 1 or 2 float4 per thread).
-template <int EPI, int NCH>
+template <int EPI, int NCH, bool SPLIT>
 __global__ void __launch_bounds__(256) k_stream_reduce_ln(GemmArgs a, int KS) {
     static_assert(EPI == EPI_RESID && (NCH == 1 || NCH == 2), "residual rows of <= 2048 floats");
     __shared__ float red[4];
@@ -1256,13 +1256,13 @@ __global__ void __launch_bounds__(256) k_stream_reduce_ln(GemmArgs a, int KS) {
         }
     const float rstd = 1.0f / sqrtf(block_sum(q) / (float)a.N + 1e-5f);
     float* orow = a.ln_out + (long)r * a.N;
-    const float sc = a.ln_scale ? *a.ln_scale : 1.f;
+    const float sc = SPLIT ? *a.ln_scale : 1.f;
 #pragma unroll
     for (int i = 0; i < NCH; i++) {
         const int c4 = tid + 256 * i;
         if (c4 < N4) {
             const f32x4 o = (y[i] - mean) * rstd * lw[i] + lb[i];
-            if (a.ln_scale) *(u32x4*)(orow + 4 * c4) = split_quad(o * sc, lane);
+            if constexpr (SPLIT) *(u32x4*)(orow + 4 * c4) = split_quad(o * sc, lane);
             else *(f32x4*)(orow + 4 * c4) = o;
         }
     }
@@ -1276,8 +1276,14 @@ hipError_t reduce_splits(const GemmArgs& a, int KS, hipStream_t s) {
     if constexpr (EPI == EPI_RESID) {
         // launch_gemm admits ln_out for the residual epilogue and N <= 2048 only
         if (a.ln_out) {
-            if (a.N <= 1024) k_stream_reduce_ln<EPI, 1><<<a.M, 256, 0, s>>>(a, KS);
-            else k_stream_reduce_ln<EPI, 2><<<a.M, 256, 0, s>>>(a, KS);
+            // (SPLIT a template argument: tested at run time it cost batched decode steps,
+            // which have two of these launches a layer, 0.2-0.3 %: 0.9494 -> 0.9515 ms at
+            // 24 layers of 1024 columns and 8 rows, 0.881 -> 0.884 at 12 of 1600 and 32)
+            if (a.ln_scale) {
+                if (a.N <= 1024) k_stream_reduce_ln<EPI, 1, true><<<a.M, 256, 0, s>>>(a, KS);
+                else k_stream_reduce_ln<EPI, 2, true><<<a.M, 256, 0, s>>>(a, KS);
+            } else if (a.N <= 1024) k_stream_reduce_ln<EPI, 1, false><<<a.M, 256, 0, s>>>(a, KS);
+            else k_stream_reduce_ln<EPI, 2, false><<<a.M, 256, 0, s>>>(a, KS);
             return hipGetLastError();
         }
     }

@@ -45,7 +45,7 @@ __global__ void __launch_bounds__(256) k_embed(const int* __restrict__ tok,
 // NCH = float4 chunks per lane, so C <= 256 * NCH. Rows are read at stride
 // in_stride and written at stride out_stride (floats), which lets the final
 // LayerNorm of the last-position pass gather rows b*T + T-1.
-template <int NCH>
+template <int NCH, bool SPLIT>
 __global__ void __launch_bounds__(256) k_layernorm(const float* __restrict__ x, long in_stride,
                                                    const float* __restrict__ w,
                                                    const float* __restrict__ b, float* __restrict__ out,
@@ -85,13 +85,13 @@ __global__ void __launch_bounds__(256) k_layernorm(const float* __restrict__ x, 
         rstd_out[row] = rs;
     }
     float* orow = out + (long)row * out_stride;
-    const float sc = split_scale ? *split_scale : 1.f;
+    const float sc = SPLIT ? *split_scale : 1.f;
 #pragma unroll
     for (int j = 0; j < NCH; j++) {
         int c = (lane + j * 64) * 4;
         if (c < C) {
             const f32x4 o = (v[j] - m) * rs * wv[j] + bv[j];
-            if (split_scale) *(u32x4*)(orow + c) = split_quad(o * sc, lane);
+            if constexpr (SPLIT) *(u32x4*)(orow + c) = split_quad(o * sc, lane);
             else *(f32x4*)(orow + c) = o;
         }
     }
@@ -125,25 +125,18 @@ hipError_t launch_layernorm(const float* x, long in_stride, const float* w, cons
                             float* mean, float* rstd, const float* split_scale) {
     if (rows == 0) return hipSuccess;
     if (!mean != !rstd || (split_scale && (C & 7))) return hipErrorInvalidValue;
-    dim3 grid((rows + 3) / 4), block(256);
-    int nch = (C + 255) / 256;
-    if (nch <= 1)
-        k_layernorm<1><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd,
-                                            split_scale);
-    else if (nch <= 2)
-        k_layernorm<2><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd,
-                                            split_scale);
-    else if (nch <= 3)
-        k_layernorm<3><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd,
-                                            split_scale);
-    else if (nch <= 4)
-        k_layernorm<4><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd,
-                                            split_scale);
-    else if (nch <= 8)
-        k_layernorm<8><<<grid, block, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd,
-                                            split_scale);
-    else
-        return hipErrorInvalidValue;
+    const dim3 grid((rows + 3) / 4);
+    const auto run = [&](auto kernel) {
+        kernel<<<grid, 256, 0, s>>>(x, in_stride, w, b, out, out_stride, rows, C, mean, rstd, split_scale);
+    };
+    const bool split = split_scale != nullptr;
+    const int nch = (C + 255) / 256;
+    if (nch <= 1) run(split ? k_layernorm<1, true> : k_layernorm<1, false>);
+    else if (nch <= 2) run(split ? k_layernorm<2, true> : k_layernorm<2, false>);
+    else if (nch <= 3) run(split ? k_layernorm<3, true> : k_layernorm<3, false>);
+    else if (nch <= 4) run(split ? k_layernorm<4, true> : k_layernorm<4, false>);
+    else if (nch <= 8) run(split ? k_layernorm<8, true> : k_layernorm<8, false>);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
