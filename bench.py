@@ -47,7 +47,9 @@ PEAK_HBM = 8.0e12
 
 
 def gemm_peak(rows: int, n_embd: int) -> float:
-    """FLOP/s of fp32 work that the forward's products over `rows` rows could reach."""
+    """FLOP/s of fp32 work that the forward's products over `rows` rows could reach
+    (split products: the seeded weights here fit them; a model whose weights do not
+    would run the fp32 ones)."""
     split = rows > 128 and n_embd % 16 == 0 and os.environ.get("CNGPT_HIP_SPLIT", "1")[:1] != "0"
     return PEAK_SPLIT_MFMA if split else PEAK_FP32_MFMA
 SEED = 1234
@@ -159,12 +161,17 @@ def train_leg(m: cngpt_amd.Model, cfg, B: int, T: int, steps: int, warmup: int) 
         m.synchronize()
         dt_f = time.perf_counter() - t0
     fl = train_flops(cfg, B, T)
+    # (the trainer's own rule: 512 columns, 768 x 768 values and up)
+    takes = cfg.n_embd >= 512 and B * T * cfg.n_embd >= 768 * 768
+    peak = gemm_peak(B * T, cfg.n_embd) if takes else PEAK_FP32_MFMA
+    split = 2 * 2.0 * B * T * 12 * cfg.n_embd ** 2 * cfg.n_layer
     return {"train_B": B, "train_T": T, "tok_s": round(B * T * steps / dt, 1),
             "ms_per_step": round(dt * 1e3 / steps, 3),
             "forward_ms": round(dt_f * 1e3 / steps, 3),
             "tflops": round(fl * steps / dt / 1e12, 2),
-            # of the fp32 rate, though part of the backward runs on the fp16 units
-            "mfma_frac": round(fl * steps / dt / PEAK_FP32_MFMA, 4),
+            # of the time that the matrix units need at their peaks: the layers'
+            # backward products as split ones, the rest in fp32
+            "mfma_frac": round(((fl - split) / PEAK_FP32_MFMA + split / peak) * steps / dt, 4),
             "first_loss": round(losses[0], 5), "last_loss": round(losses[-1], 5),
             "last_grad_norm": round(norm, 5)}
 

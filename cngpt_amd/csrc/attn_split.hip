@@ -40,14 +40,15 @@ __device__ __forceinline__ f32x16 mfma(const f16x8& a, const f16x8& b, const f32
 // granules are swizzled by key % 4, over bits that the 32 d of a read leave
 // free. Splitting fp32 rows while staging them instead took 147 of the 440
 // vector instructions a wavefront issues per tile, and those are the bound
-// (GPT-2 small B=16 T=1024: 113 us against REPLACE per layer; 285 in fp32).
+// (GPT-2 small B=16 T=1024: 113 us against 98 per layer; 285 in fp32).
 //
 // scales: q, k and v carry scales[0], [1] and [2] (powers of two); the output
 // is split rows times scales[2]. A probability carries a factor 2^12, which
 // cancels against the sum, so that lo keeps its bits down to 2^-26 of the
 // row's largest. The running max is moved only when some score of the
-// wavefront passes it by more than 3 (probabilities up to 2^15 then), which
-// leaves the output unscaled on most tiles.
+// wavefront passes it by more than 3 (probabilities up to 2^15 then, and half a
+// unit of the maximum's last place in the exponent more: k_split_scores holds
+// scores below 2^22), which leaves the output unscaled on most tiles.
 template <int HS, int KT, int OCC>
 __global__ void __launch_bounds__(256, OCC)
     k_attn_split(const float* __restrict__ qkv, float* __restrict__ out, int B, int T, int C, int H,
@@ -236,13 +237,13 @@ hipError_t launch_attention_split(const float* qkv, float* out, int B, int T, in
     const int nqb = (T + 127) / 128;
     const unsigned grid = (unsigned)nqb * B * H;
     switch (C / H) {
-        case 32: 
+        case 32:
             k_attn_split<32, 64, 4><<<grid, 256, 0, s>>>(qkv, out, B, T, C, H, nqb, scales);
             break;
-        case 64: 
+        case 64:
             k_attn_split<64, 64, 2><<<grid, 256, 0, s>>>(qkv, out, B, T, C, H, nqb, scales);
             break;
-        case 128: 
+        case 128:
             k_attn_split<128, 32, 2><<<grid, 256, 0, s>>>(qkv, out, B, T, C, H, nqb, scales);
             break;
         default: return hipErrorInvalidValue;

@@ -300,8 +300,12 @@ constexpr int SKINNY = 2;
 int run_ln(cngpt_hip_ctx* h, const float* x, long in_stride, const float* w, const float* b,
            float* out, int rows, const float* split_scale = nullptr);
 
-// Rows above which a forward's layer products take the split operands
-// (split.hip); up to them the few-row products stream the weights.
+// Rows above which a forward's layer products take the split operands (split.hip);
+// up to them the few-row products, built for so many, stream the weights. From 129
+// rows on the split forwards are the faster ones at every width (4 layers, one
+// sequence of 129 tokens, all logits, us, fp32 against split: C = 32 198 / 136, 256
+// 235 / 185, 768 555 / 355, 1600 1158 / 597; of 1024: 231 / 176, 393 / 376, 1449 /
+// 831, 3825 / 1716). Fewer rows have no split form to compare.
 constexpr int SPLIT_MIN_ROWS = 128;
 
 // Whether a forward over `rows` rows takes them.

@@ -24,8 +24,9 @@
 // lo starts losing bits: an absolute error of 2^-39 of the bound. k_split_w
 // compares that with each output's typical size and flags matrices where it
 // could exceed 2^-24 of it (gains or rows many thousands of times apart, or
-// values that are not finite); a model with a flagged matrix keeps the fp32
-// kernels.
+// values that are not finite), k_split_scores heads whose scores lose accuracy
+// or could be too large for their probabilities, k_split_scales bounds further than
+// 2^40 from 1; a model with a flag keeps the fp32 kernels.
 #include <algorithm>
 #include <cmath>
 
@@ -47,7 +48,7 @@ __device__ __forceinline__ float block_max(float v, float* red) {
 }
 
 // max that keeps a NaN (fmaxf drops it)
-__device__ __forceinline__ float max_nan(float m, float v) { return v <= m ? m : v; }
+__device__ __forceinline__ float max_nan(float m, float v) { return m != m || v <= m ? m : v; }
 
 // Bounds of the LayerNorm outputs; the other slots are cleared for
 // k_split_bound.
