@@ -502,8 +502,8 @@ def main():
     traffic, tsrc = None, None
     tpath = os.path.join(ROOT, "profiles", "gemm_traffic.json")
     split = gemm_peak(B * T, cfg.n_embd) == PEAK_SPLIT_MFMA
-    # (the counters were read over the fp32 products)
-    if name == "small" and not split and os.path.exists(tpath):
+    # (the counters were read over the split products)
+    if name == "small" and split and os.path.exists(tpath):
         with open(tpath) as f:
             tj = json.load(f)
         traffic = tj.get("measured_bytes_per_launch")

@@ -67,7 +67,11 @@ enum { CNGPT_DECODE_AUTO = 0, CNGPT_DECODE_KERNELS = 1, CNGPT_DECODE_PERSISTENT 
 const char *cngpt_hip_last_error(void);
 
 /* Handle on HIP device `device`. No reference counterpart: replaces the
- * zeroed FastCtx of fast_init (src/fast.c:29-32). */
+ * zeroed FastCtx of fast_init (src/fast.c:29-32). Forwards over more than 128
+ * rows and the backward of larger training steps run on the fp16 matrix cores
+ * over operands held as two fp16 halves, where the weights let these be as
+ * accurate as fp32 ones; CNGPT_HIP_SPLIT=0 in the environment here keeps the
+ * fp32 products everywhere. */
 int  cngpt_hip_create(int device, cngpt_hip_ctx **out);
 /* Frees the handle, its stream and both device allocations
  * (fast_free, src/fast.c:34-40). NULL is a no-op. */
@@ -256,7 +260,8 @@ int  cngpt_hip_train_forward(cngpt_hip_train *t, const int *tokens, const int *t
                              float *loss);
 
 /* gpt_backward (model.c:634-877) for the last forward: gradients add to
- * the held ones, as in the reference. */
+ * the held ones, as in the reference. Enqueues on the handle's stream; larger
+ * steps wait there for the verdict on the weights' split copies. */
 int  cngpt_hip_train_backward(cngpt_hip_train *t);
 
 /* GPTConfig.dropout (src/model.h:43) for this trainer's forwards, p in
