@@ -607,7 +607,12 @@ int cngpt_hip_train_backward(cngpt_hip_train* t) {
     // weights that do not fit take the fp32 products from now on (the device works on
     // the lm_head meanwhile)
     if (t->can_split) {
-        TRY(hipEventSynchronize(t->judged));
+        // (a thread that captures another stream may wait in relaxed mode only)
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        TRY(hipThreadExchangeStreamCaptureMode(&mode));
+        const hipError_t e = hipEventSynchronize(t->judged);
+        TRY(hipThreadExchangeStreamCaptureMode(&mode));
+        TRY(e);
         t->can_split = *t->verdict == 0;
     }
     unsigned* col = t->colmax;

@@ -1,6 +1,7 @@
 """Forwards of more than 128 rows after an optimizer step: every entry point runs the
 updated weights, on the same products whichever came first, and a captured
 no-alloc forward replays them."""
+import contextlib
 import ctypes
 
 import numpy as np
@@ -92,34 +93,61 @@ def test_captured_noalloc_forward_reads_the_live_weights(hip, monkeypatch):  # n
         out.free()
 
 
-@pytest.mark.parametrize("capture_mode", [0, 1, 2])  # global, thread-local, relaxed
-def test_noalloc_beside_a_capture(hip, capture_mode):  # noqa: F811
-    """The first no-alloc forward after an update, called while the thread captures
-    another stream."""
+@contextlib.contextmanager
+def capturing(hip, mode):  # noqa: F811
+    """The thread captures a stream of its own (mode: 0 global, 1 thread-local, 2
+    relaxed)."""
     hip.hipStreamCreate.argtypes = [ctypes.POINTER(ctypes.c_void_p)]
     hip.hipStreamBeginCapture.argtypes = [ctypes.c_void_p, ctypes.c_int]
     hip.hipStreamEndCapture.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p)]
     hip.hipStreamDestroy.argtypes = hip.hipGraphDestroy.argtypes = [ctypes.c_void_p]
-    tokens = np.random.default_rng(1).integers(0, CFG.vocab_size, (1, T), dtype=np.int32)
-    n = CFG.vocab_size * T
-    tok, out = DevBuf(hip, tokens.nbytes), DevBuf(hip, 4 * n)
-    tok.put(tokens)
     s, g = ctypes.c_void_p(), ctypes.c_void_p()
     assert hip.hipStreamCreate(ctypes.byref(s)) == 0
     try:
-        with cngpt_amd.Model(CFG, randomize(CFG, cngpt_amd.init_weights(CFG, 2), 3)) as m:
-            with cngpt_amd.Model(CFG, update(m, 4)) as fresh:
-                want = fresh.forward(tokens, cngpt_amd.ALL).ravel()
-            assert hip.hipStreamBeginCapture(s, capture_mode) == 0
-            try:
-                m.forward_noalloc(tok.ptr.value, 1, T, cngpt_amd.ALL, out.ptr.value, None)
-            finally:
-                assert hip.hipStreamEndCapture(s, ctypes.byref(g)) == 0
-            m.synchronize()
-            assert np.array_equal(out.get(n, np.float32), want)
+        assert hip.hipStreamBeginCapture(s, mode) == 0
+        try:
+            yield
+        finally:
+            assert hip.hipStreamEndCapture(s, ctypes.byref(g)) == 0
     finally:
         if g:
             hip.hipGraphDestroy(g)
         hip.hipStreamDestroy(s)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_noalloc_beside_a_capture(hip, mode):  # noqa: F811
+    """The first no-alloc forward after an update, called while the thread captures
+    another stream."""
+    tokens = np.random.default_rng(1).integers(0, CFG.vocab_size, (1, T), dtype=np.int32)
+    n = CFG.vocab_size * T
+    tok, out = DevBuf(hip, tokens.nbytes), DevBuf(hip, 4 * n)
+    tok.put(tokens)
+    try:
+        with cngpt_amd.Model(CFG, randomize(CFG, cngpt_amd.init_weights(CFG, 2), 3)) as m:
+            with cngpt_amd.Model(CFG, update(m, 4)) as fresh:
+                want = fresh.forward(tokens, cngpt_amd.ALL).ravel()
+            with capturing(hip, mode):
+                m.forward_noalloc(tok.ptr.value, 1, T, cngpt_amd.ALL, out.ptr.value, None)
+            m.synchronize()
+            same = np.array_equal(out.get(n, np.float32), want)
+            assert same
+    finally:
         tok.free()
         out.free()
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_backward_beside_a_capture(hip, mode):  # noqa: F811
+    """A backward whose products take split weights, called likewise."""
+    cfg = cngpt_amd.Config(1, 12, 768, 72, 256)
+    tok, tgt = (np.random.default_rng(i).integers(0, 72, (3, 256), dtype=np.int32) for i in (1, 2))
+    with cngpt_amd.Model(cfg, cngpt_amd.init_weights(cfg, 3)) as m, cngpt_amd.Trainer(m, 3, 256) as tr:
+        tr.forward(tok, tgt)
+        tr.backward()
+        want = tr.grads
+        tr.zero_grad()
+        tr.forward(tok, tgt)
+        with capturing(hip, mode):
+            tr.backward()
+        assert np.array_equal(tr.grads, want)
